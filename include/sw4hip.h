@@ -312,8 +312,8 @@ int sw4hip_ew_set_stream(sw4hip_ew* ew, void* stream);
  * default) as 9 with rows of odd length staged by four-byte asynchronous
  * loads and the acceleration stored for them too (the same bits as 9).
  * All give the same results to rounding.  kchunk > 0 sets the planes per
- * workgroup of every sweep; kchunk <= 0 keeps the defaults (64 for the
- * predictor and corrector sweeps, 32 for the damping sweep). */
+ * workgroup of every sweep; kchunk <= 0 lets the library choose from
+ * the grid's size (whole rounds of resident workgroups; the default). */
 int sw4hip_ew_set_kernel_variant(sw4hip_ew* ew, int variant, int kchunk);
 /* rho, mu, lambda over the whole box incl. ghosts; on_device selects whether
  * the pointers are device (1) or host (0) arrays. */

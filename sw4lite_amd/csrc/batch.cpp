@@ -159,6 +159,16 @@ int Batch::build_tables()
 {
    const int n = (int)m_shots.size();
    std::vector<SweepShot> h(9 * n);
+   int kchunk = m_kchunk;
+   if (kchunk <= 0) {  // all shots' tiles share the device
+      long tiles = 0;
+      int npl = 1;
+      for (const EW* e : m_shots) {
+         tiles += (long)((e->m_opt.grid.nx + 31) / 32) * ((e->m_opt.grid.ny + 7) / 8);
+         npl = std::max(npl, e->m_opt.grid.nz);
+      }
+      kchunk = march_kchunk(tiles, npl, 2);
+   }
    m_useacc.assign(3 * n, 0);
    for (int ph = 0; ph < 3; ph++) {
       // kinds 0 and 2: the grids whose planes take the asynchronous loads
@@ -188,15 +198,15 @@ int Batch::build_tables()
                int& gc = fa[k] ? ga[k] : g0[k];
                SweepShot* d = &t[k * n + slot[k]++];
                if (k == 0)
-                  gc = fill_sweep_shot(false, b, k1, k2, m_kchunk, nullptr, u, um, e->mMu.dev, e->mLambda.dev,
+                  gc = fill_sweep_shot(false, b, k1, k2, kchunk, nullptr, u, um, e->mMu.dev, e->mLambda.dev,
                                        e->mRho.dev, c, e->mUp.dev, g.h, e->mDt, 0.0, false, gc, d, nullptr, 0,
                                        acc ? m_acc[q] : nullptr);
                else if (k == 1)
-                  gc = fill_sweep_shot(false, b, k1, k2, m_kchunk, e->mUp.dev, u, um, e->mMu.dev, e->mLambda.dev,
+                  gc = fill_sweep_shot(false, b, k1, k2, kchunk, e->mUp.dev, u, um, e->mMu.dev, e->mLambda.dev,
                                        e->mRho.dev, c, up2, g.h, e->mDt, e->m_opt.beta, true, gc, d, nullptr, 0,
                                        acc ? m_acc[q] : nullptr);
                else
-                  gc = fill_sweep_shot(true, b, k1, damp ? k2 : k1 - 1, m_kchunk, nullptr, u, um, nullptr, nullptr,
+                  gc = fill_sweep_shot(true, b, k1, damp ? k2 : k1 - 1, kchunk, nullptr, u, um, nullptr, nullptr,
                                        e->mRho.dev, c, up2, g.h, e->mDt, e->m_opt.beta, true, gc, d, m_dtiles[q],
                                        m_ndtiles[q]);
             }

@@ -61,7 +61,7 @@ private:
    int* m_clk_max = nullptr;
    std::vector<double*> m_base;     // per shot: Um, U, Up2 of phase 0
    int m_phase = 0;
-   int m_kchunk = 64;
+   int m_kchunk = 0;  // planes per workgroup of the batched sweeps; 0: from the shots' sizes
    hipGraphExec_t m_exec = nullptr;
    std::vector<void*> m_allocs;
    std::vector<DampTile*> m_dtiles;  // per shot: its damping tile list (kernel variant 9), or null

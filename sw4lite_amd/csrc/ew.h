@@ -214,10 +214,10 @@ public:
    std::vector<int> m_first;
    hipStream_t m_stream = nullptr;
    int m_variant = 10;  // interior sweep kernels: 0 thread per point, 1-10 LDS-staged k-march
-   // planes per workgroup of the LDS sweeps: predictor and corrector, and
-   // the damping sweep over the supergrid layers (fastest measured at 512^3
-   // on one device: 64 and 32 of 32..256)
-   static constexpr int kSweepChunk = 64, kDampChunk = 32;
+   // planes per workgroup of the LDS sweeps (predictor and corrector; the
+   // damping sweep over the supergrid layers); 0: chosen from the grid's
+   // size (march_kchunk, damp_tiles)
+   static constexpr int kSweepChunk = 0, kDampChunk = 0;
    int m_kchunk = kSweepChunk;
    int m_kchunk_damp = kDampChunk;
 

@@ -211,37 +211,6 @@ __device__ void sbp_col_T(const AdjCtx& A, const double* z, int i, int j, int k,
    }
 }
 
-// Planes per workgroup for an LDS k-march of `tiles` column tiles over `npl`
-// planes when `per_cu` workgroups fit on a CU: the k-block count near npl/64
-// that minimises (rounds of resident workgroups) x (planes per workgroup +
-// the 4 planes each one primes).  Workgroups run in rounds, so a count just
-// above a multiple of the resident slots costs a whole extra round.
-int march_kchunk(long tiles, int npl, int per_cu)
-{
-   static int cus = 0;
-   if (!cus) {
-      int dev = 0, v = 0;
-      if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) {
-         (void)hipGetLastError();
-         v = 256;
-      }
-      cus = v;
-   }
-   const long slots = (long)cus * per_cu;
-   const int nc0 = std::max(1, (npl + 32) / 64);
-   int best = nc0;
-   long bcost = -1;
-   for (int nc = std::max(1, nc0 / 2); nc <= 2 * nc0 + 1; nc++) {
-      const long rounds = (tiles * nc + slots - 1) / slots;
-      const long cost = rounds * ((npl + nc - 1) / nc + 4);
-      if (bcost < 0 || cost < bcost) {
-         bcost = cost;
-         best = nc;
-      }
-   }
-   return (npl + best - 1) / best;
-}
-
 Box pad_box(const Box& b) { return make_box(b.ib - 2, b.ie + 2, b.jb - 2, b.je + 2, b.kb - 2, b.ke + 2); }
 
 long adj_pad_doubles(const Box& b)

@@ -10,6 +10,7 @@
 //   predictor:  reads U, mu, lambda, rho          writes A          (9 words)
 //   corrector:  reads A, D, U, C, mu, lambda, rho writes Dn, U, C   (24 words)
 #include "kernels_comp.h"
+#include "kernels_fast.h"
 #include "kernels_step.h"
 #include "sbp_row_body.h"
 #include "stencil_body.h"
@@ -594,7 +595,8 @@ struct SlabStenF {
 
 // The six SBP rows at a free surface (top: k = 1..6, bottom: nk..nk-5), one
 // 32 x 8 tile per workgroup with nine planes of U (predictor) or A
-// (corrector) and eight material planes staged in LDS.
+// (corrector) and eight material planes staged in LDS; block.y
+// takes the rows 1 + block.y, the next gridDim.y on.
 template <bool CORR>
 __global__ void __launch_bounds__(NT, 1)
 k_comp_rows(Box b, int top, int nk, int ntx, const SbpTablesT<float>* __restrict__ sbp, const float* __restrict__ stg,
@@ -650,8 +652,13 @@ k_comp_rows(Box b, int top, int nk, int ntx, const SbpTablesT<float>* __restrict
    if (!active) return;
    const SlabStenF st{su + o, sm + o, sl + o, ssx + tx + 2, ssy + ty + 2};
    const long colp = (i - b.ib) + ni * (j - b.jb);
+   // outside the supergrid layers every term of the damping is an exact zero
+   const int ii = i - b.ib, jj = j - b.jb;
+   const bool dxy = CORR && beta != 0 &&
+                    (sg.dcx[ii - 1] != 0 || sg.dcx[ii] != 0 || sg.dcx[ii + 1] != 0 || sg.dcy[jj - 1] != 0 ||
+                     sg.dcy[jj] != 0 || sg.dcy[jj + 1] != 0);
 #pragma unroll 1
-   for (int kr = 1; kr <= 6; kr++) {
+   for (int kr = 1 + (int)blockIdx.y; kr <= 6; kr += (int)gridDim.y) {
       const int k = kbase + sgn * (kr - 1);
       float r[3];
       sbp_row_body(st, kr, (float)sgn, sbp, r);
@@ -662,7 +669,9 @@ k_comp_rows(Box b, int top, int nk, int ntx, const SbpTablesT<float>* __restrict
          for (int c = 0; c < 3; c++) aout[p + npts * c] = sc * r[c];
       } else {
          float d[3] = {0, 0, 0};
-         if (beta != 0) damp_point_f(b, i, j, k, dold, rho, sg, beta, d);
+         const int kk = k - b.kb;
+         if (dxy || (beta != 0 && (sg.dcz[kk - 1] != 0 || sg.dcz[kk] != 0 || sg.dcz[kk + 1] != 0)))
+            damp_point_f(b, i, j, k, dold, rho, sg, beta, d);
          const float sc = c4 / rho[p];
 #pragma unroll
          for (int c = 0; c < 3; c++) {
@@ -926,10 +935,10 @@ int comp_sweep(bool corr, const Box& b, int k1, int k2, int kc, const CompState&
 {
    if (k2 < k1) return OK;
    const long nx = b.ie - b.ib - 3, ny = b.je - b.jb - 3;
-   if (kc <= 0) kc = 64;
    CompTiles map;
    map.ntx = (int)cdiv(nx, TX);
    map.nty = (int)cdiv(ny, TY);
+   if (kc <= 0) kc = march_kchunk((long)map.ntx * map.nty, k2 - k1 + 1, corr ? 2 : 4);
    map.ntiles = map.ntx * map.nty * (int)cdiv(k2 - k1 + 1, kc);
    const unsigned grd = 8 * cdiv(map.ntiles, 8);
    // asynchronous loads where every staged quad of floats lies in one row, aligned
@@ -955,12 +964,17 @@ int comp_rows(bool corr, const Box& b, int side, int nk, const SbpTablesT<float>
 {
    const long nx = b.ie - b.ib - 3, ny = b.je - b.jb - 3;
    const int ntx = (int)cdiv(nx, TX), nty = (int)cdiv(ny, TY);
+   // two workgroups fit on a CU: where the tiles leave slots idle the six rows
+   // are spread over block.y (at 301 x 301 points, where they do not, two
+   // groups of threads on one slab were slower: 82 -> 97 us)
+   const int tiles = ntx * nty, spread = tiles <= 85 ? 6 : tiles <= 170 ? 3 : tiles <= 256 ? 2 : 1;
+   const dim3 grd(tiles, spread);
    if (corr)
-      k_comp_rows<true><<<ntx * nty, NT, 0, s>>>(b, side == 4, nk, ntx, d_sbpf, st.A, st.mu, st.la, st.rho, sg, st.D,
-                                                 st.Dn, st.U, st.C, nullptr, cof, dt2, c4, beta);
+      k_comp_rows<true><<<grd, NT, 0, s>>>(b, side == 4, nk, ntx, d_sbpf, st.A, st.mu, st.la, st.rho, sg, st.D,
+                                           st.Dn, st.U, st.C, nullptr, cof, dt2, c4, beta);
    else
-      k_comp_rows<false><<<ntx * nty, NT, 0, s>>>(b, side == 4, nk, ntx, d_sbpf, st.U, st.mu, st.la, st.rho, sg,
-                                                  nullptr, nullptr, nullptr, nullptr, st.A, cof, dt2, c4, beta);
+      k_comp_rows<false><<<grd, NT, 0, s>>>(b, side == 4, nk, ntx, d_sbpf, st.U, st.mu, st.la, st.rho, sg,
+                                            nullptr, nullptr, nullptr, nullptr, st.A, cof, dt2, c4, beta);
    return check_hip(hipGetLastError(), "FP32 SBP rows launch");
 }
 }  // namespace

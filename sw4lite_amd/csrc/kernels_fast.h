@@ -10,6 +10,19 @@ struct TileMap {
    int ntx, nty, ntiles;  // tiles along i and j, tiles in all
 };
 
+// Planes per workgroup for an LDS k-march of `tiles` column tiles over `npl`
+// planes when `per_cu` workgroups fit on a CU: the k-block count that
+// minimises (rounds of resident workgroups) x (planes per workgroup + the
+// cost of priming, about 3 planes' time).  Workgroups run in rounds, so a
+// count just above a multiple of the resident slots costs a whole extra
+// round; a small grid gets short blocks, since a march of few workgroups is
+// one serial chain of planes (40 x 36 x 32 points: predictor sweep 77 -> 16
+// us in blocks of 4 planes instead of one of 26, damping 55 -> 9 us).  Never fewer than 3
+// planes, and never more than 48: workgroups that share halos drift apart
+// over a long block and no longer meet in L2 (512^3 predictor sweep 4.36 ms
+// in blocks of 32 planes, 4.46 of 64, 4.55 of 128, 4.70 of 506).
+int march_kchunk(long tiles, int npl, int per_cu);
+
 // One grid of a batched sweep: the arguments of its single-grid launch and
 // its first block id in the batched launch.
 struct DampTile;

@@ -22,8 +22,37 @@ namespace sw4amd {
 namespace {
 constexpr int TX = 32, TY = 8, HX = TX + 4, HY = TY + 4, NT = TX * TY, PL = HX * HY;
 inline unsigned cdiv(long a, long b) { return (unsigned)((a + b - 1) / b); }
+
+int compute_units()
+{
+   static const int cus = [] {
+      int dev = 0, v = 0;
+      if (hipGetDevice(&dev) != hipSuccess ||
+          hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) {
+         (void)hipGetLastError();
+         v = 256;
+      }
+      return v;
+   }();
+   return cus;
+}
 }  // namespace
 
+int march_kchunk(long tiles, int npl, int per_cu)
+{
+   const long slots = (long)compute_units() * per_cu;
+   int best = (npl + 47) / 48;
+   long bcost = -1;
+   for (int nc = (npl + 47) / 48; nc <= std::max((npl + 47) / 48, npl / 3); nc++) {
+      const long rounds = (tiles * nc + slots - 1) / slots;
+      const long cost = rounds * ((npl + nc - 1) / nc + 3);
+      if (bcost < 0 || cost < bcost) {
+         bcost = cost;
+         best = nc;
+      }
+   }
+   return (npl + best - 1) / best;
+}
 
 struct LdsSten {
    const double* p0;  // ring slot of plane k-2, offset to this thread's point
@@ -1159,7 +1188,6 @@ int launch_accel_fix(const Box& b, int k1, int k2, bool frame, bool all_planes, 
 std::vector<DampTile> damp_tiles(const Box& b, int k1, int k2, int kc, const double* dcx, const double* dcy,
                                  const double* dcz)
 {
-   if (kc <= 0) kc = 64;
    // point q (offset from the box start) can be damped along an axis when the
    // profile is nonzero at q-1, q or q+1 (the stencil of addsgd4)
    auto damped = [](const double* dc, int n) {
@@ -1171,13 +1199,27 @@ std::vector<DampTile> damp_tiles(const Box& b, int k1, int k2, int kc, const dou
    const std::vector<char> ox = damped(dcx, ni), oy = damped(dcy, nj), oz = damped(dcz, nk);
    const long nx = b.ie - b.ib - 3, ny = b.je - b.jb - 3;
    const int ntx = (int)cdiv(nx, TX), nty = (int)cdiv(ny, TY);
+   // the tile's columns meet an x or y layer: every plane
+   auto meets = [&](int tix, int tjy) {
+      bool side = false;
+      for (int q = 2 + tix * TX; q < std::min(2 + (tix + 1) * TX, ni - 2); q++) side = side || ox[q];
+      for (int q = 2 + tjy * TY; q < std::min(2 + (tjy + 1) * TY, nj - 2); q++) side = side || oy[q];
+      return side;
+   };
+   if (kc <= 0) {
+      // 32 planes a workgroup (the fastest of 16..128 at 512^3), fewer where
+      // that would leave slots of the device idle (3 workgroups per CU)
+      long zl = 0, planes = 0;
+      for (int k = k1; k <= k2; k++) zl += oz[k - b.kb];
+      for (int tjy = 0; tjy < nty; tjy++)
+         for (int tix = 0; tix < ntx; tix++) planes += meets(tix, tjy) ? k2 - k1 + 1 : zl;
+      kc = (int)std::min(32L, std::max(3L, (planes + 3L * compute_units() - 1) / (3L * compute_units())));
+   }
    std::vector<DampTile> out;
    std::vector<std::vector<DampTile>> per_chunk((size_t)cdiv(k2 - k1 + 1, kc));
    for (int tjy = 0; tjy < nty; tjy++)
       for (int tix = 0; tix < ntx; tix++) {
-         bool side = false;  // the tile's columns meet an x or y layer: every plane
-         for (int q = 2 + tix * TX; q < std::min(2 + (tix + 1) * TX, ni - 2); q++) side = side || ox[q];
-         for (int q = 2 + tjy * TY; q < std::min(2 + (tjy + 1) * TY, nj - 2); q++) side = side || oy[q];
+         const bool side = meets(tix, tjy);
          for (int c = 0; c < (int)per_chunk.size(); c++) {
             const int ka = k1 + c * kc, kb = std::min(k2, ka + kc - 1);
             int lo = kb + 1, hi = ka - 1;  // planes of the chunk to run
@@ -1210,11 +1252,11 @@ int launch_damp_lds(const Box& b, int k1, int k2, int kc, double* up, const doub
       return check_hip(hipGetLastError(), "damping sweep launch");
    }
    const long nx = b.ie - b.ib - 3, ny = b.je - b.jb - 3;
-   if (kc <= 0) kc = 64;
    constexpr int DTY = 8;
    TileMap map;
    map.ntx = (int)cdiv(nx, TX);
    map.nty = (int)cdiv(ny, DTY);
+   if (kc <= 0) kc = march_kchunk((long)map.ntx * map.nty, k2 - k1 + 1, 3);
    map.ntiles = map.ntx * map.nty * (int)cdiv(k2 - k1 + 1, kc);
    static_assert(DTY == TY, "the asynchronous-load damping sweep uses the sweeps' tile");
    if (dma_fits(b, u, um, rho) && ((uintptr_t)up & 15) == 0)
@@ -1253,8 +1295,12 @@ struct SlabSten {
 // acc = (up - 2u + um) dt2i staged in the slab; DAMP = false: without the
 // damping (a damping sweep over these rows follows; the damping's registers
 // would push this kernel's 256 into 130 accumulator-register copies).
-template <bool CORR, bool DAMP = CORR>
-__global__ void __launch_bounds__(NT, 1)
+// G groups of NT threads share the slab and take the rows kr = 1 + group + G
+// block.y, the next G gridDim.y on: one group evaluates its rows one after
+// the other, each a long chain at one wave per SIMD, so more groups (and, on
+// grids whose tiles leave CUs idle, the rows spread over block.y) shorten it.
+template <bool CORR, bool DAMP, int G>
+__global__ void __launch_bounds__(NT * G, 1)
 k_sbp_rows(Box b, int top, int nk, int ntx, const SbpTables* __restrict__ sbp, const double* __restrict__ upin,
            const double* __restrict__ u, const double* __restrict__ um, const double* __restrict__ mu,
            const double* __restrict__ la, const double* __restrict__ rho, SgCoef sg, double* __restrict__ out,
@@ -1270,7 +1316,9 @@ k_sbp_rows(Box b, int top, int nk, int ntx, const SbpTables* __restrict__ sbp, c
    __shared__ __align__(16) double sl[8 * PL];
    __shared__ double ssx[HX], ssy[HY];
    const int tix = blockIdx.x % ntx, tjy = blockIdx.x / ntx;
-   const int tid = threadIdx.x, tx = tid % TX, ty = tid / TX;
+   // thread of the group, group of the workgroup (whole waves: uniform in a wave)
+   const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
+   const int tid = threadIdx.x - grp * NT, tx = tid % TX, ty = tid / TX;
    const int ia = b.ib + tix * TX, ja = b.jb + tjy * TY;
    const int i = ia + 2 + tx, j = ja + 2 + ty;
    const bool active = i <= b.ie - 2 && j <= b.je - 2;
@@ -1303,7 +1351,7 @@ k_sbp_rows(Box b, int top, int nk, int ntx, const SbpTables* __restrict__ sbp, c
          moff = e < PL && gi <= b.ie && gj <= b.je ? (gi - b.ib) + ni * (gj - b.jb) : 0;
       }
 #pragma unroll 1
-      for (int q = 0; q <= 8; q++) {
+      for (int q = grp; q <= 8; q += G) {
          const long pb = nij * (kbase + sgn * (q - 1) - b.kb);
          double* dst = su + q * 3 * PL + 2 * 64 * wv;
 #pragma unroll
@@ -1317,7 +1365,7 @@ k_sbp_rows(Box b, int top, int nk, int ntx, const SbpTables* __restrict__ sbp, c
       }
    }
 #pragma unroll 1
-   for (int q = 0; q <= 8 && !async; q++) {
+   for (int q = grp; q <= 8 && !async; q += G) {
       const long pb = nij * (kbase + sgn * (q - 1) - b.kb);
 #pragma unroll
       for (int p = 0; p < NU; p++) {
@@ -1350,8 +1398,8 @@ k_sbp_rows(Box b, int top, int nk, int ntx, const SbpTables* __restrict__ sbp, c
          }
       }
    }
-   if (tid < HX) ssx[tid] = ia + tid <= b.ie ? sg.strx[ia + tid - b.ib] : 1.0;
-   if (tid >= 64 && tid < 64 + HY) ssy[tid - 64] = ja + tid - 64 <= b.je ? sg.stry[ja + tid - 64 - b.jb] : 1.0;
+   if (grp == 0 && tid < HX) ssx[tid] = ia + tid <= b.ie ? sg.strx[ia + tid - b.ib] : 1.0;
+   if (grp == 0 && tid >= 64 && tid < 64 + HY) ssy[tid - 64] = ja + tid - 64 <= b.je ? sg.stry[ja + tid - 64 - b.jb] : 1.0;
    __syncthreads();
    if (!active) return;
    SlabSten st{su + o, sm + o, sl + o, ssx + tx + 2, ssy + ty + 2};
@@ -1364,7 +1412,7 @@ k_sbp_rows(Box b, int top, int nk, int ntx, const SbpTables* __restrict__ sbp, c
                     (sg.dcx[ii - 1] != 0 || sg.dcx[ii] != 0 || sg.dcx[ii + 1] != 0 || sg.dcy[jj - 1] != 0 ||
                      sg.dcy[jj] != 0 || sg.dcy[jj + 1] != 0);
 #pragma unroll 1
-   for (int kr = 1; kr <= 6; kr++) {
+   for (int kr = 1 + grp + G * (int)blockIdx.y; kr <= 6; kr += G * (int)gridDim.y) {
       const int k = kbase + sgn * (kr - 1);
       double r[3];
       sbp_row_body(st, kr, (double)sgn, sbp, r);
@@ -1430,16 +1478,24 @@ int launch_sbp_rows(bool corr, const Box& b, int side, int nk, const SbpTables* 
    const long nx = b.ie - b.ib - 3, ny = b.je - b.jb - 3;
    const int ntx = (int)cdiv(nx, TX), nty = (int)cdiv(ny, TY);
    const double cof = 1.0 / (h * h), dt2i = 1.0 / (dt * dt);
+   // two groups of three rows (a third group would spill 110 registers); one
+   // row each where that still leaves every workgroup a CU of its own (the
+   // slab fills a CU's LDS).  Predictor and corrector rows: 62 + 60 -> 18 +
+   // 17 us at 40 x 36, 157 + 181 -> 129 + 122 us at 301 x 301 points.
+   constexpr int G = 2;
+   const dim3 grd(ntx * nty, 3 * ntx * nty <= compute_units() ? 3 : 1);
    if (corr && beta == 0)
-      k_sbp_rows<true, false><<<ntx * nty, NT, 0, s>>>(b, side == 4, nk, ntx, d_sbp, upin, u, um, mu, la, rho, sg,
-                                                       out, cof, dt2i, dt * dt * dt * dt / 12, 0.0,
-                                                       acc && dma_fits(b, acc, mu, la), acc);
-   else if (corr)
-      k_sbp_rows<true><<<ntx * nty, NT, 0, s>>>(b, side == 4, nk, ntx, d_sbp, upin, u, um, mu, la, rho, sg, out, cof,
-                                                dt2i, dt * dt * dt * dt / 12, beta, acc && dma_fits(b, acc, mu, la), acc);
+      k_sbp_rows<true, false, G><<<grd, G * NT, 0, s>>>(b, side == 4, nk, ntx, d_sbp, upin, u, um, mu, la, rho, sg,
+                                                        out, cof, dt2i, dt * dt * dt * dt / 12, 0.0,
+                                                        acc && dma_fits(b, acc, mu, la), acc);
+   else if (corr)  // the damping's registers leave room for one group only
+      k_sbp_rows<true, true, 1><<<ntx * nty, NT, 0, s>>>(b, side == 4, nk, ntx, d_sbp, upin, u, um, mu, la, rho, sg,
+                                                         out, cof, dt2i, dt * dt * dt * dt / 12, beta,
+                                                         acc && dma_fits(b, acc, mu, la), acc);
    else
-      k_sbp_rows<false><<<ntx * nty, NT, 0, s>>>(b, side == 4, nk, ntx, d_sbp, nullptr, u, um, mu, la, rho, sg, out,
-                                                 cof, dt2i, dt * dt, beta, dma_fits(b, u, mu, la), nullptr);
+      k_sbp_rows<false, false, G><<<grd, G * NT, 0, s>>>(b, side == 4, nk, ntx, d_sbp, nullptr, u, um, mu, la, rho, sg,
+                                                         out, cof, dt2i, dt * dt, beta, dma_fits(b, u, mu, la),
+                                                         nullptr);
    return check_hip(hipGetLastError(), "SBP rows launch");
 }
 
@@ -1449,10 +1505,10 @@ int launch_sweep_lds(bool corr, int variant, const Box& b, int k1, int k2, int k
 {
    if (k2 < k1) return OK;
    const long nx = b.ie - b.ib - 3, ny = b.je - b.jb - 3;
-   if (kc <= 0) kc = 32;
    TileMap map;
    map.ntx = (int)cdiv(nx, TX);
    map.nty = (int)cdiv(ny, TY);
+   if (kc <= 0) kc = march_kchunk((long)map.ntx * map.nty, k2 - k1 + 1, 2);
    map.ntiles = map.ntx * map.nty * (int)cdiv(k2 - k1 + 1, kc);
    const unsigned grd = 8 * cdiv(map.ntiles, 8);
    const double cof = 1.0 / (h * h), dt2i = 1.0 / (dt * dt);
@@ -1520,10 +1576,10 @@ int launch_sweep_lds_T(const Box& b, int k1, int k2, int kc, const double* w, co
 {
    if (k2 < k1) return OK;
    const long nx = b.ie - b.ib - 3, ny = b.je - b.jb - 3;
-   if (kc <= 0) kc = 32;
    TileMap map;
    map.ntx = (int)cdiv(nx, TX);
    map.nty = (int)cdiv(ny, TY);
+   if (kc <= 0) kc = march_kchunk((long)map.ntx * map.nty, k2 - k1 + 1, 2);
    map.ntiles = map.ntx * map.nty * (int)cdiv(k2 - k1 + 1, kc);
    const unsigned grd = 8 * cdiv(map.ntiles, 8);
    // rows of odd length by four-byte asynchronous loads (the same results)

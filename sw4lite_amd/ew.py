@@ -299,8 +299,8 @@ class EW:
         where the damping profiles are nonzero (same bits), 10 as 9 with
         rows of odd length staged by four-byte asynchronous loads and the
         acceleration stored for them too (the default; same bits)).
-        kchunk > 0: planes per workgroup of every sweep; 0: the library's
-        defaults (64 for the predictor and corrector, 32 for the damping)."""
+        kchunk > 0: planes per workgroup of every sweep; 0: chosen from the
+        grid's size (the default)."""
         L.check(self.lib.sw4hip_ew_set_kernel_variant(self.h, int(variant), int(kchunk)))
 
     def npoints(self):
