@@ -22,6 +22,7 @@
 // The terms are those of the reference; the grouping of sums is this file's.
 #include "kernels_common.h"
 #include "kernels_curv.h"
+#include "kernels_fast.h"
 
 namespace sw4amd {
 
@@ -161,7 +162,7 @@ __device__ __forceinline__ void t_terms(const S& s, int i, int j, int m, double 
    T[2] = la * a4 * p0 * isy + mu * a2 * p2 * sx * isy + mu * a3 * q2 * sy * isx + la * a4 * q1 * isx;
 }
 
-template <bool BND, class S>
+template <class S>
 __device__ __forceinline__ void curv_point(const S& s, int i, int j, int k, const SbpTables* __restrict__ sbp,
                                            double r[3])
 {
@@ -199,24 +200,7 @@ __device__ __forceinline__ void curv_point(const S& s, int i, int j, int k, cons
    // rr
    const double S3[3][3] = {{isxy, 1, isy}, {1, isxy, isx}, {isy, isx, isxy}};
    const int PAIR[3][3] = {{0, 3, 4}, {3, 1, 5}, {4, 5, 2}};
-   if (!BND) {
-      double R[5][6];
-#pragma unroll
-      for (int t = 0; t < 5; t++) rr_coef(s, i, j, k + t - 2, sx, sy, R[t]);
-#pragma unroll
-      for (int c = 0; c < 3; c++)
-#pragma unroll
-         for (int d = 0; d < 3; d++) {
-            double a[5], m[4], f[5];
-#pragma unroll
-            for (int t = 0; t < 5; t++) {
-               a[t] = R[t][PAIR[c][d]];
-               f[t] = s.U(d, i, j, k + t - 2);
-            }
-            vc4(a, m);
-            r[c] += i6 * vs4(m, f) * S3[c][d];
-         }
-   } else {
+   {
       // C_ab(q) = sum_m acof(k,q,m) R_ab(m), planes 1..8, then the ghost term
 #pragma unroll 1
       for (int q = 1; q <= 8; q++) {
@@ -256,13 +240,13 @@ __device__ __forceinline__ void curv_point(const S& s, int i, int j, int k, cons
    }
 
    // k-derivative weights of this row
-   constexpr int NQ = BND ? 8 : 4;
+   constexpr int NQ = 8;
    int kq[NQ];
    double wq[NQ];
 #pragma unroll
    for (int e = 0; e < NQ; e++) {
-      kq[e] = BND ? e + 1 : k + off[e];
-      wq[e] = BND ? sbp->bope[(k - 1) + 6 * e] : wc[e];
+      kq[e] = e + 1;
+      wq[e] = sbp->bope[(k - 1) + 6 * e];
    }
 
    // pr and qr
@@ -310,7 +294,7 @@ __device__ __forceinline__ void curv_point(const S& s, int i, int j, int k, cons
 // Component-blocked layout: capped at 256 registers for 2 waves/SIMD (2-4
 // spilled; 262 registers and 1 wave/SIMD without the cap).  The interleaved
 // layout's index arithmetic would spill ~120 registers under the cap.
-template <int CO, bool BND>
+template <int CO>
 __global__ void __launch_bounds__(256, CO ? 2 : 1)
 k_rhs4curv(Box b, int klo, int khi, const SbpTables* __restrict__ sbp, CurvG<CO> s,
            const double* __restrict__ jac, double* __restrict__ lu)
@@ -320,10 +304,273 @@ k_rhs4curv(Box b, int klo, int khi, const SbpTables* __restrict__ sbp, CurvG<CO>
    const int k = klo + blockIdx.z;
    if (i > b.ie - 2 || j > b.je - 2 || k > khi) return;
    double r[3];
-   curv_point<BND>(s, i, j, k, sbp, r);
+   curv_point(s, i, j, k, sbp, r);
    const double ij = s.SX(i) * s.SY(j) / jac[sidx(b, i, j, k)];
 #pragma unroll
    for (int c = 0; c < 3; c++) lu[vidx<CO>(b, c, i, j, k)] = r[c] * ij;
+}
+
+// The interior rows as a k-march with every first derivative formed once.
+// Grouped by the outer derivative the operator is
+//   r = pp + qq + rr + D_p F + D_q G + D_r T,
+// F, G, T the products of material, metric and first derivatives at one
+// point (the flux-like sums whose D_p, D_q, D_r are pq and rp, qp and rq, pr
+// and qr), so a point forms its nine first derivatives and nine products
+// once and its neighbours read the products, instead of every output forming
+// them for its twelve neighbours (about 700 operations a point instead of
+// 2126).  A workgroup owns a 32 x 8 tile; each of the 36 x 12 points of the
+// tile with its halo has a thread (four waves of outputs, two of the j halo,
+// one of the i halo and corners), which loads its point's nine values one
+// plane ahead and keeps the column n-4..n of the material and the metric in
+// registers (that of u in LDS).  Per plane n: u and
+// (mu, lambda) M1^2 go to LDS, one barrier, the in-plane derivatives give
+// pp + qq and T of plane n; plane n-2 gets F and G (to LDS, read after the
+// next barrier) and rr + D_r T; plane n-3 is finished.  The rings have five
+// slots and the plane loop is unrolled by five, so every index is a constant
+// and nothing is moved between registers.
+// Bound by latency and VALU issue at 2 waves/SIMD (one workgroup per CU, 252
+// registers): 384x384x256 points 1.90 ms against 6.7 ms of a thread per point reading every
+// neighbour through the caches (2126 operations, 256 registers).
+// (the scheduler would otherwise hoist the shared-memory reads of a whole
+// plane to its start and spill)
+#define SW4_SCHED_FENCE __builtin_amdgcn_sched_barrier(0)
+constexpr int MTX = 32, MTY = 8, MHX = MTX + 4, MHY = MTY + 4, MPL = MHX * MHY, MNT = 448;
+
+template <int CO>
+__global__ void __launch_bounds__(MNT, 1)
+k_rhs4curv_march(Box b, int ntx, int nty, int ntiles, int klo, int khi, int kc, CurvG<CO> s,
+                 const double* __restrict__ jac, double* __restrict__ lu)
+{
+   __shared__ double su[5][3 * MPL];               // u of planes n-4..n
+   __shared__ double se[2][2 * MPL];               // mu M1^2, lambda M1^2 of plane n
+   __shared__ double sf[2][3 * MHX * MTY];         // F over the tile's rows, i halo included
+   __shared__ double sg[2][3 * MTX * MHY];         // G over the tile's columns, j halo included
+   __shared__ double ssx[MHX], ssy[MHY];
+   // XCD-aware order: a contiguous run of tiles per XCD (blocks go to the 8 XCDs round-robin)
+   const int per = (ntiles + 7) / 8;
+   const int t = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+   if (t >= ntiles) return;
+   const int tix = t % ntx, tr = t / ntx, tjy = tr % nty, tkz = tr / nty;
+   const int k0 = klo + tkz * kc, k1 = min(khi, k0 + kc - 1);
+   const int tid = threadIdx.x;
+   // 0: output, 1: j halo, 2: i halo (and corners)
+   const int role = __builtin_amdgcn_readfirstlane(tid < 256 ? 0 : tid < 384 ? 1 : 2);
+   int hx, hy;
+   if (tid < 256) {
+      hx = 2 + tid % MTX;
+      hy = 2 + tid / MTX;
+   } else if (tid < 384) {
+      const int r = (tid - 256) / MTX;
+      hx = 2 + tid % MTX;
+      hy = r < 2 ? r : r + MTY;
+   } else {
+      const int q = tid - 384, c = q % 4, r = q / 4;  // rows 0..7: the tile's, 8..11: the corners'
+      hx = c < 2 ? c : c + MTX;
+      hy = r < MTY ? 2 + r : r < MTY + 2 ? r - MTY : r < MTY + 4 ? r : 2;
+   }
+   const bool own = tid < MPL;  // the last 16 threads repeat a point and store nothing
+   const Box& b_ = b;
+   const int ia = b_.ib + tix * MTX, ja = b_.jb + tjy * MTY;
+   const bool active = role == 0 && ia + hx <= b_.ie - 2 && ja + hy <= b_.je - 2;
+   // points off the box repeat its last row or column: read by inactive outputs only
+   const int i = min(ia + hx, b_.ie), j = min(ja + hy, b_.je);
+   const long nij = b_.nij, npts = b_.npts;
+   const long col = (i - b_.ib) + b_.ni * (j - b_.jb);
+   const double sx = s.SX(i), sy = s.SY(j), isx = 1 / sx, isy = 1 / sy;
+   if (tid < MHX) ssx[tid] = s.SX(min(ia + tid, b_.ie));
+   if (tid >= 64 && tid < 64 + MHY) ssy[tid - 64] = s.SY(min(ja + tid - 64, b_.je));
+   const int o = hy * MHX + hx;
+
+   double mu[5], la[5], m1[5], m2[5], m3[5], m4[5];  // column ring
+   double pq[5][4];                                  // D_p u, D_p v, D_q u, D_q v
+   // pp + qq + rr + D_r T, the terms of D_r T added as their planes come
+   double acc[5][3] = {};
+   double rp[3] = {0, 0, 0};                         // acc of the plane finished next
+   double nu[3], nmu, nla, nm[4], njac = 1.0;                 // loaded one plane ahead
+   auto load = [&](int kk) {
+      const long p = col + nij * (kk - b_.kb);
+#pragma unroll
+      for (int c = 0; c < 3; c++) nu[c] = s.u[CO ? p + npts * c : 3 * p + c];
+      nmu = s.mu[p];
+      nla = s.la[p];
+#pragma unroll
+      for (int c = 0; c < 4; c++) nm[c] = s.met[CO ? p + npts * c : 4 * p + c];
+   };
+   auto D = [](double fm2, double fm1, double fp1, double fp2) { return CC2 * (fp2 - fm2) + CC1 * (fp1 - fm1); };
+   load(k0 - 2);
+   int par = 0;
+   for (int n0 = k0 - 2; n0 <= k1 + 3; n0 += 5) {
+#pragma unroll
+      for (int ph = 0; ph < 5; ph++) {
+         const int n = n0 + ph;
+         if (n > k1 + 3) break;
+         const int s0 = ph, s1 = (ph + 4) % 5, s2 = (ph + 3) % 5, s3 = (ph + 2) % 5, s4 = (ph + 1) % 5;  // n..n-4
+         const double cjac = njac;
+         if (n <= k1 + 2) {
+            mu[s0] = nmu;
+            la[s0] = nla;
+            m1[s0] = nm[0];
+            m2[s0] = nm[1];
+            m3[s0] = nm[2];
+            m4[s0] = nm[3];
+            if (own) {
+               const double q = m1[s0] * m1[s0];
+#pragma unroll
+               for (int c = 0; c < 3; c++) su[s0][c * MPL + o] = nu[c];
+               se[par][o] = mu[s0] * q;
+               se[par][MPL + o] = la[s0] * q;
+            }
+         }
+         __syncthreads();  // plane n is in su, se, F and G of plane n-3 in sf, sg[par ^ 1]
+         if (n < k1 + 2) load(n + 1);
+         if (role == 0 && n >= k0 + 2) njac = jac[col + nij * (n - 2 - b_.kb)];
+         if (role == 0 && n >= k0 + 3 && active) {  // finish plane n-3
+            const double* f = &sf[par ^ 1][(hy - 2) * MHX + hx];
+            const double* g = &sg[par ^ 1][hy * MTX + hx - 2];
+            const double w = sx * sy / cjac;
+            const long p = col + nij * (n - 3 - b_.kb);
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+               const double* fc = f + c * MHX * MTY;
+               const double* gc = g + c * MTX * MHY;
+               const double r = rp[c] + D(fc[-2], fc[-1], fc[1], fc[2]) +
+                                D(gc[-2 * MTX], gc[-MTX], gc[MTX], gc[2 * MTX]);
+               lu[CO ? p + npts * c : 3 * p + c] = r * w;
+            }
+         }
+         if (n > k1 + 2) break;
+         SW4_SCHED_FENCE;
+         // in-plane derivatives of plane n
+         const double* pu = su[s0] + o;
+         const double* pe = se[par] + o;
+         if (role == 0) {
+            // pp and qq coefficients: cx, cy for the component along the axis, mx, my for the others
+            double mx[4], my[4], cx[4], cy[4], p[3], q[3];
+            {
+               double am[5], al[5];
+#pragma unroll
+               for (int e = 0; e < 5; e++) {
+                  am[e] = pe[e - 2] * ssx[hx + e - 2];
+                  al[e] = pe[MPL + e - 2] * ssx[hx + e - 2];
+               }
+               vc4(am, mx);
+               vc4(al, cx);
+#pragma unroll
+               for (int e = 0; e < 5; e++) {
+                  am[e] = pe[(e - 2) * MHX] * ssy[hy + e - 2];
+                  al[e] = pe[MPL + (e - 2) * MHX] * ssy[hy + e - 2];
+               }
+               vc4(am, my);
+               vc4(al, cy);
+#pragma unroll
+               for (int e = 0; e < 4; e++) {
+                  cx[e] += 2 * mx[e];
+                  cy[e] += 2 * my[e];
+               }
+            }
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+               SW4_SCHED_FENCE;
+               const double* f = pu + c * MPL;
+               const double x0 = f[-2], x1 = f[-1], x3 = f[1], x4 = f[2];
+               const double y0 = f[-2 * MHX], y1 = f[-MHX], y3 = f[MHX], y4 = f[2 * MHX], u0 = f[0];
+               p[c] = D(x0, x1, x3, x4);
+               q[c] = D(y0, y1, y3, y4);
+               const double* wx = c == 0 ? cx : mx;
+               const double* wy = c == 1 ? cy : my;
+               const double ax = wx[0] * (x0 - u0) + wx[1] * (x1 - u0) + wx[2] * (x3 - u0) + wx[3] * (x4 - u0);
+               const double ay = wy[0] * (y0 - u0) + wy[1] * (y1 - u0) + wy[2] * (y3 - u0) + wy[3] * (y4 - u0);
+               acc[s0][c] += (1.0 / 6) * (ax * isy + ay * isx);
+            }
+            SW4_SCHED_FENCE;
+            pq[s0][0] = p[0];
+            pq[s0][1] = p[1];
+            pq[s0][2] = q[0];
+            pq[s0][3] = q[1];
+            {
+               const double a2 = m2[s0] * m1[s0], a3 = m3[s0] * m1[s0], a4 = m4[s0] * m1[s0];
+               const double xy = sx * isy, yx = sy * isx, K = 2 * mu[s0] + la[s0];
+               double T[3];
+               T[0] = K * a2 * xy * p[0] + mu[s0] * (a3 * p[1] + a4 * isy * p[2] + a3 * yx * q[0]) + la[s0] * a2 * q[1];
+               T[1] = la[s0] * a3 * p[0] + mu[s0] * (a2 * xy * p[1] + a2 * q[0] + a4 * isx * q[2]) + K * a3 * yx * q[1];
+               T[2] = la[s0] * a4 * (isy * p[0] + isx * q[1]) + mu[s0] * (a2 * xy * p[2] + a3 * yx * q[2]);
+#pragma unroll
+               for (int c = 0; c < 3; c++) {  // D_r T of planes n-2, n-1, n+1 and (its first term) n+2
+                  acc[s2][c] += CC2 * T[c];
+                  acc[s1][c] += CC1 * T[c];
+                  acc[s4][c] -= CC1 * T[c];
+                  acc[s3][c] = -CC2 * T[c];
+               }
+            }
+         } else if (role == 1) {
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+               const double* f = pu + c * MPL;
+               pq[s0][c] = D(f[-2], f[-1], f[1], f[2]);
+            }
+         } else if (tid < 384 + 4 * MTY) {
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+               const double* f = pu + c * MPL;
+               pq[s0][2 + c] = D(f[-2 * MHX], f[-MHX], f[MHX], f[2 * MHX]);
+            }
+         }
+         SW4_SCHED_FENCE;
+         // plane k = n-2: F, G and the terms along the column
+         if (n >= k0 + 2) {
+            double dz[3];
+#pragma unroll
+            for (int c = 0; c < 3; c++)
+               dz[c] = D(su[s4][c * MPL + o], su[s3][c * MPL + o], su[s1][c * MPL + o], su[s0][c * MPL + o]);
+            const double q = m1[s2] * m1[s2], a2 = m2[s2] * m1[s2], a3 = m3[s2] * m1[s2], a4 = m4[s2] * m1[s2];
+            const double xy = sx * isy, yx = sy * isx, K = 2 * mu[s2] + la[s2];
+            if (role != 1 && tid < 384 + 4 * MTY) {
+               double* f = &sf[par][(hy - 2) * MHX + hx];
+               f[0] = la[s2] * (q * pq[s2][3] + isy * (a3 * sy * dz[1] + a4 * dz[2])) + K * a2 * xy * dz[0];
+               f[MHX * MTY] = mu[s2] * (q * pq[s2][2] + a3 * dz[0] + a2 * xy * dz[1]);
+               f[2 * MHX * MTY] = mu[s2] * (a4 * dz[0] + a2 * sx * dz[2]) * isy;
+            }
+            if (role != 2) {
+               double* g = &sg[par][hy * MTX + hx - 2];
+               g[0] = mu[s2] * (q * pq[s2][1] + a3 * yx * dz[0] + a2 * dz[1]);
+               g[MTX * MHY] = la[s2] * (q * pq[s2][0] + a2 * dz[0] + a4 * isx * dz[2]) + K * a3 * yx * dz[1];
+               g[2 * MTX * MHY] = mu[s2] * (a3 * sy * dz[2] + a4 * dz[1]) * isx;
+            }
+            SW4_SCHED_FENCE;
+            if (role == 0) {
+               // rr_a = 1/(6 sx sy) sum_t [mu |m|^2 w_a + (mu + lambda) m_a (m . w)]_t with m = (M2 sx, M3 sy, M4)
+               // and w_t the weights of plane t's coefficient (a combination of u(k+q) - u(k))
+               double w[5][3], rr[3] = {0, 0, 0};
+#pragma unroll
+               for (int c = 0; c < 3; c++) {
+                  const int q = c * MPL + o;
+                  const double u0 = su[s2][q], d0 = su[s4][q] - u0, d1 = su[s3][q] - u0, d3 = su[s1][q] - u0,
+                               d4 = su[s0][q] - u0;
+                  w[0][c] = d1 - 0.75 * d0;
+                  w[1][c] = d0 + 3 * d1 + d3;
+                  w[2][c] = 3 * (d1 + d3) - 0.75 * (d0 + d4);
+                  w[3][c] = d1 + 3 * d3 + d4;
+                  w[4][c] = d3 - 0.75 * d4;
+               }
+#pragma unroll
+               for (int e = 0; e < 5; e++) {
+                  const int se = (s0 + 1 + e) % 5;  // plane k - 2 + e
+                  const double x = m2[se] * sx, y = m3[se] * sy, z = m4[se];
+                  const double mn = mu[se] * (x * x + y * y + z * z);
+                  const double ml = (mu[se] + la[se]) * (x * w[e][0] + y * w[e][1] + z * w[e][2]);
+                  rr[0] += mn * w[e][0] + ml * x;
+                  rr[1] += mn * w[e][1] + ml * y;
+                  rr[2] += mn * w[e][2] + ml * z;
+               }
+               const double i6xy = (1.0 / 6) * isx * isy;
+#pragma unroll
+               for (int c = 0; c < 3; c++)
+                  rp[c] = acc[s2][c] + i6xy * rr[c];
+            }
+         }
+         par ^= 1;
+      }
+   }
 }
 
 // ---------------------------------------------------------------------------
@@ -510,10 +757,13 @@ static void rhs4curv_co(const Box& b, const int* onesided, const SbpTables* d_sb
    dim3 blk(64, 4, 1);
    const int top = onesided[4] == 1;
    const int k1 = top ? 7 : b.kb + 2, k2 = b.ke - 2;
-   if (top) k_rhs4curv<CO, true><<<dim3(cdiv(nii, 64), cdiv(njj, 4), 6), blk, 0, s>>>(b, 1, 6, d_sbp, cg, jac, lu);
-   if (k2 >= k1)
-      k_rhs4curv<CO, false><<<dim3(cdiv(nii, 64), cdiv(njj, 4), k2 - k1 + 1), blk, 0, s>>>(b, k1, k2, d_sbp, cg, jac,
-                                                                                           lu);
+   if (top) k_rhs4curv<CO><<<dim3(cdiv(nii, 64), cdiv(njj, 4), 6), blk, 0, s>>>(b, 1, 6, d_sbp, cg, jac, lu);
+   if (k2 >= k1) {
+      const int ntx = (int)cdiv(nii, MTX), nty = (int)cdiv(njj, MTY);
+      const int kc = march_kchunk((long)ntx * nty, k2 - k1 + 1, 1);
+      const int ntiles = ntx * nty * (int)cdiv(k2 - k1 + 1, kc);
+      k_rhs4curv_march<CO><<<8 * cdiv(ntiles, 8), MNT, 0, s>>>(b, ntx, nty, ntiles, k1, k2, kc, cg, jac, lu);
+   }
 }
 
 int launch_rhs4sgcurv(int co, const Box& b, const int* onesided, const SbpTables* d_sbp, const double* u,

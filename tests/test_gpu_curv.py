@@ -88,6 +88,18 @@ def test_metric_rejects_folded_grid(torch):
 def test_rhs4sgcurv(torch, coefs, corder, top, shape):
     """Against the oracle on an odd and an even row length, with and without
     the top SBP rows."""
+    check_rhs4sgcurv(torch, coefs, corder, top, shape)
+
+
+@pytest.mark.parametrize("shape", [(200, 150, 40), (161, 201, 44), (32, 8, 12), (33, 9, 13), (12, 12, 12)])
+def test_rhs4sgcurv_march(torch, coefs, shape):
+    """The k-march of the interior rows: marches of many planes (enough tiles
+    to fill the device in one block, and a last block shorter than the
+    others), whole tiles, one column and one row more, the smallest grid."""
+    check_rhs4sgcurv(torch, coefs, 1, 1, shape)
+
+
+def check_rhs4sgcurv(torch, coefs, corder, top, shape):
     from sw4lite_amd import ew
     acof, ghcof, bope, _ = coefs
     box, f, z, met, jac = curved(70 + top, *shape, 0.1)
