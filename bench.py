@@ -56,7 +56,7 @@ COMP_CORR_BYTES_PER_PT = 24 * 4
 COMP_PRED_BYTES_PER_PT = 9 * 4
 COMP_STEP_BYTES_PER_PT = 33 * 4
 STAGES = ["pred_interior", "pred_boundary_rows_shell", "pred_sources_bc", "corr_interior",
-          "corr_interior_damping", "corr_boundary_rows_shell", "corr_sources_bc"]
+          "corr_rows_damping", "corr_tail", "corr_sources_bc"]
 
 
 def parse():

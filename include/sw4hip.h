@@ -362,11 +362,12 @@ int sw4hip_ew_step(sw4hip_ew* ew, int nsteps, int mode);
  * object's stream; stage_ms[7] receives the summed milliseconds of
  * (predictor interior kernel, predictor boundary rows + ghost shell,
  * predictor sources + ghost-point BC, corrector interior kernel, corrector
- * interior supergrid damping, corrector boundary rows + ghost shell,
- * corrector sources + BC).  Synchronises. */
+ * boundary rows + supergrid damping, corrector ghost shell, corrector
+ * sources + BC).  Synchronises. */
 int sw4hip_ew_step_timed(sw4hip_ew* ew, int nsteps, double* stage_ms);
 /* Mode 2 (FP32, compensated) with the same per-stage times; the supergrid
- * damping is part of the corrector sweep, so stage 5 reads 0. */
+ * damping is part of the corrector sweep: stage 5 reads 0 and stage 6 holds
+ * the corrector's boundary rows + ghost shell. */
 int sw4hip_ew_step_comp_timed(sw4hip_ew* ew, int nsteps, double* stage_ms);
 /* Analytic point-source error of the current U (EW::exactSol +
  * normOfDifference, EW.C:3650-3669, 4526-4610). */

@@ -52,7 +52,7 @@ int EW::fused_once(double t, double* acc)
    const DampTile* dtiles = nullptr;
    int ndtiles = 0;
    int rc;
-   if ((rc = damp_tile_list(ka, kz, &dtiles, &ndtiles))) return rc;
+   if ((rc = damp_tile_list(m_box.kb + 2, m_box.ke - 2, &dtiles, &ndtiles))) return rc;
    if ((rc = launch_pred_fused(m_box, g.nz, m_onesided, m_dsbp, mU.dev, mUm.dev, mMu.dev, mLambda.dev, mRho.dev, c,
                                mUp.dev, g.h, dt, m_stream, nullptr, m_variant, m_kchunk, zf, af)) ||
        (rc = launch_src_apply(m_box, st, t, 0, dt * dt, mRho.dev, mUp.dev, m_stream)) ||

@@ -91,10 +91,7 @@ int Batch::init()
       EW* e = m_shots[q];
       if (e->m_variant < 9) continue;
       const Box& b = e->m_box;
-      const GridSetup& g = e->m_opt.grid;
-      const int k1 = e->m_onesided[4] == 1 ? 7 : b.kb + 2;
-      const int k2 = e->m_onesided[5] == 1 ? g.nz - 6 : b.ke - 2;
-      const std::vector<DampTile> v = damp_tiles(b, k1, k2, EW::kDampChunk, e->m_sg_host.dcx.data(),
+      const std::vector<DampTile> v = damp_tiles(b, b.kb + 2, b.ke - 2, EW::kDampChunk, e->m_sg_host.dcx.data(),
                                                  e->m_sg_host.dcy.data(), e->m_sg_host.dcz.data());
       if (hipMalloc(&p, sizeof(DampTile) * std::max<size_t>(v.size(), 1)) != hipSuccess) {
          (void)hipGetLastError();
@@ -171,8 +168,8 @@ int Batch::build_tables()
    }
    m_useacc.assign(3 * n, 0);
    for (int ph = 0; ph < 3; ph++) {
-      // kinds 0 and 2: the grids whose planes take the asynchronous loads
-      // first (their own launch, block ids from 0), then the others
+      // the grids whose planes take the asynchronous loads first (their own
+      // launch, block ids from 0), then the others
       int g0[3] = {0, 0, 0}, ga[3] = {0, 0, 0}, slot[3] = {0, 0, 0};
       for (int pass = 0; pass < 2; pass++)
          for (int q = 0; q < n; q++) {
@@ -206,7 +203,7 @@ int Batch::build_tables()
                                        e->mRho.dev, c, up2, g.h, e->mDt, e->m_opt.beta, true, gc, d, nullptr, 0,
                                        acc ? m_acc[q] : nullptr);
                else
-                  gc = fill_sweep_shot(true, b, k1, damp ? k2 : k1 - 1, kchunk, nullptr, u, um, nullptr, nullptr,
+                  gc = fill_sweep_shot(true, b, b.kb + 2, damp ? b.ke - 2 : b.kb + 1, kchunk, nullptr, u, um, nullptr, nullptr,
                                        e->mRho.dev, c, up2, g.h, e->mDt, e->m_opt.beta, true, gc, d, m_dtiles[q],
                                        m_ndtiles[q]);
             }
@@ -248,10 +245,12 @@ int Batch::one_step(int ph)
       EW* e = m_shots[q];
       const GridSetup& g = e->m_opt.grid;
       const double* acc = m_useacc[ph * n + q] ? m_acc[q] : nullptr;
-      return launch_corr_tail(e->m_box, g.nz, e->m_onesided, e->m_dsbp, e->mUp.dev, m_base[3 * q + (ph + 1) % 3],
-                              m_base[3 * q + ph % 3], e->mMu.dev, e->mLambda.dev, e->mRho.dev, e->sg(),
-                              e->m_opt.beta, m_base[3 * q + (ph + 2) % 3], g.h, e->mDt, m_side[q % NSIDE], e->zfill(),
-                              acc, e->m_variant >= 9);
+      double* up2 = m_base[3 * q + (ph + 2) % 3];
+      hipStream_t st = m_side[q % NSIDE];
+      const int r = launch_corr_rows(e->m_box, g.nz, e->m_onesided, e->m_dsbp, e->mUp.dev, m_base[3 * q + (ph + 1) % 3],
+                                     m_base[3 * q + ph % 3], e->mMu.dev, e->mLambda.dev, e->mRho.dev, e->sg(), up2,
+                                     g.h, e->mDt, st, acc);
+      return r ? r : launch_corr_shell(e->m_box, e->mUp.dev, up2, st, e->zfill());
    };
    if ((rc = fork())) return rc;
    for (int q = 0; q < n; q++)
@@ -287,8 +286,9 @@ int Batch::one_step(int ph)
       if ((rc = corr_tail(q))) return rc;
    if ((rc = launch_sweep_batch_async(1, tab + n, a1, m_nblk_async[ph][1], m_s)) ||
        (rc = launch_sweep_batch(1, tab + n + a1, n - a1, m_nblk[ph][1], m_s)) ||
+       (rc = join()) ||  // the damping acts on the rows too
        (rc = launch_sweep_batch_async(2, tab + 2 * n, a2, m_nblk_async[ph][2], m_s)) ||
-       (rc = launch_sweep_batch(2, tab + 2 * n + a2, n - a2, m_nblk[ph][2], m_s)) || (rc = join()) || (rc = fork()))
+       (rc = launch_sweep_batch(2, tab + 2 * n + a2, n - a2, m_nblk[ph][2], m_s)) || (rc = fork()))
       return rc;
    for (int q = 0; q < n; q++) {
       EW* e = m_shots[q];

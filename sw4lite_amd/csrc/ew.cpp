@@ -649,7 +649,7 @@ int EW::step_fused(int n, double* stage_ms)
    if (rc == OK && kz >= ka) rc = accel_field(&accf);
    const DampTile* dtiles = nullptr;
    int ndtiles = 0;
-   if (rc == OK) rc = damp_tile_list(ka, kz, &dtiles, &ndtiles);
+   if (rc == OK) rc = damp_tile_list(m_box.kb + 2, m_box.ke - 2, &dtiles, &ndtiles);
    // completes the stored acceleration from the final Up (after sources and BC)
    auto accel_rest = [&](double dt) -> int {
       if (!accf) return OK;

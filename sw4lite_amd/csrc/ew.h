@@ -118,9 +118,9 @@ public:
    int step_reference(int n);  // stage order of EW::timesteploop (EW.C:2527-2842)
    // two fused sweeps per step; with stage_ms, kStages accumulated stage
    // times (ms): predictor interior, predictor boundary rows + ghost shell,
-   // predictor sources + BC, corrector interior, corrector interior damping
-   // (LDS variant; 0 otherwise), corrector boundary rows + ghost shell,
-   // corrector sources + BC
+   // predictor sources + BC, corrector interior, corrector boundary rows +
+   // damping (LDS variants; 0 otherwise), corrector ghost shell (with the rows
+   // in variant 0 and the FP32 form), corrector sources + BC
    static constexpr int kStages = 7;
    int step_fused(int n, double* stage_ms = nullptr);
    // The fused step in FP32 with the compensated time update

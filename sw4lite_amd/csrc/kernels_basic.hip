@@ -9,6 +9,7 @@
 // fused, LDS-staged kernels of the fast step live in kernels_fused.hip and
 // are checked against these.
 #include "kernels_common.h"
+#include "sbp_rows.h"
 
 namespace sw4amd {
 
@@ -31,21 +32,20 @@ k_rhs4_interior(Box b, int klo, int khi, const double* __restrict__ u,
    for (int c = 0; c < 3; c++) lu[vidx<CO>(b, c, i, j, k)] = cof * r[c];
 }
 
+// The six SBP rows next to a free surface (sbp_rows.h).
 template <int CO>
-__global__ void __launch_bounds__(256)
-k_rhs4_sbp(Box b, int top, int nk, const SbpTables* __restrict__ sbp, const double* __restrict__ u,
-           const double* __restrict__ mu, const double* __restrict__ la,
-           const double* __restrict__ strx, const double* __restrict__ stry,
-           double* __restrict__ lu, double cof)
+__global__ void __launch_bounds__(RNT, 1)
+k_rhs4_sbp(Box b, int top, int nk, int ntx, const SbpTables* __restrict__ sbp, const double* __restrict__ u,
+           const double* __restrict__ mu, const double* __restrict__ la, const double* __restrict__ strx,
+           const double* __restrict__ stry, double* __restrict__ lu, double cof)
 {
-   const int i = b.ib + 2 + blockIdx.x * blockDim.x + threadIdx.x;
-   const int j = b.jb + 2 + blockIdx.y * blockDim.y + threadIdx.y;
-   const int kr = 1 + blockIdx.z;  // boundary row 1..6
-   if (i > b.ie - 2 || j > b.je - 2) return;
-   const int k = top ? kr : nk - kr + 1;
-   double r[3];
-   rhs_sbp_point<CO>(b, i, j, k, kr, top ? 1 : nk, top ? 1 : -1, sbp, Plain{u}, mu, la, strx, stry, r);
-   for (int c = 0; c < 3; c++) lu[vidx<CO>(b, c, i, j, k)] = cof * r[c];
+   const long npts = b.npts;
+   sbp_rows_body<double>(
+       b, top, nk, ntx, sbp, mu, la, strx, stry, [=](int c, long p) { return u[CO ? p + npts * c : 3 * p + c]; },
+       [=](int, int, int, long p, const double r[3], const double*) {
+#pragma unroll
+          for (int c = 0; c < 3; c++) lu[CO ? p + npts * c : 3 * p + c] = cof * r[c];
+       });
 }
 
 // ---------------------------------------------------------------------------
@@ -219,11 +219,12 @@ int launch_rhs4sg(int co, const Box& b, int nk, const int* onesided, const SbpTa
    }
    for (int side = 4; side <= 5; side++) {
       if (onesided[side] != 1) continue;
-      dim3 grd(cdiv(nii, 64), cdiv(njj, 4), 6);
+      const int ntx = (int)cdiv(nii, RTX), tiles = ntx * (int)cdiv(njj, RTY);
+      const dim3 grd(tiles, sbp_rows_spread(tiles, 1));
       if (co)
-         k_rhs4_sbp<1><<<grd, blk, 0, s>>>(b, side == 4, nk, d_sbp, u, mu, la, strx, stry, lu, cof);
+         k_rhs4_sbp<1><<<grd, RNT, 0, s>>>(b, side == 4, nk, ntx, d_sbp, u, mu, la, strx, stry, lu, cof);
       else
-         k_rhs4_sbp<0><<<grd, blk, 0, s>>>(b, side == 4, nk, d_sbp, u, mu, la, strx, stry, lu, cof);
+         k_rhs4_sbp<0><<<grd, RNT, 0, s>>>(b, side == 4, nk, ntx, d_sbp, u, mu, la, strx, stry, lu, cof);
    }
    return check_hip(hipGetLastError(), "rhs4sg launch");
 }

@@ -12,7 +12,7 @@
 #include "kernels_comp.h"
 #include "kernels_fast.h"
 #include "kernels_step.h"
-#include "sbp_row_body.h"
+#include "sbp_rows.h"
 #include "stencil_body.h"
 
 namespace sw4amd {
@@ -542,149 +542,106 @@ k_comp_dma(Box b, CompTiles map, int kbeg, int kend, int kc, const float* __rest
    }
 }
 
-// Damping increment of one point from the stored D (addsgd4_point on
-// D = U - Um, ew-cfromfort.C:985-1041), FP32.
-__device__ __forceinline__ void damp_point_f(const Box& b, int i, int j, int k, const float* __restrict__ d,
-                                             const float* __restrict__ rho, const SgCoefF& sg, float beta,
-                                             float out[3])
+// The damping of the corrector on the six SBP rows, into Dn, where
+// k_comp_rows takes it from: its 46 loads a point beside the rows' columns
+// would take that kernel 245 registers and with them the second workgroup
+// per CU.  A thread walks the six rows of a column with D's column in
+// registers.  Columns and rows no damping coefficient reaches get the exact
+// zero they would have.
+__global__ void __launch_bounds__(256)
+k_comp_rows_damp(Box b, int top, int nk, const float* __restrict__ dold, const float* __restrict__ rho, SgCoefF sg,
+                 float* __restrict__ dnew, float beta)
 {
-   const int ii = i - b.ib, jj = j - b.jb, kk = k - b.kb;
-   const float r0 = rho[sidx(b, i, j, k)];
-   const float birho = beta / r0;
-   const float rxp = rho[sidx(b, i + 1, j, k)] * sg.dcx[ii + 1], rx0 = r0 * sg.dcx[ii],
-               rxm = rho[sidx(b, i - 1, j, k)] * sg.dcx[ii - 1];
-   const float ryp = rho[sidx(b, i, j + 1, k)] * sg.dcy[jj + 1], ry0 = r0 * sg.dcy[jj],
-               rym = rho[sidx(b, i, j - 1, k)] * sg.dcy[jj - 1];
-   const float rzp = rho[sidx(b, i, j, k + 1)] * sg.dcz[kk + 1], rz0 = r0 * sg.dcz[kk],
-               rzm = rho[sidx(b, i, j, k - 1)] * sg.dcz[kk - 1];
-   const float wx = sg.strx[ii] * sg.coy[jj] * sg.coz[kk];
-   const float wy = sg.stry[jj] * sg.cox[ii] * sg.coz[kk];
-   const float wz = sg.strz[kk] * sg.cox[ii] * sg.coy[jj];
+   const int i = b.ib + 2 + blockIdx.x * blockDim.x + threadIdx.x;
+   const int j = b.jb + 2 + blockIdx.y * blockDim.y + threadIdx.y;
+   if (i > b.ie - 2 || j > b.je - 2) return;
+   const int ii = i - b.ib, jj = j - b.jb;
+   const float gx0 = sg.dcx[ii - 1], gx1 = sg.dcx[ii], gx2 = sg.dcx[ii + 1];
+   const float gy0 = sg.dcy[jj - 1], gy1 = sg.dcy[jj], gy2 = sg.dcy[jj + 1];
+   const bool dxy = gx0 != 0 || gx1 != 0 || gx2 != 0 || gy0 != 0 || gy1 != 0 || gy2 != 0;
+   const float sxi = sg.strx[ii], cxi = sg.cox[ii], syj = sg.stry[jj], cyj = sg.coy[jj];
+   const int k0 = top ? 1 : nk - 5;
+   const long ni = b.ni, nij = b.nij, npts = b.npts;
+   const long p0 = ii + ni * jj + nij * (k0 - b.kb);
+   float q[5][3], rm = rho[p0 - nij], r0 = rho[p0];
 #pragma unroll
-   for (int c = 0; c < 3; c++) {
-      float dx[5], dy[5], dz[5];
+   for (int t = 0; t < 4; t++)
 #pragma unroll
-      for (int t = 0; t < 5; t++) {
-         dx[t] = d[vidx<1>(b, c, i + t - 2, j, k)];
-         dy[t] = d[vidx<1>(b, c, i, j + t - 2, k)];
-         dz[t] = d[vidx<1>(b, c, i, j, k + t - 2)];
+      for (int c = 0; c < 3; c++) q[t][c] = dold[p0 + nij * (t - 2) + npts * c];
+#pragma unroll 1
+   for (int k = k0; k < k0 + 6; k++) {
+      const long p = p0 + nij * (k - k0);
+      const int kk = k - b.kb;
+      const float gz0 = sg.dcz[kk - 1], gz1 = sg.dcz[kk], gz2 = sg.dcz[kk + 1];
+      const float rp = rho[p + nij];
+#pragma unroll
+      for (int c = 0; c < 3; c++) q[4][c] = dold[p + 2 * nij + npts * c];
+      float out[3] = {0, 0, 0};
+      if (dxy || gz0 != 0 || gz1 != 0 || gz2 != 0) {
+         const float birho = beta / r0, szk = sg.strz[kk], czk = sg.coz[kk];
+         const float rxp = rho[p + 1] * gx2, rx0 = r0 * gx1, rxm = rho[p - 1] * gx0;
+         const float ryp = rho[p + ni] * gy2, ry0 = r0 * gy1, rym = rho[p - ni] * gy0;
+         const float rzp = rp * gz2, rz0 = r0 * gz1, rzm = rm * gz0;
+         const float wx = sxi * cyj * czk, wy = syj * cxi * czk, wz = szk * cxi * cyj;
+#pragma unroll
+         for (int c = 0; c < 3; c++) {
+            const float* d = dold + p + npts * c;
+            const float ax = rxp * (d[2] - 2 * d[1] + q[2][c]) - 2 * rx0 * (d[1] - 2 * q[2][c] + d[-1]) +
+                             rxm * (q[2][c] - 2 * d[-1] + d[-2]);
+            const float ay = ryp * (d[2 * ni] - 2 * d[ni] + q[2][c]) - 2 * ry0 * (d[ni] - 2 * q[2][c] + d[-ni]) +
+                             rym * (q[2][c] - 2 * d[-ni] + d[-2 * ni]);
+            const float az = rzp * (q[4][c] - 2 * q[3][c] + q[2][c]) - 2 * rz0 * (q[3][c] - 2 * q[2][c] + q[1][c]) +
+                             rzm * (q[2][c] - 2 * q[1][c] + q[0][c]);
+            out[c] = birho * (wx * ax + wy * ay + wz * az);
+         }
       }
-      const float ax = rxp * (dx[4] - 2 * dx[3] + dx[2]) - 2 * rx0 * (dx[3] - 2 * dx[2] + dx[1]) +
-                       rxm * (dx[2] - 2 * dx[1] + dx[0]);
-      const float ay = ryp * (dy[4] - 2 * dy[3] + dy[2]) - 2 * ry0 * (dy[3] - 2 * dy[2] + dy[1]) +
-                       rym * (dy[2] - 2 * dy[1] + dy[0]);
-      const float az = rzp * (dz[4] - 2 * dz[3] + dz[2]) - 2 * rz0 * (dz[3] - 2 * dz[2] + dz[1]) +
-                       rzm * (dz[2] - 2 * dz[1] + dz[0]);
-      out[c] = birho * (wx * ax + wy * ay + wz * az);
+#pragma unroll
+      for (int c = 0; c < 3; c++) dnew[p + npts * c] = out[c];
+#pragma unroll
+      for (int t = 0; t < 4; t++)
+#pragma unroll
+         for (int c = 0; c < 3; c++) q[t][c] = q[t + 1][c];
+      rm = r0;
+      r0 = rp;
    }
 }
 
-// Row-space accessor of the staged slab (sbp_row_body.h), FP32.
-struct SlabStenF {
-   const float* ub;  // staged plane q = 0 at this thread's point
-   const float* mb;  // mu plane q = 1
-   const float* lb;
-   const float* psx;
-   const float* psy;
-   __device__ __forceinline__ float u(int c, int di, int dj, int q) const { return ub[(q * 3 + c) * PL + dj * HX + di]; }
-   __device__ __forceinline__ float mu(int di, int dj, int q) const { return mb[(q - 1) * PL + dj * HX + di]; }
-   __device__ __forceinline__ float la(int di, int dj, int q) const { return lb[(q - 1) * PL + dj * HX + di]; }
-   __device__ __forceinline__ float sx(int d) const { return psx[d]; }
-   __device__ __forceinline__ float sy(int d) const { return psy[d]; }
-};
-
-// The six SBP rows at a free surface (top: k = 1..6, bottom: nk..nk-5), one
-// 32 x 8 tile per workgroup with nine planes of U (predictor) or A
-// (corrector) and eight material planes staged in LDS; block.y
-// takes the rows 1 + block.y, the next gridDim.y on.
+// The six SBP rows at a free surface (sbp_rows.h) from U (predictor) or A
+// (corrector; beta != 0: k_comp_rows_damp left the damping in Dn).
 template <bool CORR>
-__global__ void __launch_bounds__(NT, 1)
+__global__ void __launch_bounds__(RNT, CORR ? 2 : 4)
 k_comp_rows(Box b, int top, int nk, int ntx, const SbpTablesT<float>* __restrict__ sbp, const float* __restrict__ stg,
             const float* __restrict__ mu, const float* __restrict__ la, const float* __restrict__ rho, SgCoefF sg,
             const float* __restrict__ dold, float* __restrict__ dnew, float* __restrict__ uu, float* __restrict__ cc,
             float* __restrict__ aout, float cof, float dt2, float c4, float beta)
 {
-   constexpr int NU = (3 * PL + NT - 1) / NT;
-   constexpr int NM = (PL + NT - 1) / NT;
-   __shared__ float su[9 * 3 * PL];
-   __shared__ float sm[8 * PL], sl[8 * PL];
-   __shared__ float ssx[HX], ssy[HY];
-   const int tix = blockIdx.x % ntx, tjy = blockIdx.x / ntx;
-   const int tid = threadIdx.x, tx = tid % TX, ty = tid / TX;
-   const int ia = b.ib + tix * TX, ja = b.jb + tjy * TY;
-   const int i = ia + 2 + tx, j = ja + 2 + ty;
-   const bool active = i <= b.ie - 2 && j <= b.je - 2;
-   const long ni = b.ni, nij = b.nij, npts = b.npts;
-   const int kbase = top ? 1 : nk;
-   const int sgn = top ? 1 : -1;
-   const int o = (ty + 2) * HX + tx + 2;
-#pragma unroll 1
-   for (int q = 0; q <= 8; q++) {
-      const long pb = nij * (kbase + sgn * (q - 1) - b.kb);
+   const long npts = b.npts;
+   sbp_rows_body<float>(
+       b, top, nk, ntx, sbp, mu, la, sg.strx, sg.stry, [=](int c, long p) { return stg[p + npts * c]; },
+       [=](int, int, int, long p, const float r[3], const float uc[3]) {
+          if (!CORR) {
+             const float sc = cof / rho[p];
 #pragma unroll
-      for (int p = 0; p < NU; p++) {
-         const int e = tid + p * NT;
-         const int c = e / PL, r = e - c * PL, y = r / HX, x = r - y * HX;
-         const int gi = ia + x, gj = ja + y;
-         const bool ok = e < 3 * PL && gi <= b.ie && gj <= b.je;
-         const float v = stg[ok ? pb + (gi - b.ib) + ni * (gj - b.jb) + npts * c : 0];
-         if (e < 3 * PL) su[(q * 3 + c) * PL + r] = ok ? v : 0.0f;
-      }
-      if (q >= 1) {
+             for (int c = 0; c < 3; c++) aout[p + npts * c] = sc * r[c];
+          } else {
+             // its loads stay behind the stencil and their addresses are formed here, not kept over
+             // the rows: 128 registers
+             __builtin_amdgcn_sched_barrier(0);
+             asm volatile("" : "+v"(p));
+             const float sc = c4 / rho[p];
 #pragma unroll
-         for (int p = 0; p < NM; p++) {
-            const int e = tid + p * NT;
-            const int y = e / HX, x = e - y * HX;
-            const int gi = ia + x, gj = ja + y;
-            const bool ok = e < PL && gi <= b.ie && gj <= b.je;
-            const long g = ok ? pb + (gi - b.ib) + ni * (gj - b.jb) : 0;
-            const float vm = mu[g], vl = la[g];
-            if (e < PL) {
-               sm[(q - 1) * PL + e] = ok ? vm : 0.0f;
-               sl[(q - 1) * PL + e] = ok ? vl : 0.0f;
-            }
-         }
-      }
-   }
-   if (tid < HX) ssx[tid] = ia + tid <= b.ie ? sg.strx[ia + tid - b.ib] : 1.0f;
-   if (tid >= 64 && tid < 64 + HY) ssy[tid - 64] = ja + tid - 64 <= b.je ? sg.stry[ja + tid - 64 - b.jb] : 1.0f;
-   __syncthreads();
-   if (!active) return;
-   const SlabStenF st{su + o, sm + o, sl + o, ssx + tx + 2, ssy + ty + 2};
-   const long colp = (i - b.ib) + ni * (j - b.jb);
-   // outside the supergrid layers every term of the damping is an exact zero
-   const int ii = i - b.ib, jj = j - b.jb;
-   const bool dxy = CORR && beta != 0 &&
-                    (sg.dcx[ii - 1] != 0 || sg.dcx[ii] != 0 || sg.dcx[ii + 1] != 0 || sg.dcy[jj - 1] != 0 ||
-                     sg.dcy[jj] != 0 || sg.dcy[jj + 1] != 0);
-#pragma unroll 1
-   for (int kr = 1 + (int)blockIdx.y; kr <= 6; kr += (int)gridDim.y) {
-      const int k = kbase + sgn * (kr - 1);
-      float r[3];
-      sbp_row_body(st, kr, (float)sgn, sbp, r);
-      const long p = colp + nij * (k - b.kb);
-      if (!CORR) {
-         const float sc = cof / rho[p];
-#pragma unroll
-         for (int c = 0; c < 3; c++) aout[p + npts * c] = sc * r[c];
-      } else {
-         float d[3] = {0, 0, 0};
-         const int kk = k - b.kb;
-         if (dxy || (beta != 0 && (sg.dcz[kk - 1] != 0 || sg.dcz[kk] != 0 || sg.dcz[kk + 1] != 0)))
-            damp_point_f(b, i, j, k, dold, rho, sg, beta, d);
-         const float sc = c4 / rho[p];
-#pragma unroll
-         for (int c = 0; c < 3; c++) {
-            const long g = p + npts * c;
-            const float dn = ((dold[g] + dt2 * st.u(c, 0, 0, kr)) + sc * (cof * r[c])) - d[c];
-            float U = uu[g], C = cc[g];
-            comp_add(U, C, dn);
-            dnew[g] = dn;
-            uu[g] = U;
-            cc[g] = C;
-         }
-      }
-   }
+             for (int c = 0; c < 3; c++) {
+                const long g = p + npts * c;
+                const float dmp = beta != 0 ? dnew[g] : 0.0f;
+                const float dn = ((dold[g] + dt2 * uc[c]) + sc * (cof * r[c])) - dmp;
+                float U = uu[g], C = cc[g];
+                comp_add(U, C, dn);
+                dnew[g] = dn;
+                uu[g] = U;
+                cc[g] = C;
+             }
+          }
+       });
 }
 
 // Ghost shell (shell_point): the predictor has A = 0 there (L(u) and F
@@ -964,16 +921,16 @@ int comp_rows(bool corr, const Box& b, int side, int nk, const SbpTablesT<float>
 {
    const long nx = b.ie - b.ib - 3, ny = b.je - b.jb - 3;
    const int ntx = (int)cdiv(nx, TX), nty = (int)cdiv(ny, TY);
-   // two workgroups fit on a CU: where the tiles leave slots idle the six rows
-   // are spread over block.y (at 301 x 301 points, where they do not, two
-   // groups of threads on one slab were slower: 82 -> 97 us)
-   const int tiles = ntx * nty, spread = tiles <= 85 ? 6 : tiles <= 170 ? 3 : tiles <= 256 ? 2 : 1;
-   const dim3 grd(tiles, spread);
+   const int tiles = ntx * nty;
+   const dim3 grd(tiles, sbp_rows_spread(tiles, 2));
+   if (corr && beta != 0)
+      k_comp_rows_damp<<<dim3(cdiv(nx, 64), cdiv(ny, 4)), dim3(64, 4), 0, s>>>(b, side == 4, nk, st.D, st.rho, sg,
+                                                                               st.Dn, beta);
    if (corr)
-      k_comp_rows<true><<<grd, NT, 0, s>>>(b, side == 4, nk, ntx, d_sbpf, st.A, st.mu, st.la, st.rho, sg, st.D,
+      k_comp_rows<true><<<grd, RNT, 0, s>>>(b, side == 4, nk, ntx, d_sbpf, st.A, st.mu, st.la, st.rho, sg, st.D,
                                            st.Dn, st.U, st.C, nullptr, cof, dt2, c4, beta);
    else
-      k_comp_rows<false><<<grd, NT, 0, s>>>(b, side == 4, nk, ntx, d_sbpf, st.U, st.mu, st.la, st.rho, sg,
+      k_comp_rows<false><<<grd, RNT, 0, s>>>(b, side == 4, nk, ntx, d_sbpf, st.U, st.mu, st.la, st.rho, sg,
                                             nullptr, nullptr, nullptr, nullptr, st.A, cof, dt2, c4, beta);
    return check_hip(hipGetLastError(), "FP32 SBP rows launch");
 }

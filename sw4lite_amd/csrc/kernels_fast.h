@@ -67,20 +67,15 @@ bool async_loads_fit(const Box& b, const double* const* arrays, int n);
 // variant 1: plain k-march, 2 waves/SIMD; 2: register prefetch of the next
 // plane, 2 waves/SIMD; 3: prefetch, 1 wave/SIMD; 4: as 3 with the corrector's
 // supergrid damping (beta != 0) applied in the same sweep; 5: corrector as 4,
-// predictor as 1; 6: both as 1, the damping by launch_damp_lds; 7: as 6, the
+// predictor as 1; 6: both as 1, the damping by launch_damp; 7: as 6, the
 // predictor by asynchronous global-to-LDS loads where the rows allow it; 8:
 // as 7, with acc the acceleration stored and staged (below); 9: as 8, the
 // damping sweep restricted to the supergrid layers (damp_tiles).
-// The six SBP rows next to side 4 (top) or 5 (bottom) of one sweep from an
-// LDS slab (corr: with the acceleration and the supergrid damping).
-// The corrector's damping on the six SBP rows of a side (4 top, 5 bottom),
-// for rows k_sbp_rows wrote without it (launch_sbp_rows with beta 0); the
-// same bits as the rows kernel with its damping.
-int launch_rows_damp(const Box& b, int side, int nk, double* up, const double* u, const double* um,
-                     const double* rho, const SgCoef& sg, double beta, hipStream_t s);
+// The six SBP rows next to side 4 (top) or 5 (bottom) of one sweep (corr:
+// from the acceleration, without the damping).
 int launch_sbp_rows(bool corr, const Box& b, int side, int nk, const SbpTables* d_sbp, const double* upin,
                     const double* u, const double* um, const double* mu, const double* la, const double* rho,
-                    const SgCoef& sg, double* out, double h, double dt, double beta, hipStream_t s,
+                    const SgCoef& sg, double* out, double h, double dt, hipStream_t s,
                     const double* acc = nullptr);
 // Column tile (tix, tjy) of the 32 x 8 sweeps and its planes k0..k1.
 struct DampTile {
@@ -97,8 +92,8 @@ std::vector<DampTile> damp_tiles(const Box& b, int k1, int k2, int kc, const dou
                                  const double* dcz);
 // up -= supergrid damping(u, um) on planes k1..k2, k-marching LDS sweep;
 // with tiles (device array of damp_tiles for the same k1, k2, kc) only those
-// tiles run (asynchronous-load sweep; otherwise the whole box).
-int launch_damp_lds(const Box& b, int k1, int k2, int kc, double* up, const double* u, const double* um,
+// tiles run (else the whole box).
+int launch_damp(const Box& b, int k1, int k2, int kc, double* up, const double* u, const double* um,
                     const double* rho, const SgCoef& sg, double beta, hipStream_t s,
                     const DampTile* tiles = nullptr, int ntiles = 0);
 // Variant 8 with acc (3 npts doubles, even row length, aligned arrays): the

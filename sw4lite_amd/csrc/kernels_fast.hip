@@ -14,7 +14,7 @@
 
 #include "kernels_common.h"
 #include "kernels_fast.h"
-#include "sbp_row_body.h"
+#include "sbp_rows.h"
 #include "stencil_body.h"
 
 namespace sw4amd {
@@ -653,133 +653,8 @@ static bool dma_fits(const Box& b, const double* u, const double* mu, const doub
    return b.ni % 2 == 0 && al(u) && al(mu) && al(la);
 }
 
-// Supergrid damping of the corrector on planes kbeg..kend as a k-marching LDS
-// sweep (ew-cfromfort.C:985-1041): up -= damping(u - um).  d = u - um of plane
-// k and rho of plane k are staged with their (i,j) halo in LDS; the thread's
-// own column of d for k-2..k+2 and rho at k+-1 live in registers.  Small LDS
-// and register footprint, so several workgroups share a CU and hide latency.
-// Tiles of 32 x DTY columns (DTY * 32 threads); taller tiles re-read less halo.
-// Column tile (tix, tjy), planes k0..k1.
-template <int DTY>
-__device__ __forceinline__ void damp_lds_tile(int tix, int tjy, int k0, int k1, Box b, double* __restrict__ up,
-                                              const double* __restrict__ u, const double* __restrict__ um,
-                                              const double* __restrict__ rho, SgCoef sg, double beta)
-{
-   constexpr int TY = DTY, HY = TY + 4, NT = TX * TY, PL = HX * HY;
-   constexpr int NU = (3 * PL + NT - 1) / NT;
-   constexpr int NM = (PL + NT - 1) / NT;
-   __shared__ double sdp[3 * PL];
-   __shared__ double srp[PL];
-   const int tid = threadIdx.x, tx = tid % TX, ty = tid / TX;
-   const int ia = b.ib + tix * TX, ja = b.jb + tjy * TY;
-   const int i = ia + 2 + tx, j = ja + 2 + ty;
-   const bool active = i <= b.ie - 2 && j <= b.je - 2;
-   const long ni = b.ni, nij = b.nij, npts = b.npts;
-   const long col = active ? (i - b.ib) + ni * (j - b.jb) : 0;
-   const int o = (ty + 2) * HX + tx + 2;
-   const int ii = i - b.ib, jj = j - b.jb;
-   double dq[5][3];
-   double rkm = 0, rkp = 0;
-#pragma unroll
-   for (int q = 0; q < 4; q++)
-#pragma unroll
-      for (int c = 0; c < 3; c++) {
-         const long g = col + nij * (k0 - 2 + q - b.kb) + npts * c;
-         const double a = u[g], e = um[g];
-         dq[q][c] = active ? a - e : 0.0;
-      }
-   {
-      const double a = rho[col + nij * (k0 - 1 - b.kb)];
-      rkm = active ? a : 0.0;
-   }
-   double gx[5] = {0, 0, 0, 0, 0}, gy[5] = {0, 0, 0, 0, 0};
-   if (active) {
-      gx[0] = sg.dcx[ii - 1]; gx[1] = sg.dcx[ii]; gx[2] = sg.dcx[ii + 1]; gx[3] = sg.strx[ii]; gx[4] = sg.cox[ii];
-      gy[0] = sg.dcy[jj - 1]; gy[1] = sg.dcy[jj]; gy[2] = sg.dcy[jj + 1]; gy[3] = sg.stry[jj]; gy[4] = sg.coy[jj];
-   }
-   for (int k = k0; k <= k1; k++) {
-      const long pb = nij * (k - b.kb);
-      // this point's values of up, updated below: loaded with the plane so
-      // that their latency overlaps the staging loads'
-      double upc[3];
-#pragma unroll
-      for (int c = 0; c < 3; c++) upc[c] = up[col + pb + npts * c];  // col = 0 where inactive: a valid address
-#pragma unroll
-      for (int p = 0; p < NU; p++) {
-         const int e = tid + p * NT;
-         const int c = e / PL, r = e - c * PL, y = r / HX, x = r - y * HX;
-         const int gi = ia + x, gj = ja + y;
-         const bool ok = e < 3 * PL && gi <= b.ie && gj <= b.je;
-         const long g = ok ? pb + (gi - b.ib) + ni * (gj - b.jb) + npts * c : 0;
-         const double a = u[g], m = um[g];
-         if (e < 3 * PL) sdp[e] = ok ? a - m : 0.0;
-      }
-#pragma unroll
-      for (int p = 0; p < NM; p++) {
-         const int e = tid + p * NT;
-         const int y = e / HX, x = e - y * HX;
-         const int gi = ia + x, gj = ja + y;
-         const bool ok = e < PL && gi <= b.ie && gj <= b.je;
-         const double a = rho[ok ? pb + (gi - b.ib) + ni * (gj - b.jb) : 0];
-         if (e < PL) srp[e] = ok ? a : 0.0;
-      }
-#pragma unroll
-      for (int c = 0; c < 3; c++) {
-         const long g = col + nij * (k + 2 - b.kb) + npts * c;
-         const double a = u[g], m = um[g];
-         dq[4][c] = active ? a - m : 0.0;
-      }
-      {
-         const double a = rho[col + nij * (k + 1 - b.kb)];
-         rkp = active ? a : 0.0;
-      }
-      const int kz = k - b.kb;
-      const double gz0 = sg.dcz[kz - 1], gz1 = sg.dcz[kz], gz2 = sg.dcz[kz + 1], gz3 = sg.strz[kz], gz4 = sg.coz[kz];
-      __syncthreads();
-      double r0 = 0;
-      if (active) {
-         r0 = srp[o];
-         const double birho = beta / r0;
-         const double rxp = srp[o + 1] * gx[2], rx0 = r0 * gx[1], rxm = srp[o - 1] * gx[0];
-         const double ryp = srp[o + HX] * gy[2], ry0 = r0 * gy[1], rym = srp[o - HX] * gy[0];
-         const double rzp = rkp * gz2, rz0 = r0 * gz1, rzm = rkm * gz0;
-         const double wx = gx[3] * gy[4] * gz4, wy = gy[3] * gx[4] * gz4, wz = gz3 * gx[4] * gy[4];
-#pragma unroll
-         for (int c = 0; c < 3; c++) {
-            const double* q = sdp + c * PL + o;
-            const double ax = rxp * (q[2] - 2 * q[1] + q[0]) - 2 * rx0 * (q[1] - 2 * q[0] + q[-1]) +
-                              rxm * (q[0] - 2 * q[-1] + q[-2]);
-            const double ay = ryp * (q[2 * HX] - 2 * q[HX] + q[0]) - 2 * ry0 * (q[HX] - 2 * q[0] + q[-HX]) +
-                              rym * (q[0] - 2 * q[-HX] + q[-2 * HX]);
-            const double az = rzp * (dq[4][c] - 2 * dq[3][c] + dq[2][c]) -
-                              2 * rz0 * (dq[3][c] - 2 * dq[2][c] + dq[1][c]) +
-                              rzm * (dq[2][c] - 2 * dq[1][c] + dq[0][c]);
-            up[col + pb + npts * c] = upc[c] - birho * (wx * ax + wy * ay + wz * az);
-         }
-      }
-      __syncthreads();
-#pragma unroll
-      for (int q = 0; q < 4; q++)
-#pragma unroll
-         for (int c = 0; c < 3; c++) dq[q][c] = dq[q + 1][c];
-      rkm = r0;
-   }
-}
-
-template <int DTY>
-__device__ __forceinline__ void damp_lds_body(unsigned bid, Box b, TileMap map, int kbeg, int kend, int kc,
-                                              double* __restrict__ up, const double* __restrict__ u,
-                                              const double* __restrict__ um, const double* __restrict__ rho,
-                                              SgCoef sg, double beta)
-{
-   const int per = (int)((map.ntiles + 7) / 8);
-   const int t = (int)(bid % 8) * per + (int)(bid / 8);
-   if (t >= map.ntiles) return;
-   const int tix = t % map.ntx, tr = t / map.ntx, tjy = tr % map.nty, tkz = tr / map.nty;
-   const int k0 = kbeg + tkz * kc;
-   damp_lds_tile<DTY>(tix, tjy, k0, min(kend, k0 + kc - 1), b, up, u, um, rho, sg, beta);
-}
-
+// Supergrid damping of the corrector as a k-marching LDS sweep
+// (ew-cfromfort.C:985-1041): up -= damping(u - um), d = u - um.
 // The damping sweep with its planes brought to LDS by asynchronous
 // global-to-LDS loads (as sweep_dma_body): raw u, um and rho of plane k+1
 // land while plane k is computed, d = u - um is formed from LDS; the column
@@ -787,14 +662,20 @@ __device__ __forceinline__ void damp_lds_body(unsigned bid, Box b, TileMap map, 
 // one plane ahead into registers, and the results of plane k are stored
 // after the next barrier.  Two slots of 7 staged values per point (48 KB):
 // three workgroups per CU.  Same conditions as sweep_dma_body (even ni,
-// 16-byte aligned arrays).
+// 16-byte aligned arrays); DW: rows of any length by four-byte loads
+// (301 x 301 x 171 points: 358 us against 417 us staged through registers;
+// 512^3 1.22 ms).  A column march with d in registers and LDS that loads
+// every value once was slower (410 us, 1.27 ms): two workgroups per CU
+// instead of three, and loads no further ahead.
 // Column tile (tix, tjy), planes k0..k1.
+template <bool DW>
 __device__ __forceinline__ void damp_dma_tile(int tix, int tjy, int k0, int k1, Box b, double* __restrict__ up,
                                               const double* __restrict__ u, const double* __restrict__ um,
                                               const double* __restrict__ rho, SgCoef sg, double beta)
 {
    constexpr int PP = 3 * PL / 2, NP = (PP + NT - 1) / NT, MP = PL / 2;
-   static_assert(HX % 2 == 0 && MP <= NT, "pairs must tile the rows; one rho load per thread");
+   static_assert(HX % 2 == 0 && MP <= NT && HY % (NT / 64) == 0,
+                 "pairs tile the rows; one rho load per thread; whole rows per wave");
    __shared__ __align__(16) double su[2 * 3 * PL];  // u of plane kp in half (kp - k0) & 1
    __shared__ __align__(16) double sq[2 * 3 * PL];  // um
    __shared__ __align__(16) double sr[2 * PL];      // rho
@@ -807,23 +688,47 @@ __device__ __forceinline__ void damp_dma_tile(int tix, int tjy, int k0, int k1, 
    const long col = active ? (i - b.ib) + ni * (j - b.jb) : 0;
    const int o = (ty + 2) * HX + tx + 2;
    const int ii = i - b.ib, jj = j - b.jb;
-   long goff[NP];
+   long goff[NP], roff = 0;
+   int dwo0 = 0, dwo1 = 0;  // DW: this lane's dword offsets in a staged row (as sweep_dma_body)
+   if constexpr (DW) {
+      const int lane = tid & 63, d0 = lane >> 1, d1 = 32 + (lane >> 1);
+      dwo0 = 2 * (ia + d0 <= b.ie ? d0 : 0) + (lane & 1);
+      dwo1 = 2 * (ia + d1 <= b.ie ? d1 : 0) + (lane & 1);
+   } else {
 #pragma unroll
-   for (int p = 0; p < NP; p++) {
-      const int e = 2 * (tid + p * NT);
-      const int c = e / PL, r = e - c * PL, y = r / HX, x = r - y * HX;
-      const int gi = ia + x, gj = ja + y;
-      const bool ok = e < 3 * PL && gi <= b.ie && gj <= b.je;
-      goff[p] = ok ? (gi - b.ib) + ni * (gj - b.jb) + npts * c : 0;
-   }
-   long roff;
-   {
+      for (int p = 0; p < NP; p++) {
+         const int e = 2 * (tid + p * NT);
+         const int c = e / PL, r = e - c * PL, y = r / HX, x = r - y * HX;
+         const int gi = ia + x, gj = ja + y;
+         const bool ok = e < 3 * PL && gi <= b.ie && gj <= b.je;
+         goff[p] = ok ? (gi - b.ib) + ni * (gj - b.jb) + npts * c : 0;
+      }
       const int e = 2 * tid, y = e / HX, x = e - y * HX;
       const int gi = ia + x, gj = ja + y;
       roff = e < PL && gi <= b.ie && gj <= b.je ? (gi - b.ib) + ni * (gj - b.jb) : 0;
    }
+   auto dma_row = [&](const double* row, double* lds) {
+      const float* g = reinterpret_cast<const float*>(row);
+      __builtin_amdgcn_global_load_lds(g + dwo0, SW4_LDS(lds), 4, 0, 0);
+      if ((tid & 63) < 2 * HX - 64) __builtin_amdgcn_global_load_lds(g + dwo1, SW4_LDS(lds + 32), 4, 0, 0);
+   };
    auto dma_plane = [&](int kp, int half) {
       const long pb = nij * (kp - b.kb);
+      if constexpr (DW) {
+         constexpr int NW = NT / 64;
+#pragma unroll
+         for (int t = 0; t < HY / NW; t++) {  // the wave's rows of the tile; rows off the box load the last one
+            const int r = wv + NW * t;
+            const long ro = pb + ni * (min(ja + r, b.je) - b.jb) + (ia - b.ib);
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+               dma_row(u + ro + npts * c, su + half * 3 * PL + c * PL + r * HX);
+               dma_row(um + ro + npts * c, sq + half * 3 * PL + c * PL + r * HX);
+            }
+            dma_row(rho + ro, sr + half * PL + r * HX);
+         }
+         return;
+      }
       double* du = su + half * 3 * PL + 2 * 64 * wv;
       double* dq = sq + half * 3 * PL + 2 * 64 * wv;
 #pragma unroll
@@ -931,46 +836,33 @@ __device__ __forceinline__ void damp_dma_tile(int tix, int tjy, int k0, int k1, 
    }
 }
 
-__device__ __forceinline__ void damp_dma_body(unsigned bid, Box b, TileMap map, int kbeg, int kend, int kc,
-                                              double* __restrict__ up, const double* __restrict__ u,
-                                              const double* __restrict__ um, const double* __restrict__ rho,
-                                              SgCoef sg, double beta)
+// All tiles of the box, planes kbeg..kend in blocks of kc.
+template <bool DW>
+__global__ void __launch_bounds__(NT, 3)
+k_damp(Box b, TileMap map, int kbeg, int kend, int kc, double* __restrict__ up, const double* __restrict__ u,
+       const double* __restrict__ um, const double* __restrict__ rho, SgCoef sg, double beta)
 {
    const int per = (int)((map.ntiles + 7) / 8);
-   const int t = (int)(bid % 8) * per + (int)(bid / 8);
+   const int t = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
    if (t >= map.ntiles) return;
    const int tix = t % map.ntx, tr = t / map.ntx, tjy = tr % map.nty, tkz = tr / map.nty;
    const int k0 = kbeg + tkz * kc;
-   damp_dma_tile(tix, tjy, k0, min(kend, k0 + kc - 1), b, up, u, um, rho, sg, beta);
+   damp_dma_tile<DW>(tix, tjy, k0, min(kend, k0 + kc - 1), b, up, u, um, rho, sg, beta);
 }
 
+// The damping over a list of tiles (damp_tiles): the XCD of a block is its id
+// mod 8 and each XCD takes one contiguous run of the list.
+template <bool DW>
 __global__ void __launch_bounds__(NT, 3)
-k_damp_dma(Box b, TileMap map, int kbeg, int kend, int kc, double* __restrict__ up, const double* __restrict__ u,
-           const double* __restrict__ um, const double* __restrict__ rho, SgCoef sg, double beta)
-{
-   damp_dma_body(blockIdx.x, b, map, kbeg, kend, kc, up, u, um, rho, sg, beta);
-}
-
-// The damping sweep over a list of tiles (damp_tiles): the XCD of a block is
-// its id mod 8 and each XCD takes one contiguous run of the list.
-__global__ void __launch_bounds__(NT, 3)
-k_damp_dma_tiles(Box b, const DampTile* __restrict__ tiles, int ntiles, double* __restrict__ up,
-                 const double* __restrict__ u, const double* __restrict__ um, const double* __restrict__ rho,
-                 SgCoef sg, double beta)
+k_damp_tiles(Box b, const DampTile* __restrict__ tiles, int ntiles, double* __restrict__ up,
+             const double* __restrict__ u, const double* __restrict__ um, const double* __restrict__ rho, SgCoef sg,
+             double beta)
 {
    const int per = (ntiles + 7) / 8;
    const int t = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
    if (t >= ntiles) return;
    const DampTile d = tiles[t];
-   damp_dma_tile(d.tix, d.tjy, d.k0, d.k1, b, up, u, um, rho, sg, beta);
-}
-
-template <int DTY>
-__global__ void __launch_bounds__(32 * DTY, 4)
-k_damp_lds(Box b, TileMap map, int kbeg, int kend, int kc, double* __restrict__ up, const double* __restrict__ u,
-           const double* __restrict__ um, const double* __restrict__ rho, SgCoef sg, double beta)
-{
-   damp_lds_body<DTY>(blockIdx.x, b, map, kbeg, kend, kc, up, u, um, rho, sg, beta);
+   damp_dma_tile<DW>(d.tix, d.tjy, d.k0, d.k1, b, up, u, um, rho, sg, beta);
 }
 
 // ---------------------------------------------------------------------------
@@ -1018,28 +910,6 @@ __device__ __forceinline__ bool damp_batch_tile(const SweepShot& h, unsigned bid
    return true;
 }
 
-__global__ void __launch_bounds__(32 * 8, 4) k_damp_batch(const SweepShot* __restrict__ shots, int nshots)
-{
-   const SweepShot& h = shots[find_shot(shots, nshots, blockIdx.x)];
-   int tix, tjy, k0, k1;
-   if (!damp_batch_tile(h, blockIdx.x - h.grid0, tix, tjy, k0, k1)) return;
-   damp_lds_tile<8>(tix, tjy, k0, k1, h.b, h.out, h.u, h.um, h.rho, h.sg, h.beta);
-}
-
-// The register-staged damping over a tile list of one grid (entry t of the
-// list, each XCD taking one contiguous run), for rows of odd length.
-__global__ void __launch_bounds__(32 * 8, 4) k_damp_lds_tiles(Box b, const DampTile* __restrict__ tiles, int ntiles,
-                                                              double* __restrict__ up, const double* __restrict__ u,
-                                                              const double* __restrict__ um,
-                                                              const double* __restrict__ rho, SgCoef sg, double beta)
-{
-   const int per = (ntiles + 7) / 8;
-   const int t = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
-   if (t >= ntiles) return;
-   const DampTile d = tiles[t];
-   damp_lds_tile<8>(d.tix, d.tjy, d.k0, d.k1, b, up, u, um, rho, sg, beta);
-}
-
 int fill_sweep_shot(bool damping, const Box& b, int k1, int k2, int kc, const double* upin, const double* u,
                     const double* um, const double* mu, const double* la, const double* rho, const SgCoef& sg,
                     double* out, double h, double dt, double beta, bool corr, int grid0, SweepShot* sh,
@@ -1073,8 +943,8 @@ int fill_sweep_shot(bool damping, const Box& b, int k1, int k2, int kc, const do
    return grid0 + 8 * (int)cdiv(sh->map.ntiles, 8);
 }
 
-// Batched predictor (kind 0) and damping (kind 2) sweeps of grids whose
-// planes take the asynchronous global-to-LDS loads (async_loads_fit).
+// Batched predictor of grids whose planes take the 16-byte asynchronous
+// loads (async_loads_fit).
 // (the predictor stores the acceleration in acc where the shot has one)
 __global__ void __launch_bounds__(NT, 2) k_sweep_dma_batch(const SweepShot* __restrict__ shots, int nshots)
 {
@@ -1092,12 +962,13 @@ __global__ void __launch_bounds__(NT, 2) k_sweep_dma_corr_batch(const SweepShot*
                                          h.mu, h.la, h.rho, h.sg, h.out, nullptr, h.cof, h.cupd, h.dt2i);
 }
 
-__global__ void __launch_bounds__(NT, 3) k_damp_dma_batch(const SweepShot* __restrict__ shots, int nshots)
+template <bool DW>
+__global__ void __launch_bounds__(NT, 3) k_damp_batch(const SweepShot* __restrict__ shots, int nshots)
 {
    const SweepShot& h = shots[find_shot(shots, nshots, blockIdx.x)];
    int tix, tjy, k0, k1;
    if (!damp_batch_tile(h, blockIdx.x - h.grid0, tix, tjy, k0, k1)) return;
-   damp_dma_tile(tix, tjy, k0, k1, h.b, h.out, h.u, h.um, h.rho, h.sg, h.beta);
+   damp_dma_tile<DW>(tix, tjy, k0, k1, h.b, h.out, h.u, h.um, h.rho, h.sg, h.beta);
 }
 
 bool async_loads_fit(const Box& b, const double* const* arrays, int n)
@@ -1116,7 +987,7 @@ int launch_sweep_batch_async(int kind, const SweepShot* d_shots, int nshots, int
    else if (kind == 1)
       k_sweep_dma_corr_batch<<<nblocks, NT, 0, s>>>(d_shots, nshots);
    else
-      k_damp_dma_batch<<<nblocks, NT, 0, s>>>(d_shots, nshots);
+      k_damp_batch<false><<<nblocks, NT, 0, s>>>(d_shots, nshots);
    return check_hip(hipGetLastError(), "batched asynchronous-load sweep launch");
 }
 
@@ -1128,7 +999,7 @@ int launch_sweep_batch(int kind, const SweepShot* d_shots, int nshots, int nbloc
    else if (kind == 1)
       k_sweep_batch<true><<<nblocks, NT, 0, s>>>(d_shots, nshots);
    else
-      k_damp_batch<<<nblocks, 32 * 8, 0, s>>>(d_shots, nshots);
+      k_damp_batch<true><<<nblocks, NT, 0, s>>>(d_shots, nshots);
    return check_hip(hipGetLastError(), "batched sweep launch");
 }
 
@@ -1236,266 +1107,79 @@ std::vector<DampTile> damp_tiles(const Box& b, int k1, int k2, int kc, const dou
    return out;
 }
 
-int launch_damp_lds(const Box& b, int k1, int k2, int kc, double* up, const double* u, const double* um,
+int launch_damp(const Box& b, int k1, int k2, int kc, double* up, const double* u, const double* um,
                     const double* rho, const SgCoef& sg, double beta, hipStream_t s, const DampTile* tiles,
                     int ntiles)
 {
    if (k2 < k1 || beta == 0) return OK;
-   if (tiles && dma_fits(b, u, um, rho) && ((uintptr_t)up & 15) == 0) {
-      if (ntiles > 0)
-         k_damp_dma_tiles<<<8 * cdiv(ntiles, 8), NT, 0, s>>>(b, tiles, ntiles, up, u, um, rho, sg, beta);
-      return check_hip(hipGetLastError(), "damping sweep launch");
-   }
-   if (tiles) {  // odd rows: the register-staged tile over the listed tiles only
-      if (ntiles > 0)
-         k_damp_lds_tiles<<<8 * cdiv(ntiles, 8), 32 * 8, 0, s>>>(b, tiles, ntiles, up, u, um, rho, sg, beta);
+   const bool fit = dma_fits(b, u, um, rho) && ((uintptr_t)up & 15) == 0;
+   if (tiles) {
+      if (ntiles > 0 && fit)
+         k_damp_tiles<false><<<8 * cdiv(ntiles, 8), NT, 0, s>>>(b, tiles, ntiles, up, u, um, rho, sg, beta);
+      else if (ntiles > 0)
+         k_damp_tiles<true><<<8 * cdiv(ntiles, 8), NT, 0, s>>>(b, tiles, ntiles, up, u, um, rho, sg, beta);
       return check_hip(hipGetLastError(), "damping sweep launch");
    }
    const long nx = b.ie - b.ib - 3, ny = b.je - b.jb - 3;
-   constexpr int DTY = 8;
    TileMap map;
    map.ntx = (int)cdiv(nx, TX);
-   map.nty = (int)cdiv(ny, DTY);
+   map.nty = (int)cdiv(ny, TY);
    if (kc <= 0) kc = march_kchunk((long)map.ntx * map.nty, k2 - k1 + 1, 3);
    map.ntiles = map.ntx * map.nty * (int)cdiv(k2 - k1 + 1, kc);
-   static_assert(DTY == TY, "the asynchronous-load damping sweep uses the sweeps' tile");
-   if (dma_fits(b, u, um, rho) && ((uintptr_t)up & 15) == 0)
-      k_damp_dma<<<8 * cdiv(map.ntiles, 8), NT, 0, s>>>(b, map, k1, k2, kc, up, u, um, rho, sg, beta);
+   if (fit)
+      k_damp<false><<<8 * cdiv(map.ntiles, 8), NT, 0, s>>>(b, map, k1, k2, kc, up, u, um, rho, sg, beta);
    else
-      k_damp_lds<DTY><<<8 * cdiv(map.ntiles, 8), 32 * DTY, 0, s>>>(b, map, k1, k2, kc, up, u, um, rho, sg, beta);
+      k_damp<true><<<8 * cdiv(map.ntiles, 8), NT, 0, s>>>(b, map, k1, k2, kc, up, u, um, rho, sg, beta);
    return check_hip(hipGetLastError(), "damping sweep launch");
 }
 
 // ---------------------------------------------------------------------------
 // SBP boundary rows (k = 1..6 below a free surface, or the six rows above
-// one at the bottom) of both sweeps, LDS-staged.  Row space: plane q = 0..8
-// is grid plane KK(q) = kbase + sgn (q - 1) (rhs4sg_rev.C:353-629); row kr
-// lives on q = kr.  One workgroup stages the nine planes of the displacement
-// (or of the acceleration, corrector) and the eight material planes of its
-// 32 x 8 tile once and evaluates all six rows of its columns from LDS.
+// one at the bottom) of both sweeps (sbp_rows.h).
 // ---------------------------------------------------------------------------
-struct SlabSten {
-   const double* ub;  // staged plane q = 0, this thread's point
-   const double* mb;  // mu plane q = 1
-   const double* lb;
-   const double* psx;
-   const double* psy;
-   __device__ __forceinline__ double u(int c, int di, int dj, int q) const
-   {
-      return ub[(q * 3 + c) * PL + dj * HX + di];
-   }
-   __device__ __forceinline__ double mu(int di, int dj, int q) const { return mb[(q - 1) * PL + dj * HX + di]; }
-   __device__ __forceinline__ double la(int di, int dj, int q) const { return lb[(q - 1) * PL + dj * HX + di]; }
-   __device__ __forceinline__ double sx(int d) const { return psx[d]; }
-   __device__ __forceinline__ double sy(int d) const { return psy[d]; }
-};
-
-// CORR = false: up = 2u - um + dt2/rho cof L(u) on the six rows;
-// CORR = true:  upo = up + dt4/(12 rho) cof L(acc) - damping(u, um) with
-// acc = (up - 2u + um) dt2i staged in the slab; DAMP = false: without the
-// damping (a damping sweep over these rows follows; the damping's registers
-// would push this kernel's 256 into 130 accumulator-register copies).
-// G groups of NT threads share the slab and take the rows kr = 1 + group + G
-// block.y, the next G gridDim.y on: one group evaluates its rows one after
-// the other, each a long chain at one wave per SIMD, so more groups (and, on
-// grids whose tiles leave CUs idle, the rows spread over block.y) shorten it.
-template <bool CORR, bool DAMP, int G>
-__global__ void __launch_bounds__(NT * G, 1)
+// CORR = false: out = 2u - um + dt2/rho cof L(u) on the six rows;
+// CORR = true:  out = up + dt4/(12 rho) cof L(acc), acc = (up - 2u + um) dt2i
+// stored (acc) or formed from the three fields; the damping sweep that follows
+// damps the rows as well.
+template <bool CORR>
+__global__ void __launch_bounds__(RNT, 1)
 k_sbp_rows(Box b, int top, int nk, int ntx, const SbpTables* __restrict__ sbp, const double* __restrict__ upin,
            const double* __restrict__ u, const double* __restrict__ um, const double* __restrict__ mu,
            const double* __restrict__ la, const double* __restrict__ rho, SgCoef sg, double* __restrict__ out,
-           double cof, double dt2i, double cupd, double beta, bool dma, const double* __restrict__ acc)
+           double cof, double dt2i, double cupd, const double* __restrict__ acc)
 {
-   constexpr int NU = (3 * PL + NT - 1) / NT;
-   constexpr int NM = (PL + NT - 1) / NT;
-   // destinations of 16-byte asynchronous loads: every staged plane starts
-   // on a 16-byte boundary
-   static_assert((PL * sizeof(double)) % 16 == 0, "staged planes must stay 16-byte aligned");
-   __shared__ __align__(16) double su[9 * 3 * PL];  // planes q = 0..8, components
-   __shared__ __align__(16) double sm[8 * PL];
-   __shared__ __align__(16) double sl[8 * PL];
-   __shared__ double ssx[HX], ssy[HY];
-   const int tix = blockIdx.x % ntx, tjy = blockIdx.x / ntx;
-   // thread of the group, group of the workgroup (whole waves: uniform in a wave)
-   const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
-   const int tid = threadIdx.x - grp * NT, tx = tid % TX, ty = tid / TX;
-   const int ia = b.ib + tix * TX, ja = b.jb + tjy * TY;
-   const int i = ia + 2 + tx, j = ja + 2 + ty;
-   const bool active = i <= b.ie - 2 && j <= b.je - 2;
-   const long ni = b.ni, nij = b.nij, npts = b.npts;
-   const int kbase = top ? 1 : nk;
-   const int sgn = top ? 1 : -1;
-   const int o = (ty + 2) * HX + tx + 2;
-   // stage: displacement (or acceleration) planes q = 0..8, material 1..8.
-   // The predictor's raw planes go by asynchronous global-to-LDS loads when
-   // the rows allow it (dma: even ni, aligned arrays), all issued before one
-   // wait; pairs off the box load the plane's first point (read only by
-   // inactive points, as every staged value off the box).
-   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-   // (the corrector's planes too when the acceleration is stored: acc)
-   const bool async = dma && (!CORR || acc);
-   const double* __restrict__ src = CORR ? acc : u;
-   if (async) {
-      constexpr int PP = 3 * PL / 2, NP = (PP + NT - 1) / NT, MP = PL / 2;
-      long goff[NP], moff = 0;
+   const long npts = b.npts;
+   sbp_rows_body<double>(
+       b, top, nk, ntx, sbp, mu, la, sg.strx, sg.stry,
+       [=](int c, long p) {
+          const long q = p + npts * c;
+          if (!CORR) return u[q];
+          return acc ? acc[q] : dt2i * (upin[q] - 2 * u[q] + um[q]);
+       },
+       [=](int, int, int, long p, const double r[3], const double uc[3]) {
+          const double sc = cupd / rho[p];
 #pragma unroll
-      for (int p = 0; p < NP; p++) {
-         const int e = 2 * (tid + p * NT);
-         const int c = e / PL, r = e - c * PL, y = r / HX, x = r - y * HX;
-         const int gi = ia + x, gj = ja + y;
-         goff[p] = e < 3 * PL && gi <= b.ie && gj <= b.je ? (gi - b.ib) + ni * (gj - b.jb) + npts * c : 0;
-      }
-      {
-         const int e = 2 * tid, y = e / HX, x = e - y * HX;
-         const int gi = ia + x, gj = ja + y;
-         moff = e < PL && gi <= b.ie && gj <= b.je ? (gi - b.ib) + ni * (gj - b.jb) : 0;
-      }
-#pragma unroll 1
-      for (int q = grp; q <= 8; q += G) {
-         const long pb = nij * (kbase + sgn * (q - 1) - b.kb);
-         double* dst = su + q * 3 * PL + 2 * 64 * wv;
-#pragma unroll
-         for (int p = 0; p < NP; p++)
-            if (tid + p * NT < PP)
-               __builtin_amdgcn_global_load_lds(src + pb + goff[p], SW4_LDS(dst + 2 * p * NT), 16, 0, 0);
-         if (q >= 1 && tid < MP) {
-            __builtin_amdgcn_global_load_lds(mu + pb + moff, SW4_LDS(sm + (q - 1) * PL + 2 * 64 * wv), 16, 0, 0);
-            __builtin_amdgcn_global_load_lds(la + pb + moff, SW4_LDS(sl + (q - 1) * PL + 2 * 64 * wv), 16, 0, 0);
-         }
-      }
-   }
-#pragma unroll 1
-   for (int q = grp; q <= 8 && !async; q += G) {
-      const long pb = nij * (kbase + sgn * (q - 1) - b.kb);
-#pragma unroll
-      for (int p = 0; p < NU; p++) {
-         const int e = tid + p * NT;
-         const int c = e / PL, r = e - c * PL, y = r / HX, x = r - y * HX;
-         const int gi = ia + x, gj = ja + y;
-         const bool ok = e < 3 * PL && gi <= b.ie && gj <= b.je;
-         const long g = ok ? pb + (gi - b.ib) + ni * (gj - b.jb) + npts * c : 0;
-         const double vu = u[g];
-         double v = vu;
-         if (CORR) {
-            const double vp = upin[g], vq = um[g];
-            v = dt2i * (vp - 2 * vu + vq);
-         }
-         if (e < 3 * PL) su[(q * 3 + c) * PL + r] = ok ? v : 0.0;
-      }
-      if (q >= 1) {
-#pragma unroll
-         for (int p = 0; p < NM; p++) {
-            const int e = tid + p * NT;
-            const int y = e / HX, x = e - y * HX;
-            const int gi = ia + x, gj = ja + y;
-            const bool ok = e < PL && gi <= b.ie && gj <= b.je;
-            const long g = ok ? pb + (gi - b.ib) + ni * (gj - b.jb) : 0;
-            const double vm = mu[g], vl = la[g];
-            if (e < PL) {
-               sm[(q - 1) * PL + e] = ok ? vm : 0.0;
-               sl[(q - 1) * PL + e] = ok ? vl : 0.0;
-            }
-         }
-      }
-   }
-   if (grp == 0 && tid < HX) ssx[tid] = ia + tid <= b.ie ? sg.strx[ia + tid - b.ib] : 1.0;
-   if (grp == 0 && tid >= 64 && tid < 64 + HY) ssy[tid - 64] = ja + tid - 64 <= b.je ? sg.stry[ja + tid - 64 - b.jb] : 1.0;
-   __syncthreads();
-   if (!active) return;
-   SlabSten st{su + o, sm + o, sl + o, ssx + tx + 2, ssy + ty + 2};
-   const long colp = (i - b.ib) + ni * (j - b.jb);
-   // every term of the damping carries a damping coefficient at the point or
-   // a neighbour along its axis: outside the supergrid layers it subtracts
-   // exactly zero and is not evaluated
-   const int ii = i - b.ib, jj = j - b.jb;
-   const bool dxy = DAMP && beta != 0 &&
-                    (sg.dcx[ii - 1] != 0 || sg.dcx[ii] != 0 || sg.dcx[ii + 1] != 0 || sg.dcy[jj - 1] != 0 ||
-                     sg.dcy[jj] != 0 || sg.dcy[jj + 1] != 0);
-#pragma unroll 1
-   for (int kr = 1 + grp + G * (int)blockIdx.y; kr <= 6; kr += G * (int)gridDim.y) {
-      const int k = kbase + sgn * (kr - 1);
-      double r[3];
-      sbp_row_body(st, kr, (double)sgn, sbp, r);
-      const long p = colp + nij * (k - b.kb);
-      const double sc = cupd / rho[p];
-      double d[3] = {0, 0, 0};
-      const int kk = k - b.kb;
-      if (DAMP && beta != 0 && (dxy || sg.dcz[kk - 1] != 0 || sg.dcz[kk] != 0 || sg.dcz[kk + 1] != 0))
-         addsgd4_point<1>(b, i, j, k, u, um, rho, sg, beta, d);
-#pragma unroll
-      for (int c = 0; c < 3; c++) {
-         const long q = p + npts * c;
-         if (CORR)
-            out[q] = (upin[q] + sc * (cof * r[c])) - d[c];
-         else
-            out[q] = 2 * st.u(c, 0, 0, kr) - um[q] + sc * (cof * r[c]);
-      }
-   }
-}
-
-// The damping of the corrector on the six SBP rows of a side, after
-// k_sbp_rows<true, false> wrote them: up -= damping(u, um) where a damping
-// coefficient reaches the point (every term carries one; elsewhere the
-// term is an exact zero).  The same arithmetic as the damping inside
-// k_sbp_rows<true> (addsgd4_point, then the subtraction), so the same bits.
-__global__ void __launch_bounds__(256)
-k_rows_damp(Box b, int top, int nk, double* __restrict__ up, const double* __restrict__ u,
-            const double* __restrict__ um, const double* __restrict__ rho, SgCoef sg, double beta)
-{
-   const int i = b.ib + 2 + blockIdx.x * blockDim.x + threadIdx.x;
-   const int j = b.jb + 2 + blockIdx.y * blockDim.y + threadIdx.y;
-   if (i > b.ie - 2 || j > b.je - 2) return;
-   const int k = top ? 1 + (int)blockIdx.z : nk - (int)blockIdx.z;
-   const int ii = i - b.ib, jj = j - b.jb, kk = k - b.kb;
-   const bool damped = sg.dcx[ii - 1] != 0 || sg.dcx[ii] != 0 || sg.dcx[ii + 1] != 0 || sg.dcy[jj - 1] != 0 ||
-                       sg.dcy[jj] != 0 || sg.dcy[jj + 1] != 0 || sg.dcz[kk - 1] != 0 || sg.dcz[kk] != 0 ||
-                       sg.dcz[kk + 1] != 0;
-   if (!damped) return;
-   double d[3] = {0, 0, 0};
-   if (beta != 0) addsgd4_point<1>(b, i, j, k, u, um, rho, sg, beta, d);
-   const long p = sidx(b, i, j, k);
-#pragma unroll
-   for (int c = 0; c < 3; c++) {
-      const long q = p + b.npts * c;
-      up[q] = up[q] - d[c];
-   }
-}
-
-int launch_rows_damp(const Box& b, int side, int nk, double* up, const double* u, const double* um,
-                     const double* rho, const SgCoef& sg, double beta, hipStream_t s)
-{
-   if (beta == 0) return OK;
-   const long nx = b.ie - b.ib - 3, ny = b.je - b.jb - 3;
-   k_rows_damp<<<dim3(cdiv(nx, 64), cdiv(ny, 4), 6), dim3(64, 4, 1), 0, s>>>(b, side == 4, nk, up, u, um, rho, sg,
-                                                                             beta);
-   return check_hip(hipGetLastError(), "SBP rows damping launch");
+          for (int c = 0; c < 3; c++) {
+             const long q = p + npts * c;
+             out[q] = CORR ? upin[q] + sc * (cof * r[c]) : 2 * uc[c] - um[q] + sc * (cof * r[c]);
+          }
+       });
 }
 
 int launch_sbp_rows(bool corr, const Box& b, int side, int nk, const SbpTables* d_sbp, const double* upin,
                     const double* u, const double* um, const double* mu, const double* la, const double* rho,
-                    const SgCoef& sg, double* out, double h, double dt, double beta, hipStream_t s, const double* acc)
+                    const SgCoef& sg, double* out, double h, double dt, hipStream_t s, const double* acc)
 {
    const long nx = b.ie - b.ib - 3, ny = b.je - b.jb - 3;
    const int ntx = (int)cdiv(nx, TX), nty = (int)cdiv(ny, TY);
    const double cof = 1.0 / (h * h), dt2i = 1.0 / (dt * dt);
-   // two groups of three rows (a third group would spill 110 registers); one
-   // row each where that still leaves every workgroup a CU of its own (the
-   // slab fills a CU's LDS).  Predictor and corrector rows: 62 + 60 -> 18 +
-   // 17 us at 40 x 36, 157 + 181 -> 129 + 122 us at 301 x 301 points.
-   constexpr int G = 2;
-   const dim3 grd(ntx * nty, 3 * ntx * nty <= compute_units() ? 3 : 1);
-   if (corr && beta == 0)
-      k_sbp_rows<true, false, G><<<grd, G * NT, 0, s>>>(b, side == 4, nk, ntx, d_sbp, upin, u, um, mu, la, rho, sg,
-                                                        out, cof, dt2i, dt * dt * dt * dt / 12, 0.0,
-                                                        acc && dma_fits(b, acc, mu, la), acc);
-   else if (corr)  // the damping's registers leave room for one group only
-      k_sbp_rows<true, true, 1><<<ntx * nty, NT, 0, s>>>(b, side == 4, nk, ntx, d_sbp, upin, u, um, mu, la, rho, sg,
-                                                         out, cof, dt2i, dt * dt * dt * dt / 12, beta,
-                                                         acc && dma_fits(b, acc, mu, la), acc);
+   const dim3 grd(ntx * nty, sbp_rows_spread(ntx * nty, 1));
+   if (corr)
+      k_sbp_rows<true><<<grd, RNT, 0, s>>>(b, side == 4, nk, ntx, d_sbp, upin, u, um, mu, la, rho, sg, out, cof, dt2i,
+                                           dt * dt * dt * dt / 12, acc);
    else
-      k_sbp_rows<false, false, G><<<grd, G * NT, 0, s>>>(b, side == 4, nk, ntx, d_sbp, nullptr, u, um, mu, la, rho, sg,
-                                                         out, cof, dt2i, dt * dt, beta, dma_fits(b, u, mu, la),
-                                                         nullptr);
+      k_sbp_rows<false><<<grd, RNT, 0, s>>>(b, side == 4, nk, ntx, d_sbp, nullptr, u, um, mu, la, rho, sg, out, cof,
+                                            dt2i, dt * dt, nullptr);
    return check_hip(hipGetLastError(), "SBP rows launch");
 }
 
@@ -1529,7 +1213,7 @@ int launch_sweep_lds(bool corr, int variant, const Box& b, int k1, int k2, int k
    case 5:  // corrector as 4; predictor without prefetch at 2 waves/SIMD
       if (corr) SW4_SWEEP(true, true, 1, true); else SW4_SWEEP(false, false, 2, false);
       break;
-   case 6:  // both sweeps without prefetch at 2 waves/SIMD; damping by launch_damp_lds
+   case 6:  // both sweeps without prefetch at 2 waves/SIMD; damping by launch_damp
       if (corr) SW4_SWEEP(true, false, 2, false); else SW4_SWEEP(false, false, 2, false);
       break;
    case 7:  // as 6, the predictor's planes by asynchronous global-to-LDS loads where they fit

@@ -47,11 +47,12 @@ int launch_accel_points(const Box& b, const SourceTable& st, const double* up, c
 int launch_pred_tail(const Box& b, int nk, const int* onesided, const SbpTables* d_sbp, const double* u,
                      const double* um, const double* mu, const double* la, const double* rho, const SgCoef& sg,
                      double* up, double h, double dt, hipStream_t s, int zfill = 0, double* accf = nullptr);
-int launch_corr_tail(const Box& b, int nk, const int* onesided, const SbpTables* d_sbp, const double* up,
+// The corrector's rows run before the damping sweep, which acts on them too;
+// its ghost shell at any time.
+int launch_corr_rows(const Box& b, int nk, const int* onesided, const SbpTables* d_sbp, const double* up,
                      const double* u, const double* um, const double* mu, const double* la, const double* rho,
-                     const SgCoef& sg, double beta, double* upo, double h, double dt, hipStream_t s,
-                     int zfill = 0,
-                     const double* accf = nullptr, bool split_damp = false);
+                     const SgCoef& sg, double* upo, double h, double dt, hipStream_t s, const double* accf = nullptr);
+int launch_corr_shell(const Box& b, const double* up, double* upo, hipStream_t s, int zfill = 0);
 // tdev: when not null the time is read from device memory (graph replay)
 int launch_src_apply(const Box& b, const SourceTable& st, double t, int deriv2, double coef,
                      const double* rho, double* up, hipStream_t s, const double* tdev = nullptr);

@@ -563,7 +563,7 @@ int launch_pred_tail(const Box& b, int nk, const int* onesided, const SbpTables*
 {
    for (int side = 4; side <= 5; side++) {  // LDS slab of the six rows
       if (onesided[side] != 1) continue;
-      const int rc = launch_sbp_rows(false, b, side, nk, d_sbp, nullptr, u, um, mu, la, rho, sg, up, h, dt, 0.0, s);
+      const int rc = launch_sbp_rows(false, b, side, nk, d_sbp, nullptr, u, um, mu, la, rho, sg, up, h, dt, s);
       if (rc) return rc;
    }
    const long ns = shell_count(b);
@@ -571,21 +571,23 @@ int launch_pred_tail(const Box& b, int nk, const int* onesided, const SbpTables*
    return check_hip(hipGetLastError(), "predictor rows and shell launch");
 }
 
-int launch_corr_tail(const Box& b, int nk, const int* onesided, const SbpTables* d_sbp, const double* up,
+int launch_corr_rows(const Box& b, int nk, const int* onesided, const SbpTables* d_sbp, const double* up,
                      const double* u, const double* um, const double* mu, const double* la, const double* rho,
-                     const SgCoef& sg, double beta, double* upo, double h, double dt, hipStream_t s,
-                     int zfill, const double* accf, bool split_damp)
+                     const SgCoef& sg, double* upo, double h, double dt, hipStream_t s, const double* accf)
 {
-   for (int side = 4; side <= 5; side++) {  // LDS slab, acceleration formed while staging (or stored: accf)
+   for (int side = 4; side <= 5; side++) {  // the acceleration formed while staging (or stored: accf)
       if (onesided[side] != 1) continue;
-      int rc = launch_sbp_rows(true, b, side, nk, d_sbp, up, u, um, mu, la, rho, sg, upo, h, dt,
-                               split_damp ? 0.0 : beta, s, accf);
-      if (rc == OK && split_damp) rc = launch_rows_damp(b, side, nk, upo, u, um, rho, sg, beta, s);
+      const int rc = launch_sbp_rows(true, b, side, nk, d_sbp, up, u, um, mu, la, rho, sg, upo, h, dt, s, accf);
       if (rc) return rc;
    }
+   return OK;
+}
+
+int launch_corr_shell(const Box& b, const double* up, double* upo, hipStream_t s, int zfill)
+{
    const long ns = shell_count(b);
    k_shell<<<cdiv(ns, 256), 256, 0, s>>>(b, 1, up, nullptr, nullptr, upo, zfill);
-   return check_hip(hipGetLastError(), "corrector rows and shell launch");
+   return check_hip(hipGetLastError(), "corrector shell launch");
 }
 
 int launch_corr_fused(const Box& b, int nk, const int* onesided, const SbpTables* d_sbp,
@@ -601,36 +603,45 @@ int launch_corr_fused(const Box& b, int nk, const int* onesided, const SbpTables
    const int k2 = onesided[5] == 1 ? nk - 6 : b.ke - 2;
    const int nii = b.ie - b.ib - 3, njj = b.je - b.jb - 3;
    dim3 blk(64, 4, 1);
-   if (k2 >= k1 && variant >= 1) {
-      int rc = launch_sweep_lds(true, variant, b, k1, k2, kchunk, up, u, um, mu, la, rho, sg, upo, h, dt, beta, s,
-                                const_cast<double*>(accf));
-      if (rc) return rc;
+   if (variant >= 1) {
+      int rc = OK;
+      if (k2 >= k1 && (rc = launch_sweep_lds(true, variant, b, k1, k2, kchunk, up, u, um, mu, la, rho, sg, upo, h, dt,
+                                             beta, s, const_cast<double*>(accf))))
+         return rc;
       if (after_interior && (rc = after_interior())) return rc;
+      if ((rc = launch_corr_rows(b, nk, onesided, d_sbp, up, u, um, mu, la, rho, sg, upo, h, dt, s, accf))) return rc;
       if (beta != 0 && variant >= 6) {
-         if ((rc = launch_damp_lds(b, k1, k2, kchunk, upo, u, um, rho, sg, beta, s, variant >= 9 ? dtiles : nullptr,
-                                   ndtiles)))
+         // the SBP rows too: every plane addsgd4 acts on
+         if ((rc = launch_damp(b, b.kb + 2, b.ke - 2, kchunk, upo, u, um, rho, sg, beta, s,
+                                   variant >= 9 ? dtiles : nullptr, ndtiles)))
             return rc;
-      } else if (beta != 0 && variant < 4) {  // variants 4, 5 damp inside the sweep
-         dim3 grd(cdiv(nii, 64), cdiv(njj, 4), k2 - k1 + 1);
-         k_addsgd4_planes<<<grd, blk, 0, s>>>(b, k1, k2, upo, u, um, rho, sg, beta);
+      } else if (beta != 0) {
+         if (variant < 4 && k2 >= k1) {  // variants 4, 5 damp inside the sweep
+            dim3 grd(cdiv(nii, 64), cdiv(njj, 4), k2 - k1 + 1);
+            k_addsgd4_planes<<<grd, blk, 0, s>>>(b, k1, k2, upo, u, um, rho, sg, beta);
+         }
+         for (int side = 4; side <= 5; side++) {
+            const int r1 = side == 4 ? 1 : nk - 5;
+            if (onesided[side] == 1)
+               k_addsgd4_planes<<<dim3(cdiv(nii, 64), cdiv(njj, 4), 6), blk, 0, s>>>(b, r1, r1 + 5, upo, u, um, rho, sg,
+                                                                                     beta);
+         }
       }
-   } else {
-      if (k2 >= k1) {
-         dim3 grd(cdiv(nii, 64), cdiv(njj, 4), k2 - k1 + 1);
-         k_corr_interior<<<grd, blk, 0, s>>>(b, k1, k2, up, u, um, mu, la, rho, sg, upo, cof, dt2i, dt4i12, beta);
-      }
-      int rc;
-      if (after_interior && (rc = after_interior())) return rc;
+      if (after_damping && (rc = after_damping())) return rc;
+      return launch_corr_shell(b, up, upo, s, zfill);
+   }
+   if (k2 >= k1) {
+      dim3 grd(cdiv(nii, 64), cdiv(njj, 4), k2 - k1 + 1);
+      k_corr_interior<<<grd, blk, 0, s>>>(b, k1, k2, up, u, um, mu, la, rho, sg, upo, cof, dt2i, dt4i12, beta);
+   }
+   if (after_interior) {
+      const int rc = after_interior();
+      if (rc) return rc;
    }
    if (after_damping) {
       const int rc = after_damping();
       if (rc) return rc;
    }
-   // kernel variant 9: the rows' damping in a pass of its own after them
-   // (inside the rows kernel its registers cost that kernel's occupancy)
-   if (variant >= 1)
-      return launch_corr_tail(b, nk, onesided, d_sbp, up, u, um, mu, la, rho, sg, beta, upo, h, dt, s, zfill, accf,
-                              variant >= 9);
    for (int side = 4; side <= 5; side++) {
       if (onesided[side] != 1) continue;
       const int ks = side == 4 ? 0 : nk - SLAB_PLANES + 2;  // planes KK(0)..KK(8) of the rows

@@ -52,6 +52,29 @@ def test_rhs4sg(torch, coefs, corder, os45):
 
 
 @pytest.mark.parametrize("corder", [0, 1])
+@pytest.mark.parametrize("shape", [(32, 8, 12), (33, 9, 13), (12, 12, 12), (100, 81, 14), (130, 90, 13),
+                                   (190, 150, 12), (201, 150, 13)])
+def test_rhs4sg_rows_over_tiles(torch, coefs, corder, shape):
+    """The SBP rows at both ends: whole 32 x 8 tiles, one column and row more,
+    the smallest grid, and grids whose six rows are spread over six, three,
+    two and one workgroup per tile."""
+    from sw4lite_amd import ew
+    acof, ghcof, bope, _ = coefs
+    nx, ny, nz = shape
+    box, f = random_inputs(300 + corder, nx, ny, nz)
+    u = to_layout(f["u"], box, corder)
+    os_ = [0, 0, 0, 0, 1, 1]
+    want = np.zeros_like(u)
+    O.rhs4sg(corder, box, nz, os_, acof, bope, ghcof, want, u, f["mu"], f["la"], 0.3, f["strx"], f["stry"], f["strz"])
+    lu = dev(torch, np.zeros_like(u))
+    ew.rhs4sg(corder, box, nz, os_, acof, bope, ghcof, lu, dev(torch, u), dev(torch, f["mu"]), dev(torch, f["la"]),
+              0.3, dev(torch, f["strx"]), dev(torch, f["stry"]), dev(torch, f["strz"]))
+    err = relerr(host(lu), want)
+    print("rhs4sg rows corder", corder, "shape", shape, "relerr", err, flush=True)
+    assert err < TOL
+
+
+@pytest.mark.parametrize("corder", [0, 1])
 def test_pointwise_updates(torch, corder):
     from sw4lite_amd import ew
     box, f = random_inputs(7, 20, 18, 16)
