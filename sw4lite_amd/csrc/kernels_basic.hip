@@ -1,14 +1,14 @@
-// kernels_basic.hip -- one-thread-per-point gfx950 kernels for every stage of
-// the sw4lite time step, behind the reference's kernel-level entry points:
+// kernels_basic.hip -- gfx950 kernels for every stage of the sw4lite time
+// step (rhs4sg's interior rows and addsgd4: kernels_fast.hip), behind the
+// reference's kernel-level entry points:
 //   rhs4sg / rhs4sg_rev       rhs4sg.C:38-849, rhs4sg_rev.C:43-864
 //   predfort/corrfort/dpdmt   ew-cfromfort.C:40-141
 //   addsgd4fort(_indrev)      ew-cfromfort.C:748-849, :952-1056
 //   bcfortsg(_indrev)         ew-cfromfort.C:205-747
 //   Force (point sources)     EW.C:3085-3123, GridPointSource.C:330-586
-// Both Sarray layouts are supported through the CO template parameter.  The
-// fused, LDS-staged kernels of the fast step live in kernels_fused.hip and
-// are checked against these.
+// Both Sarray layouts are supported through the CO template parameter.
 #include "kernels_common.h"
+#include "kernels_fast.h"
 #include "sbp_rows.h"
 
 namespace sw4amd {
@@ -16,22 +16,6 @@ namespace sw4amd {
 // ---------------------------------------------------------------------------
 // Divergence of stress
 // ---------------------------------------------------------------------------
-template <int CO>
-__global__ void __launch_bounds__(256)
-k_rhs4_interior(Box b, int klo, int khi, const double* __restrict__ u,
-                const double* __restrict__ mu, const double* __restrict__ la,
-                const double* __restrict__ strx, const double* __restrict__ stry,
-                const double* __restrict__ strz, double* __restrict__ lu, double cof)
-{
-   const int i = b.ib + 2 + blockIdx.x * blockDim.x + threadIdx.x;
-   const int j = b.jb + 2 + blockIdx.y * blockDim.y + threadIdx.y;
-   const int k = klo + blockIdx.z;
-   if (i > b.ie - 2 || j > b.je - 2 || k > khi) return;
-   double r[3];
-   rhs_interior_point<CO>(b, i, j, k, Plain{u}, mu, la, strx, stry, strz, r);
-   for (int c = 0; c < 3; c++) lu[vidx<CO>(b, c, i, j, k)] = cof * r[c];
-}
-
 // The six SBP rows next to a free surface (sbp_rows.h).
 template <int CO>
 __global__ void __launch_bounds__(RNT, 1)
@@ -87,30 +71,6 @@ __global__ void k_dpdmt(long n, const double* __restrict__ up, const double* __r
 }
 
 // ---------------------------------------------------------------------------
-// Supergrid damping
-// ---------------------------------------------------------------------------
-template <int CO>
-__global__ void __launch_bounds__(256)
-k_addsgd4(Box b, double* __restrict__ up, const double* __restrict__ u,
-          const double* __restrict__ um, const double* __restrict__ rho, SgCoef sg, double beta)
-{
-   const int i = b.ib + 2 + blockIdx.x * blockDim.x + threadIdx.x;
-   const int j = b.jb + 2 + blockIdx.y * blockDim.y + threadIdx.y;
-   const int k = b.kb + 2 + blockIdx.z;
-   if (i > b.ie - 2 || j > b.je - 2 || k > b.ke - 2) return;
-   // every term carries one of these damping coefficients: where all nine
-   // vanish (away from the supergrid layers) the update subtracts zero for
-   // finite data, and the point is left as it is
-   const int ii = i - b.ib, jj = j - b.jb, kk = k - b.kb;
-   if (sg.dcx[ii - 1] == 0 && sg.dcx[ii] == 0 && sg.dcx[ii + 1] == 0 && sg.dcy[jj - 1] == 0 && sg.dcy[jj] == 0 &&
-       sg.dcy[jj + 1] == 0 && sg.dcz[kk - 1] == 0 && sg.dcz[kk] == 0 && sg.dcz[kk + 1] == 0)
-      return;
-   double d[3];
-   addsgd4_point<CO>(b, i, j, k, u, um, rho, sg, beta, d);
-   for (int c = 0; c < 3; c++) up[vidx<CO>(b, c, i, j, k)] -= d[c];
-}
-
-// ---------------------------------------------------------------------------
 // Ghost-point boundary conditions
 // ---------------------------------------------------------------------------
 struct Window {
@@ -127,7 +87,32 @@ __global__ void k_bc_fill(Box b, Window w, double* __restrict__ u, const double*
    const int i = w.i0 + (int)(q % wi);
    const int j = w.j0 + (int)((q / wi) % wj);
    const int k = w.k0 + (int)(q / (wi * wj));
-   for (int c = 0; c < 3; c++) u[vidx<CO>(b, c, i, j, k)] = bf ? bf[3 * q + c] : 0.0;
+   for (int c = 0; c < 3; c++) u[vidx<CO>(b, c, i, j, k)] = bf[3 * q + c];
+}
+
+// Zero ghost values of several sides in one launch: thread q of the windows
+// laid end to end (off[s] is where window s begins).  Points in two windows
+// get the same zero from both.
+struct WindowList {
+   Window w[6];
+   long off[7];
+   int n;
+};
+
+template <int CO>
+__global__ void k_bc_zero(Box b, WindowList l, double* __restrict__ u)
+{
+   long q = blockIdx.x * (long)blockDim.x + threadIdx.x;
+   if (q >= l.off[l.n]) return;
+   int s = 0;
+   while (s + 1 < l.n && q >= l.off[s + 1]) s++;
+   const Window w = l.w[s];
+   q -= l.off[s];
+   const long wi = w.i1 - w.i0 + 1, wj = w.j1 - w.j0 + 1;
+   const int i = w.i0 + (int)(q % wi);
+   const int j = w.j0 + (int)((q / wi) % wj);
+   const int k = w.k0 + (int)(q / (wi * wj));
+   for (int c = 0; c < 3; c++) u[vidx<CO>(b, c, i, j, k)] = 0.0;
 }
 
 template <int CO>
@@ -209,14 +194,11 @@ int launch_rhs4sg(int co, const Box& b, int nk, const int* onesided, const SbpTa
    const int k2 = onesided[5] == 1 ? nk - 6 : b.ke - 2;
    const int nii = b.ie - b.ib - 3, njj = b.je - b.jb - 3;
    if (nii <= 0 || njj <= 0) return OK;
-   dim3 blk(64, 4, 1);
-   if (k2 >= k1) {
-      dim3 grd(cdiv(nii, 64), cdiv(njj, 4), k2 - k1 + 1);
-      if (co)
-         k_rhs4_interior<1><<<grd, blk, 0, s>>>(b, k1, k2, u, mu, la, strx, stry, strz, lu, cof);
-      else
-         k_rhs4_interior<0><<<grd, blk, 0, s>>>(b, k1, k2, u, mu, la, strx, stry, strz, lu, cof);
-   }
+   SgCoef sg{};
+   sg.strx = strx;
+   sg.stry = stry;
+   sg.strz = strz;
+   if (const int rc = launch_rhs4_march(co, b, k1, k2, u, mu, la, sg, lu, h, s)) return rc;
    for (int side = 4; side <= 5; side++) {
       if (onesided[side] != 1) continue;
       const int ntx = (int)cdiv(nii, RTX), tiles = ntx * (int)cdiv(njj, RTY);
@@ -258,29 +240,35 @@ int launch_dpdmt(const Box& b, const double* up, const double* u, const double* 
    return check_hip(hipGetLastError(), "dpdmtfort launch");
 }
 
-int launch_addsgd4(int co, const Box& b, double* up, const double* u, const double* um,
-                   const double* rho, const SgCoef& sg, double beta, hipStream_t s)
-{
-   if (beta == 0) return OK;
-   const int nii = b.ie - b.ib - 3, njj = b.je - b.jb - 3, nkk = b.ke - b.kb - 3;
-   if (nii <= 0 || njj <= 0 || nkk <= 0) return OK;
-   dim3 blk(64, 4, 1), grd(cdiv(nii, 64), cdiv(njj, 4), nkk);
-   if (co)
-      k_addsgd4<1><<<grd, blk, 0, s>>>(b, up, u, um, rho, sg, beta);
-   else
-      k_addsgd4<0><<<grd, blk, 0, s>>>(b, up, u, um, rho, sg, beta);
-   return check_hip(hipGetLastError(), "addsgd4 launch");
-}
-
 int launch_bcfortsg(int co, const Box& b, const int* wind, int nx, int ny, int nz, double* u,
                     double h, const int* bccnd, const SbpTables* d_sbp, const double* mu,
                     const double* la, const double* const* bforce, const double* strx,
                     const double* stry, hipStream_t s)
 {
+   // sides with zero data that follow each other go in one launch, queued
+   // before the next side of another kind (sides act in order)
+   WindowList zero{};
+   auto flush = [&]() {
+      if (zero.n == 0) return;
+      const unsigned g = cdiv(zero.off[zero.n], 256);
+      if (co)
+         k_bc_zero<1><<<g, 256, 0, s>>>(b, zero, u);
+      else
+         k_bc_zero<0><<<g, 256, 0, s>>>(b, zero, u);
+      zero.n = 0;
+   };
    for (int side = 0; side < 6; side++) {
       const int* w = wind + 6 * side;
       Window win{w[0], w[1], w[2], w[3], w[4], w[5]};
       const long n = (long)(w[1] - w[0] + 1) * (w[3] - w[2] + 1) * (w[5] - w[4] + 1);
+      if ((bccnd[side] == 1 || bccnd[side] == 2) && !bforce[side]) {
+         if (n <= 0) continue;
+         zero.w[zero.n] = win;
+         zero.off[zero.n + 1] = zero.off[zero.n] + n;
+         zero.n++;
+         continue;
+      }
+      if (bccnd[side] >= 0 && bccnd[side] <= 3) flush();
       if (bccnd[side] == 1 || bccnd[side] == 2) {
          if (n <= 0) continue;
          if (co)
@@ -308,6 +296,7 @@ int launch_bcfortsg(int co, const Box& b, const int* wind, int nx, int ny, int n
             k_bc_freesurf<0><<<grd, blk, 0, s>>>(b, k, kl, h, d_sbp, u, mu, la, bforce[side], strx, stry);
       }
    }
+   flush();
    return check_hip(hipGetLastError(), "bcfortsg launch");
 }
 

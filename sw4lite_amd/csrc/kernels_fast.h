@@ -71,6 +71,10 @@ bool async_loads_fit(const Box& b, const double* const* arrays, int n);
 // predictor by asynchronous global-to-LDS loads where the rows allow it; 8:
 // as 7, with acc the acceleration stored and staged (below); 9: as 8, the
 // damping sweep restricted to the supergrid layers (damp_tiles).
+// out = L(u) on planes k1..k2 (rhs4sg's interior rows) of either array
+// layout, the columns of the box two points inside its i and j ends.
+int launch_rhs4_march(int co, const Box& b, int k1, int k2, const double* u, const double* mu, const double* la,
+                      const SgCoef& sg, double* out, double h, hipStream_t s);
 // The six SBP rows next to side 4 (top) or 5 (bottom) of one sweep (corr:
 // from the acceleration, without the damping).
 int launch_sbp_rows(bool corr, const Box& b, int side, int nk, const SbpTables* d_sbp, const double* upin,

@@ -54,7 +54,9 @@ int march_kchunk(long tiles, int npl, int per_cu)
    return (npl + best - 1) / best;
 }
 
-struct LdsSten {
+// CO: staged planes component-blocked (1) or interleaved (0).
+template <int CO>
+struct LdsStenT {
    const double* p0;  // ring slot of plane k-2, offset to this thread's point
    const double* p1;
    const double* p2;
@@ -69,7 +71,7 @@ struct LdsSten {
    __device__ __forceinline__ double u(int c, int di, int dj, int dk) const
    {
       const double* p = dk == -2 ? p0 : dk == -1 ? p1 : dk == 0 ? p2 : dk == 1 ? p3 : p4;
-      return p[c * PL + dj * HX + di];
+      return CO ? p[c * PL + dj * HX + di] : p[3 * (dj * HX + di) + c];
    }
    __device__ __forceinline__ double mu(int di, int dj, int dk) const { return dk ? muc[dk + 2] : pm[dj * HX + di]; }
    __device__ __forceinline__ double la(int di, int dj, int dk) const { return dk ? lac[dk + 2] : pl[dj * HX + di]; }
@@ -77,6 +79,7 @@ struct LdsSten {
    __device__ __forceinline__ double sy(int d) const { return psy[d]; }
    __device__ __forceinline__ double sz(int d) const { return szv[d + 2]; }
 };
+using LdsSten = LdsStenT<1>;
 
 // CORR = false: out = 2u - um + dt2/rho cof L(u)                  (predictor)
 // CORR = true:  out = up + dt4/(12 rho) cof L((up - 2u + um) dt2i)  (corrector)
@@ -401,8 +404,9 @@ k_sweep_lds(Box b, TileMap map, int kbeg, int kend, int kc, const double* __rest
 // um = Um; with acc, also the acceleration (Up - 2U + Um)/dt^2 at the points
 // it computes, the expression the corrector stages), the transposed operator
 // (TR above: u = W, no um, no rho), and the corrector from the stored
-// acceleration (u = A, um = Up for the centre values, cupd = dt^4/12).
-enum DmaMode { DMA_PRED = 0, DMA_TR = 1, DMA_CORR = 2 };
+// acceleration (u = A, um = Up for the centre values, cupd = dt^4/12), and
+// the operator alone (out = cof L(u); no um, no rho).
+enum DmaMode { DMA_PRED = 0, DMA_TR = 1, DMA_CORR = 2, DMA_LU = 3 };
 
 // The acceleration the corrector applies its stencil to (dpdmtfort,
 // ew-cfromfort.C:116-141), one expression wherever it is formed so that a
@@ -431,14 +435,14 @@ __device__ __forceinline__ double accel_of(double up, double u, double um, doubl
 // specialization that a non-template kernel instantiated when a kernel
 // template uses it as well).
 #define SW4_LDS(p) ((__attribute__((address_space(3))) void*)(p))
-template <int MODE, bool DW = false, bool BATCH = false>
+template <int MODE, bool DW = false, bool BATCH = false, int CO = 1>
 __device__ __forceinline__ void sweep_dma_body(unsigned bid, Box b, TileMap map, int kbeg, int kend, int kc,
                                                const double* __restrict__ u, const double* __restrict__ um,
                                                const double* __restrict__ mu, const double* __restrict__ la,
                                                const double* __restrict__ rho, SgCoef sg, double* __restrict__ out,
                                                double* __restrict__ acc, double cof, double cupd, double dt2i)
 {
-   constexpr bool TR = MODE == DMA_TR;
+   constexpr bool TR = MODE == DMA_TR || MODE == DMA_LU;  // nothing but the staged planes is read
    constexpr int PP = 3 * PL / 2;          // pairs of a staged displacement plane
    constexpr int NP = (PP + NT - 1) / NT;  // asynchronous loads per thread and plane
    constexpr int MP = PL / 2;              // pairs of a material plane
@@ -469,18 +473,33 @@ __device__ __forceinline__ void sweep_dma_body(unsigned bid, Box b, TileMap map,
    long moff = 0;
    // DW: this lane's dword offsets in a staged row (first and second load)
    int dwo0 = 0, dwo1 = 0;
+   constexpr int NI = CO ? 1 : (6 * HX + 63) / 64;  // loads of an interleaved row (3 HX doubles)
+   int dwi[NI] = {};
    if constexpr (DW) {
       const int lane = tid & 63, d0 = lane >> 1, d1 = 32 + (lane >> 1);
       dwo0 = 2 * (ia + d0 <= b.ie ? d0 : 0) + (lane & 1);
       dwo1 = 2 * (ia + d1 <= b.ie ? d1 : 0) + (lane & 1);
+      if (!CO) {
+#pragma unroll
+         for (int p = 0; p < NI; p++) {
+            const int d = 32 * p + (lane >> 1);
+            dwi[p] = 2 * (d < 3 * (b.ie - ia + 1) ? d : 0) + (lane & 1);
+         }
+      }
    } else {
 #pragma unroll
       for (int p = 0; p < NP; p++) {
          const int e = 2 * (tid + p * NT);
-         const int c = e / PL, r = e - c * PL, jj = r / HX, ii = r - jj * HX;
-         const int gi = ia + ii, gj = ja + jj;
-         const bool ok = e < 3 * PL && gi <= b.ie && gj <= b.je;
-         goff[p] = ok ? (gi - b.ib) + ni * (gj - b.jb) + npts * c : 0;
+         if (CO) {
+            const int c = e / PL, r = e - c * PL, jj = r / HX, ii = r - jj * HX;
+            const int gi = ia + ii, gj = ja + jj;
+            const bool ok = e < 3 * PL && gi <= b.ie && gj <= b.je;
+            goff[p] = ok ? (gi - b.ib) + ni * (gj - b.jb) + npts * c : 0;
+         } else {  // rows of 3 HX doubles; an even row length leaves an even number of them on the box
+            const int jj = e / (3 * HX), x = e - jj * 3 * HX, gj = ja + jj;
+            const bool ok = e < 3 * PL && x < 3 * (b.ie - ia + 1) && gj <= b.je;
+            goff[p] = ok ? 3 * ((ia - b.ib) + ni * (gj - b.jb)) + x : 0;
+         }
       }
       const int e = 2 * tid, jj = e / HX, ii = e - jj * HX;
       const int gi = ia + ii, gj = ja + jj;
@@ -493,8 +512,21 @@ __device__ __forceinline__ void sweep_dma_body(unsigned bid, Box b, TileMap map,
       if ((tid & 63) < 2 * HX - 64) __builtin_amdgcn_global_load_lds(g + dwo1, SW4_LDS(lds + 32), 4, 0, 0);
    };
    auto dma_plane = [&](int kp, int slot) {
-      const double* src = u + nij * (kp - b.kb);
-      if constexpr (DW) {
+      const double* src = u + (CO ? 1 : 3) * nij * (kp - b.kb);
+      if constexpr (DW && !CO) {
+         double* dst = su + slot * 3 * PL;
+#pragma unroll
+         for (int t = 0; t < (HY + NW - 1) / NW; t++) {
+            const int r = wv + NW * t;
+            if (r < HY) {
+               const float* g = reinterpret_cast<const float*>(src + 3 * (ni * (min(ja + r, b.je) - b.jb) + (ia - b.ib)));
+#pragma unroll
+               for (int p = 0; p < NI; p++)
+                  if (64 * p + (tid & 63) < 6 * HX)
+                     __builtin_amdgcn_global_load_lds(g + dwi[p], SW4_LDS(dst + 3 * r * HX + 32 * p), 4, 0, 0);
+            }
+         }
+      } else if constexpr (DW) {
          // rows r = (c, jj) of the plane, r = wv, wv + NW, ...; rows off the box load the last one
          double* dst = su + slot * 3 * PL;
 #pragma unroll
@@ -531,7 +563,8 @@ __device__ __forceinline__ void sweep_dma_body(unsigned bid, Box b, TileMap map,
       }
    };
 
-   LdsSten s;
+   LdsStenT<CO> s;
+   constexpr int US = CO ? 1 : 3;  // stride of a staged point
    if (tid >= 128 && tid < 128 + HX) ssx[tid - 128] = ia + tid - 128 <= b.ie ? sg.strx[ia + tid - 128 - b.ib] : 1.0;
    if (tid >= 192 && tid < 192 + HY) ssy[tid - 192] = ja + tid - 192 <= b.je ? sg.stry[ja + tid - 192 - b.jb] : 1.0;
 #pragma unroll
@@ -565,7 +598,7 @@ __device__ __forceinline__ void sweep_dma_body(unsigned bid, Box b, TileMap map,
       if (op >= 0) {
 #pragma unroll
          for (int c = 0; c < 3; c++) {
-            out[op + npts * c] = ov[c];
+            out[CO ? op + npts * c : 3 * op + c] = ov[c];
             if (wacc) acc[op + npts * c] = av[c];
          }
       }
@@ -587,19 +620,21 @@ __device__ __forceinline__ void sweep_dma_body(unsigned bid, Box b, TileMap map,
          csz = sg.strz[k + 3 - b.kb];
       }
       if (active) {
-         s.p0 = su + (sl0 * 3) * PL + o;
-         s.p1 = su + (((sl0 + 1) % 6) * 3) * PL + o;
-         s.p2 = su + (((sl0 + 2) % 6) * 3) * PL + o;
-         s.p3 = su + (((sl0 + 3) % 6) * 3) * PL + o;
-         s.p4 = su + (((sl0 + 4) % 6) * 3) * PL + o;
+         s.p0 = su + (sl0 * 3) * PL + US * o;
+         s.p1 = su + (((sl0 + 1) % 6) * 3) * PL + US * o;
+         s.p2 = su + (((sl0 + 2) % 6) * 3) * PL + US * o;
+         s.p3 = su + (((sl0 + 3) % 6) * 3) * PL + US * o;
+         s.p4 = su + (((sl0 + 4) % 6) * 3) * PL + US * o;
          s.pm = sm + ((k - k0) & 1) * PL + o;
          s.pl = sl + ((k - k0) & 1) * PL + o;
          double r[3];
          rhs4_interior_body(s, r);
-         const double sc = TR ? 1.0 / (s.psx[0] * s.psy[0] * s.szv[2]) : cupd / crho;
+         const double sc = MODE == DMA_TR ? 1.0 / (s.psx[0] * s.psy[0] * s.szv[2]) : MODE == DMA_LU ? 1.0 : cupd / crho;
 #pragma unroll
          for (int c = 0; c < 3; c++) {
-            if (MODE == DMA_TR)
+            if (MODE == DMA_LU)
+               ov[c] = cof * r[c];
+            else if (MODE == DMA_TR)
                ov[c] = sc * (cof * r[c]);
             else if (MODE == DMA_CORR)
                ov[c] = ctr[c] + sc * (cof * r[c]);
@@ -619,7 +654,7 @@ __device__ __forceinline__ void sweep_dma_body(unsigned bid, Box b, TileMap map,
    if (op >= 0) {
 #pragma unroll
       for (int c = 0; c < 3; c++) {
-         out[op + npts * c] = ov[c];
+         out[CO ? op + npts * c : 3 * op + c] = ov[c];
          if (wacc) acc[op + npts * c] = av[c];
       }
    }
@@ -646,6 +681,19 @@ k_sweep_dma_dw(Box b, TileMap map, int kbeg, int kend, int kc, const double* __r
    sweep_dma_body<MODE, true>(blockIdx.x, b, map, kbeg, kend, kc, u, um, mu, la, rho, sg, out, acc, cof, cupd, dt2i);
 }
 
+// The operator alone (rhs4sg's interior rows), either layout, against a
+// thread per point reading its 135 neighbours through the caches: 201 x 201 x
+// 101 points 616 -> 170 us, 301 x 301 x 171 interleaved 2166 -> 539 us.
+template <bool DW, int CO>
+__global__ void __launch_bounds__(NT, 2)
+k_rhs4_dma(Box b, TileMap map, int kbeg, int kend, int kc, const double* __restrict__ u,
+           const double* __restrict__ mu, const double* __restrict__ la, SgCoef sg, double* __restrict__ out,
+           double cof)
+{
+   sweep_dma_body<DMA_LU, DW, false, CO>(blockIdx.x, b, map, kbeg, kend, kc, u, nullptr, mu, la, nullptr, sg, out,
+                                         nullptr, cof, 1.0, 1.0);
+}
+
 // The asynchronous loads need whole 16-byte pairs: even row length, aligned arrays.
 static bool dma_fits(const Box& b, const double* u, const double* mu, const double* la)
 {
@@ -667,8 +715,10 @@ static bool dma_fits(const Box& b, const double* u, const double* mu, const doub
 // 512^3 1.22 ms).  A column march with d in registers and LDS that loads
 // every value once was slower (410 us, 1.27 ms): two workgroups per CU
 // instead of three, and loads no further ahead.
-// Column tile (tix, tjy), planes k0..k1.
-template <bool DW>
+// Column tile (tix, tjy), planes k0..k1.  POINT: points that no damping
+// coefficient reaches are left as they are (elsewhere in the tile the update
+// subtracts an exact zero for finite data).
+template <bool DW, int CO = 1, bool POINT = false>
 __device__ __forceinline__ void damp_dma_tile(int tix, int tjy, int k0, int k1, Box b, double* __restrict__ up,
                                               const double* __restrict__ u, const double* __restrict__ um,
                                               const double* __restrict__ rho, SgCoef sg, double beta)
@@ -690,18 +740,35 @@ __device__ __forceinline__ void damp_dma_tile(int tix, int tjy, int k0, int k1, 
    const int ii = i - b.ib, jj = j - b.jb;
    long goff[NP], roff = 0;
    int dwo0 = 0, dwo1 = 0;  // DW: this lane's dword offsets in a staged row (as sweep_dma_body)
+   constexpr int NI = CO ? 1 : (6 * HX + 63) / 64;  // loads of an interleaved row (3 HX doubles)
+   int dwi[NI] = {};
+   constexpr int US = CO ? 1 : 3;  // stride of a staged point
+   auto at = [=](int c, long p) { return CO ? p + npts * c : 3 * p + c; };
    if constexpr (DW) {
       const int lane = tid & 63, d0 = lane >> 1, d1 = 32 + (lane >> 1);
       dwo0 = 2 * (ia + d0 <= b.ie ? d0 : 0) + (lane & 1);
       dwo1 = 2 * (ia + d1 <= b.ie ? d1 : 0) + (lane & 1);
+      if (!CO) {
+#pragma unroll
+         for (int p = 0; p < NI; p++) {
+            const int d = 32 * p + (lane >> 1);
+            dwi[p] = 2 * (d < 3 * (b.ie - ia + 1) ? d : 0) + (lane & 1);
+         }
+      }
    } else {
 #pragma unroll
       for (int p = 0; p < NP; p++) {
          const int e = 2 * (tid + p * NT);
-         const int c = e / PL, r = e - c * PL, y = r / HX, x = r - y * HX;
-         const int gi = ia + x, gj = ja + y;
-         const bool ok = e < 3 * PL && gi <= b.ie && gj <= b.je;
-         goff[p] = ok ? (gi - b.ib) + ni * (gj - b.jb) + npts * c : 0;
+         if (CO) {
+            const int c = e / PL, r = e - c * PL, y = r / HX, x = r - y * HX;
+            const int gi = ia + x, gj = ja + y;
+            const bool ok = e < 3 * PL && gi <= b.ie && gj <= b.je;
+            goff[p] = ok ? (gi - b.ib) + ni * (gj - b.jb) + npts * c : 0;
+         } else {
+            const int y = e / (3 * HX), x = e - y * 3 * HX, gj = ja + y;
+            const bool ok = e < 3 * PL && x < 3 * (b.ie - ia + 1) && gj <= b.je;
+            goff[p] = ok ? 3 * ((ia - b.ib) + ni * (gj - b.jb)) + x : 0;
+         }
       }
       const int e = 2 * tid, y = e / HX, x = e - y * HX;
       const int gi = ia + x, gj = ja + y;
@@ -720,10 +787,21 @@ __device__ __forceinline__ void damp_dma_tile(int tix, int tjy, int k0, int k1, 
          for (int t = 0; t < HY / NW; t++) {  // the wave's rows of the tile; rows off the box load the last one
             const int r = wv + NW * t;
             const long ro = pb + ni * (min(ja + r, b.je) - b.jb) + (ia - b.ib);
+            if (CO) {
 #pragma unroll
-            for (int c = 0; c < 3; c++) {
-               dma_row(u + ro + npts * c, su + half * 3 * PL + c * PL + r * HX);
-               dma_row(um + ro + npts * c, sq + half * 3 * PL + c * PL + r * HX);
+               for (int c = 0; c < 3; c++) {
+                  dma_row(u + ro + npts * c, su + half * 3 * PL + c * PL + r * HX);
+                  dma_row(um + ro + npts * c, sq + half * 3 * PL + c * PL + r * HX);
+               }
+            } else {
+               const float* gu = reinterpret_cast<const float*>(u + 3 * ro);
+               const float* gm = reinterpret_cast<const float*>(um + 3 * ro);
+#pragma unroll
+               for (int p = 0; p < NI; p++)
+                  if (64 * p + (tid & 63) < 6 * HX) {
+                     __builtin_amdgcn_global_load_lds(gu + dwi[p], SW4_LDS(su + half * 3 * PL + 3 * r * HX + 32 * p), 4, 0, 0);
+                     __builtin_amdgcn_global_load_lds(gm + dwi[p], SW4_LDS(sq + half * 3 * PL + 3 * r * HX + 32 * p), 4, 0, 0);
+                  }
             }
             dma_row(rho + ro, sr + half * PL + r * HX);
          }
@@ -734,8 +812,8 @@ __device__ __forceinline__ void damp_dma_tile(int tix, int tjy, int k0, int k1, 
 #pragma unroll
       for (int p = 0; p < NP; p++)
          if (tid + p * NT < PP) {
-            __builtin_amdgcn_global_load_lds(u + pb + goff[p], SW4_LDS(du + 2 * p * NT), 16, 0, 0);
-            __builtin_amdgcn_global_load_lds(um + pb + goff[p], SW4_LDS(dq + 2 * p * NT), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds(u + US * pb + goff[p], SW4_LDS(du + 2 * p * NT), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds(um + US * pb + goff[p], SW4_LDS(dq + 2 * p * NT), 16, 0, 0);
          }
       if (tid < MP) __builtin_amdgcn_global_load_lds(rho + pb + roff, SW4_LDS(sr + half * PL + 2 * 64 * wv), 16, 0, 0);
    };
@@ -745,7 +823,7 @@ __device__ __forceinline__ void damp_dma_tile(int tix, int tjy, int k0, int k1, 
    for (int q = 0; q < 4; q++)
 #pragma unroll
       for (int c = 0; c < 3; c++) {
-         const long g = col + nij * (k0 - 2 + q - b.kb) + npts * c;
+         const long g = at(c, col + nij * (k0 - 2 + q - b.kb));
          const double a = u[g], e = um[g];
          dq[q][c] = active ? a - e : 0.0;
       }
@@ -760,9 +838,9 @@ __device__ __forceinline__ void damp_dma_tile(int tix, int tjy, int k0, int k1, 
    double nu[3], nm[3], nup[3], nrk;
 #pragma unroll
    for (int c = 0; c < 3; c++) {
-      nu[c] = u[col + nij * (k0 + 2 - b.kb) + npts * c];  // col = 0 where inactive: a valid address
-      nm[c] = um[col + nij * (k0 + 2 - b.kb) + npts * c];
-      nup[c] = up[col + nij * (k0 - b.kb) + npts * c];
+      nu[c] = u[at(c, col + nij * (k0 + 2 - b.kb))];  // col = 0 where inactive: a valid address
+      nm[c] = um[at(c, col + nij * (k0 + 2 - b.kb))];
+      nup[c] = up[at(c, col + nij * (k0 - b.kb))];
    }
    nrk = rho[col + nij * (k0 + 1 - b.kb)];
    double ov[3] = {0, 0, 0};
@@ -772,7 +850,7 @@ __device__ __forceinline__ void damp_dma_tile(int tix, int tjy, int k0, int k1, 
       __syncthreads();  // plane k has landed; plane k-1 is done
       if (op >= 0) {
 #pragma unroll
-         for (int c = 0; c < 3; c++) up[op + npts * c] = ov[c];
+         for (int c = 0; c < 3; c++) up[at(c, op)] = ov[c];
       }
       double upc[3];
 #pragma unroll
@@ -785,9 +863,9 @@ __device__ __forceinline__ void damp_dma_tile(int tix, int tjy, int k0, int k1, 
          dma_plane(k + 1, h ^ 1);
 #pragma unroll
          for (int c = 0; c < 3; c++) {
-            nu[c] = u[col + nij * (k + 3 - b.kb) + npts * c];
-            nm[c] = um[col + nij * (k + 3 - b.kb) + npts * c];
-            nup[c] = up[col + nij * (k + 1 - b.kb) + npts * c];
+            nu[c] = u[at(c, col + nij * (k + 3 - b.kb))];
+            nm[c] = um[at(c, col + nij * (k + 3 - b.kb))];
+            nup[c] = up[at(c, col + nij * (k + 1 - b.kb))];
          }
          nrk = rho[col + nij * (k + 2 - b.kb)];
       }
@@ -804,15 +882,15 @@ __device__ __forceinline__ void damp_dma_tile(int tix, int tjy, int k0, int k1, 
          const double wx = gx[3] * gy[4] * gz4, wy = gy[3] * gx[4] * gz4, wz = gz3 * gx[4] * gy[4];
 #pragma unroll
          for (int c = 0; c < 3; c++) {
-            const double* pu = su + (h * 3 + c) * PL + o;
-            const double* pm = sq + (h * 3 + c) * PL + o;
+            const double* pu = su + h * 3 * PL + (CO ? c * PL + o : 3 * o + c);
+            const double* pm = sq + h * 3 * PL + (CO ? c * PL + o : 3 * o + c);
             double q[9];  // d at x-2..x+2 (q[0..4]), y-2, y-1, y+1, y+2 (q[5..8])
 #pragma unroll
-            for (int d = -2; d <= 2; d++) q[d + 2] = pu[d] - pm[d];
-            q[5] = pu[-2 * HX] - pm[-2 * HX];
-            q[6] = pu[-HX] - pm[-HX];
-            q[7] = pu[HX] - pm[HX];
-            q[8] = pu[2 * HX] - pm[2 * HX];
+            for (int d = -2; d <= 2; d++) q[d + 2] = pu[US * d] - pm[US * d];
+            q[5] = pu[US * (-2 * HX)] - pm[US * (-2 * HX)];
+            q[6] = pu[US * (-HX)] - pm[US * (-HX)];
+            q[7] = pu[US * (HX)] - pm[US * (HX)];
+            q[8] = pu[US * (2 * HX)] - pm[US * (2 * HX)];
             const double ax = rxp * (q[4] - 2 * q[3] + q[2]) - 2 * rx0 * (q[3] - 2 * q[2] + q[1]) +
                               rxm * (q[2] - 2 * q[1] + q[0]);
             const double ay = ryp * (q[8] - 2 * q[7] + q[2]) - 2 * ry0 * (q[7] - 2 * q[2] + q[6]) +
@@ -823,6 +901,9 @@ __device__ __forceinline__ void damp_dma_tile(int tix, int tjy, int k0, int k1, 
             ov[c] = upc[c] - birho * (wx * ax + wy * ay + wz * az);
          }
          op = col + nij * (k - b.kb);
+         if (POINT && gx[0] == 0 && gx[1] == 0 && gx[2] == 0 && gy[0] == 0 && gy[1] == 0 && gy[2] == 0 && gz0 == 0 &&
+             gz1 == 0 && gz2 == 0)
+            op = -1;
       }
 #pragma unroll
       for (int q = 0; q < 4; q++)
@@ -832,7 +913,7 @@ __device__ __forceinline__ void damp_dma_tile(int tix, int tjy, int k0, int k1, 
    }
    if (op >= 0) {
 #pragma unroll
-      for (int c = 0; c < 3; c++) up[op + npts * c] = ov[c];
+      for (int c = 0; c < 3; c++) up[at(c, op)] = ov[c];
    }
 }
 
@@ -863,6 +944,61 @@ k_damp_tiles(Box b, const DampTile* __restrict__ tiles, int ntiles, double* __re
    if (t >= ntiles) return;
    const DampTile d = tiles[t];
    damp_dma_tile<DW>(d.tix, d.tjy, d.k0, d.k1, b, up, u, um, rho, sg, beta);
+}
+
+// addsgd4 at kernel level, either layout: every tile of the box, each finding
+// from the profiles whether its columns meet an x or y layer, else which of
+// its planes a z layer reaches (kc <= 64), and leaving where none is
+// (against a thread per point: 201 x 201 x 101 points 315 -> 135 us, 301 x 301
+// x 171 interleaved 636 -> 360 us).
+template <bool DW, int CO>
+__global__ void __launch_bounds__(NT, CO ? 3 : 2)
+k_addsgd4(Box b, TileMap map, int kbeg, int kend, int kc, double* __restrict__ up, const double* __restrict__ u,
+          const double* __restrict__ um, const double* __restrict__ rho, SgCoef sg, double beta)
+{
+   const int per = (int)((map.ntiles + 7) / 8);
+   const int t = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+   if (t >= map.ntiles) return;
+   const int tix = t % map.ntx, tr = t / map.ntx, tjy = tr % map.nty, tkz = tr / map.nty;
+   int k0 = kbeg + tkz * kc, k1 = min(kend, k0 + kc - 1);
+   const int tid = threadIdx.x;
+   bool meets = false;  // dc of the tile's columns and of one more at each end
+   if (tid < TX + 2)
+      meets = sg.dcx[min(tix * TX + 1 + tid, (int)b.ni - 1)] != 0;
+   else if (tid >= 64 && tid < 64 + TY + 2)
+      meets = sg.dcy[min(tjy * TY + 1 + tid - 64, b.je - b.jb)] != 0;
+   if (!__syncthreads_or(meets)) {
+      const int k = k0 + (tid & 63), kk = k - b.kb;
+      const bool z = k <= k1 && (sg.dcz[kk - 1] != 0 || sg.dcz[kk] != 0 || sg.dcz[kk + 1] != 0);
+      const unsigned long long m = __ballot(z);  // the same in every wave
+      if (!m) return;
+      k1 = k0 + 63 - __clzll((long long)m);
+      k0 += __ffsll(m) - 1;
+   }
+   damp_dma_tile<DW, CO, true>(tix, tjy, k0, k1, b, up, u, um, rho, sg, beta);
+}
+
+int launch_addsgd4(int co, const Box& b, double* up, const double* u, const double* um, const double* rho,
+                   const SgCoef& sg, double beta, hipStream_t s)
+{
+   const int k1 = b.kb + 2, k2 = b.ke - 2;
+   if (beta == 0 || k2 < k1) return OK;
+   TileMap map;
+   map.ntx = (int)cdiv(b.ie - b.ib - 3, TX);
+   map.nty = (int)cdiv(b.je - b.jb - 3, TY);
+   const int kc = std::min(32, march_kchunk((long)map.ntx * map.nty, k2 - k1 + 1, 3));
+   map.ntiles = map.ntx * map.nty * (int)cdiv(k2 - k1 + 1, kc);
+   const unsigned grd = 8 * cdiv(map.ntiles, 8);
+   const bool fit = dma_fits(b, u, um, rho);
+   if (co && fit)
+      k_addsgd4<false, 1><<<grd, NT, 0, s>>>(b, map, k1, k2, kc, up, u, um, rho, sg, beta);
+   else if (co)
+      k_addsgd4<true, 1><<<grd, NT, 0, s>>>(b, map, k1, k2, kc, up, u, um, rho, sg, beta);
+   else if (fit)
+      k_addsgd4<false, 0><<<grd, NT, 0, s>>>(b, map, k1, k2, kc, up, u, um, rho, sg, beta);
+   else
+      k_addsgd4<true, 0><<<grd, NT, 0, s>>>(b, map, k1, k2, kc, up, u, um, rho, sg, beta);
+   return check_hip(hipGetLastError(), "addsgd4 launch");
 }
 
 // ---------------------------------------------------------------------------
@@ -1253,6 +1389,29 @@ int launch_sweep_lds(bool corr, int variant, const Box& b, int k1, int k2, int k
    }
 #undef SW4_SWEEP
    return check_hip(hipGetLastError(), corr ? "LDS corrector launch" : "LDS predictor launch");
+}
+
+int launch_rhs4_march(int co, const Box& b, int k1, int k2, const double* u, const double* mu, const double* la,
+                      const SgCoef& sg, double* out, double h, hipStream_t s)
+{
+   if (k2 < k1) return OK;
+   TileMap map;
+   map.ntx = (int)cdiv(b.ie - b.ib - 3, TX);
+   map.nty = (int)cdiv(b.je - b.jb - 3, TY);
+   const int kc = march_kchunk((long)map.ntx * map.nty, k2 - k1 + 1, 2);
+   map.ntiles = map.ntx * map.nty * (int)cdiv(k2 - k1 + 1, kc);
+   const unsigned grd = 8 * cdiv(map.ntiles, 8);
+   const double cof = 1.0 / (h * h);
+   const bool fit = dma_fits(b, u, mu, la);
+   if (co && fit)
+      k_rhs4_dma<false, 1><<<grd, NT, 0, s>>>(b, map, k1, k2, kc, u, mu, la, sg, out, cof);
+   else if (co)
+      k_rhs4_dma<true, 1><<<grd, NT, 0, s>>>(b, map, k1, k2, kc, u, mu, la, sg, out, cof);
+   else if (fit)
+      k_rhs4_dma<false, 0><<<grd, NT, 0, s>>>(b, map, k1, k2, kc, u, mu, la, sg, out, cof);
+   else
+      k_rhs4_dma<true, 0><<<grd, NT, 0, s>>>(b, map, k1, k2, kc, u, mu, la, sg, out, cof);
+   return check_hip(hipGetLastError(), "rhs4sg march launch");
 }
 
 int launch_sweep_lds_T(const Box& b, int k1, int k2, int kc, const double* w, const double* mu, const double* la,

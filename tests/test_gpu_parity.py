@@ -149,6 +149,46 @@ def test_addsgd4(torch, corder):
 
 
 @pytest.mark.parametrize("corder", [0, 1])
+@pytest.mark.parametrize("shape", [(45, 37, 70), (100, 60, 41), (96, 24, 30)])
+def test_addsgd4_layers(torch, corder, shape):
+    """Supergrid profiles, zero away from the layers: tiles that meet an x or
+    y layer, tiles with z layers only (whose planes the kernel selects), odd
+    and even rows; points that no profile reaches stay as they are, whatever
+    the data next to them."""
+    from sw4lite_amd import ew
+    from sw4lite_amd import lib as L
+    nx, ny, nz = shape
+    box, f = random_inputs(500 + corder, nx, ny, nz)
+    sg = ew.host_supergrid(L.grid_desc(nx, ny, nz, 0.1, [2] * 6, corder=corder, sg_gp_thickness=7))
+    one = [sg[k] for k in ("dcx", "dcy", "dcz", "strx", "stry", "strz", "cox", "coy", "coz")]
+    u, um, up0 = (to_layout(f[k], box, corder) for k in ("u", "um", "up"))
+    want = up0.copy()
+    O.addsgd4(corder, box, want, u, um, f["rho"], *one, 0.02)
+    on = [np.convolve(sg[k] != 0, [1, 1, 1], "same") > 0 for k in ("dcz", "dcy", "dcx")]
+    damped = on[0][:, None, None] | on[1][None, :, None] | on[2][None, None, :]
+    assert damped.any() and not damped.all()
+    args = [dev(torch, a) for a in (f["rho"], *one)]
+    up = dev(torch, up0)
+    ew.addsgd4(corder, box, up, dev(torch, u), dev(torch, um), *args, 0.02)
+    err = relerr(host(up) - up0, want - up0)
+    print("addsgd4 layers corder", corder, "shape", shape, "relerr", err, flush=True)
+    assert err < TOL
+    # an infinity everywhere outside the reach of the damped points
+    far = ~damped
+    for ax in range(3):
+        for s in (-2, -1, 1, 2):
+            far &= ~np.roll(damped, s, ax)
+    m = far.reshape(-1)
+    mask = np.concatenate([m, m, m]) if corder else np.repeat(m, 3)
+    bad = u.copy()
+    bad[mask] = np.inf
+    up = dev(torch, up0)
+    ew.addsgd4(corder, box, up, dev(torch, bad), dev(torch, um), *args, 0.02)
+    assert np.array_equal(host(up)[mask], up0[mask])
+    assert relerr(host(up) - up0, want - up0) < TOL
+
+
+@pytest.mark.parametrize("corder", [0, 1])
 @pytest.mark.parametrize("bc", [[2, 2, 2, 2, 0, 2], [1, 1, 2, 2, 2, 0], [3, 3, 3, 3, 0, 0], [2, 2, 1, 1, 1, 1]])
 def test_bcfortsg(torch, coefs, corder, bc):
     from sw4lite_amd import ew
