@@ -116,6 +116,7 @@ public:
 
    // --- time loop ---
    int step_reference(int n);  // stage order of EW::timesteploop (EW.C:2527-2842)
+   int step_curv(int n);       // the same on a curvilinear grid, pointwise stages merged (corder 1)
    // two fused sweeps per step; with stage_ms, kStages accumulated stage
    // times (ms): predictor interior, predictor boundary rows + ghost shell,
    // predictor sources + BC, corrector interior, corrector boundary rows +

@@ -28,6 +28,14 @@ int launch_addsgd4c(int co, const Box& b, double* up, const double* u, const dou
 // curv are the two grids' boxes (same i, j bounds).
 int launch_enforce_cart_topo(int co, const Box& cart, double* ucart, const Box& curv, double* ucurv, int g,
                              hipStream_t s);
+// The pointwise stages of the curvilinear step, component-blocked, sources
+// left out: up = 2u - um + dt^2/rho lu and acc = (up - 2u + um)/dt^2 on the
+// whole box; up += dt^4/(12 rho) lu - damping(u - um) on the planes k1..k2 of
+// the interior columns.
+int launch_curv_pred(const Box& b, const double* lu, const double* u, const double* um, const double* rho, double* up,
+                     double* acc, double dt, hipStream_t s);
+int launch_curv_corr(const Box& b, int k1, int k2, double* up, const double* lu, const double* u, const double* um,
+                     const double* rho, const double* jac, const SgCoef& sg, double beta, double dt, hipStream_t s);
 int launch_freesurf_curv(int co, const Box& b, int nz, int side, double* u, const double* mu, const double* la,
                          const double* met, const SbpTables* d_sbp, const double* forcing, const double* strx,
                          const double* stry, hipStream_t s);

@@ -23,6 +23,7 @@
 #include "kernels_common.h"
 #include "kernels_curv.h"
 #include "kernels_fast.h"
+#include "sbp_rows.h"
 
 namespace sw4amd {
 
@@ -130,21 +131,6 @@ __device__ __forceinline__ double vs4(const double m[4], const double f[5])
    return m[0] * (f[0] - f[2]) + m[1] * (f[1] - f[2]) + m[2] * (f[3] - f[2]) + m[3] * (f[4] - f[2]);
 }
 
-// rr coupling at (i,j,m): R[0..5] = 00, 11, 22, 01, 02, 12
-template <class S>
-__device__ __forceinline__ void rr_coef(const S& s, int i, int j, int m, double sx, double sy, double R[6])
-{
-   const double mu = s.MU(i, j, m), la = s.LA(i, j, m);
-   const double m2 = s.M(1, i, j, m), m3 = s.M(2, i, j, m), m4 = s.M(3, i, j, m);
-   const double x2 = m2 * sx * m2 * sx, y2 = m3 * sy * m3 * sy, z2 = m4 * m4;
-   R[0] = (2 * mu + la) * x2 + mu * (y2 + z2);
-   R[1] = (2 * mu + la) * y2 + mu * (x2 + z2);
-   R[2] = (2 * mu + la) * z2 + mu * (x2 + y2);
-   R[3] = (mu + la) * m2 * m3;
-   R[4] = (mu + la) * m2 * m4;
-   R[5] = (mu + la) * m3 * m4;
-}
-
 // traction-like combination of in-plane derivatives on plane m, column (i,j):
 // the pr/qr terms of the operator and the tangential part of the free-
 // surface traction (curvilinear-c.C:520-578)
@@ -160,154 +146,6 @@ __device__ __forceinline__ void t_terms(const S& s, int i, int j, int m, double 
    T[0] = K * a2 * p0 * sx * isy + mu * a3 * p1 + mu * a4 * p2 * isy + mu * a3 * q0 * sy * isx + la * a2 * q1;
    T[1] = la * a3 * p0 + mu * a2 * p1 * sx * isy + mu * a2 * q0 + K * a3 * q1 * sy * isx + mu * a4 * q2 * isx;
    T[2] = la * a4 * p0 * isy + mu * a2 * p2 * sx * isy + mu * a3 * q2 * sy * isx + la * a4 * q1 * isx;
-}
-
-template <class S>
-__device__ __forceinline__ void curv_point(const S& s, int i, int j, int k, const SbpTables* __restrict__ sbp,
-                                           double r[3])
-{
-   const double i6 = 1.0 / 6;
-   const double sx = s.SX(i), sy = s.SY(j);
-   const double isx = 1 / sx, isy = 1 / sy, isxy = isy * isx;
-   const int off[4] = {-2, -1, 1, 2};
-   const double wc[4] = {-CC2, -CC1, CC1, CC2};
-   r[0] = r[1] = r[2] = 0;
-
-   // pp and qq
-#pragma unroll
-   for (int c = 0; c < 3; c++) {
-      double a[5], m[4], f[5];
-#pragma unroll
-      for (int t = 0; t < 5; t++) {
-         const int ii = i + t - 2;
-         const double mu = s.MU(ii, j, k), m1 = s.M(0, ii, j, k);
-         a[t] = (c == 0 ? 2 * mu + s.LA(ii, j, k) : mu) * m1 * m1 * s.SX(ii);
-         f[t] = s.U(c, ii, j, k);
-      }
-      vc4(a, m);
-      r[c] += i6 * vs4(m, f) * isy;
-#pragma unroll
-      for (int t = 0; t < 5; t++) {
-         const int jj = j + t - 2;
-         const double mu = s.MU(i, jj, k), m1 = s.M(0, i, jj, k);
-         a[t] = (c == 1 ? 2 * mu + s.LA(i, jj, k) : mu) * m1 * m1 * s.SY(jj);
-         f[t] = s.U(c, i, jj, k);
-      }
-      vc4(a, m);
-      r[c] += i6 * vs4(m, f) * isx;
-   }
-
-   // rr
-   const double S3[3][3] = {{isxy, 1, isy}, {1, isxy, isx}, {isy, isx, isxy}};
-   const int PAIR[3][3] = {{0, 3, 4}, {3, 1, 5}, {4, 5, 2}};
-   {
-      // C_ab(q) = sum_m acof(k,q,m) R_ab(m), planes 1..8, then the ghost term
-#pragma unroll 1
-      for (int q = 1; q <= 8; q++) {
-         double Cq[6] = {0, 0, 0, 0, 0, 0};
-#pragma unroll 1
-         for (int mm = 1; mm <= 8; mm++) {
-            const double a = sbp->acof[(k - 1) + 6 * (q - 1) + 48 * (mm - 1)];
-            if (a == 0) continue;
-            double R[6];
-            rr_coef(s, i, j, mm, sx, sy, R);
-#pragma unroll
-            for (int e = 0; e < 6; e++) Cq[e] += a * R[e];
-         }
-#pragma unroll
-         for (int c = 0; c < 3; c++)
-#pragma unroll
-            for (int d = 0; d < 3; d++) r[c] += S3[c][d] * Cq[PAIR[c][d]] * s.U(d, i, j, q);
-      }
-      double R[6];
-      rr_coef(s, i, j, 1, sx, sy, R);
-      const double g = sbp->ghcof[k - 1];
-#pragma unroll
-      for (int c = 0; c < 3; c++)
-#pragma unroll
-         for (int d = 0; d < 3; d++) r[c] += S3[c][d] * (g * R[PAIR[c][d]]) * s.U(d, i, j, 0);
-   }
-
-   // pq and qp (u and v equations)
-#pragma unroll
-   for (int t = 0; t < 4; t++) {
-      const int d = off[t];
-      const double mq = s.M(0, i, j + d, k), mp = s.M(0, i + d, j, k);
-      r[0] += wc[t] * (s.MU(i, j + d, k) * mq * mq * s.Dp(1, i, j + d, k) +
-                       s.LA(i + d, j, k) * mp * mp * s.Dq(1, i + d, j, k));
-      r[1] += wc[t] * (s.LA(i, j + d, k) * mq * mq * s.Dp(0, i, j + d, k) +
-                       s.MU(i + d, j, k) * mp * mp * s.Dq(0, i + d, j, k));
-   }
-
-   // k-derivative weights of this row
-   constexpr int NQ = 8;
-   int kq[NQ];
-   double wq[NQ];
-#pragma unroll
-   for (int e = 0; e < NQ; e++) {
-      kq[e] = e + 1;
-      wq[e] = sbp->bope[(k - 1) + 6 * e];
-   }
-
-   // pr and qr
-#pragma unroll
-   for (int e = 0; e < NQ; e++) {
-      double T[3];
-      t_terms(s, i, j, kq[e], sx, sy, isx, isy, T);
-#pragma unroll
-      for (int c = 0; c < 3; c++) r[c] += wq[e] * T[c];
-   }
-
-   // rp and rq
-#pragma unroll
-   for (int t = 0; t < 4; t++) {
-      const int d = off[t];
-      double dx[3] = {0, 0, 0}, dy[3] = {0, 0, 0};
-#pragma unroll
-      for (int e = 0; e < NQ; e++)
-#pragma unroll
-         for (int c = 0; c < 3; c++) {
-            dx[c] += wq[e] * s.U(c, i + d, j, kq[e]);
-            dy[c] += wq[e] * s.U(c, i, j + d, kq[e]);
-         }
-      {
-         const int ii = i + d;
-         const double mu = s.MU(ii, j, k), la = s.LA(ii, j, k), sxi = s.SX(ii);
-         const double m1 = s.M(0, ii, j, k), m2 = s.M(1, ii, j, k), m3 = s.M(2, ii, j, k), m4 = s.M(3, ii, j, k);
-         r[0] += wc[t] * ((2 * mu + la) * m2 * m1 * sxi * dx[0] + la * m3 * m1 * dx[1] * sy + la * m4 * m1 * dx[2]) *
-                 isy;
-         r[1] += wc[t] * (mu * m3 * m1 * dx[0] + mu * m2 * m1 * dx[1] * sxi * isy);
-         r[2] += wc[t] * (mu * m4 * m1 * dx[0] + mu * m2 * m1 * dx[2] * sxi) * isy;
-      }
-      {
-         const int jj = j + d;
-         const double mu = s.MU(i, jj, k), la = s.LA(i, jj, k), syj = s.SY(jj);
-         const double m1 = s.M(0, i, jj, k), m2 = s.M(1, i, jj, k), m3 = s.M(2, i, jj, k), m4 = s.M(3, i, jj, k);
-         r[0] += wc[t] * (mu * m3 * m1 * dy[0] * syj * isx + mu * m2 * m1 * dy[1]);
-         r[1] += wc[t] * (la * m2 * m1 * dy[0] + (2 * mu + la) * m3 * m1 * dy[1] * syj * isx +
-                          la * m4 * m1 * dy[2] * isx);
-         r[2] += wc[t] * (mu * m3 * m1 * dy[2] * syj + mu * m4 * m1 * dy[1]) * isx;
-      }
-   }
-}
-
-// Component-blocked layout: capped at 256 registers for 2 waves/SIMD (2-4
-// spilled; 262 registers and 1 wave/SIMD without the cap).  The interleaved
-// layout's index arithmetic would spill ~120 registers under the cap.
-template <int CO>
-__global__ void __launch_bounds__(256, CO ? 2 : 1)
-k_rhs4curv(Box b, int klo, int khi, const SbpTables* __restrict__ sbp, CurvG<CO> s,
-           const double* __restrict__ jac, double* __restrict__ lu)
-{
-   const int i = b.ib + 2 + blockIdx.x * blockDim.x + threadIdx.x;
-   const int j = b.jb + 2 + blockIdx.y * blockDim.y + threadIdx.y;
-   const int k = klo + blockIdx.z;
-   if (i > b.ie - 2 || j > b.je - 2 || k > khi) return;
-   double r[3];
-   curv_point(s, i, j, k, sbp, r);
-   const double ij = s.SX(i) * s.SY(j) / jac[sidx(b, i, j, k)];
-#pragma unroll
-   for (int c = 0; c < 3; c++) lu[vidx<CO>(b, c, i, j, k)] = r[c] * ij;
 }
 
 // The interior rows as a k-march with every first derivative formed once.
@@ -336,6 +174,25 @@ k_rhs4curv(Box b, int klo, int khi, const SbpTables* __restrict__ sbp, CurvG<CO>
 #define SW4_SCHED_FENCE __builtin_amdgcn_sched_barrier(0)
 constexpr int MTX = 32, MTY = 8, MHX = MTX + 4, MHY = MTY + 4, MPL = MHX * MHY, MNT = 448;
 
+// A thread's point of the tile with its halo, and its part: 0 output, 1 j
+// halo, 2 i halo and corners (whole waves; the last 16 threads repeat a point).
+__device__ __forceinline__ void march_point(int tid, int& role, int& hx, int& hy)
+{
+   role = __builtin_amdgcn_readfirstlane(tid < 256 ? 0 : tid < 384 ? 1 : 2);
+   if (tid < 256) {
+      hx = 2 + tid % MTX;
+      hy = 2 + tid / MTX;
+   } else if (tid < 384) {
+      const int r = (tid - 256) / MTX;
+      hx = 2 + tid % MTX;
+      hy = r < 2 ? r : r + MTY;
+   } else {
+      const int q = tid - 384, c = q % 4, r = q / 4;  // rows 0..7: the tile's, 8..11: the corners'
+      hx = c < 2 ? c : c + MTX;
+      hy = r < MTY ? 2 + r : r < MTY + 2 ? r - MTY : r < MTY + 4 ? r : 2;
+   }
+}
+
 template <int CO>
 __global__ void __launch_bounds__(MNT, 1)
 k_rhs4curv_march(Box b, int ntx, int nty, int ntiles, int klo, int khi, int kc, CurvG<CO> s,
@@ -353,21 +210,8 @@ k_rhs4curv_march(Box b, int ntx, int nty, int ntiles, int klo, int khi, int kc, 
    const int tix = t % ntx, tr = t / ntx, tjy = tr % nty, tkz = tr / nty;
    const int k0 = klo + tkz * kc, k1 = min(khi, k0 + kc - 1);
    const int tid = threadIdx.x;
-   // 0: output, 1: j halo, 2: i halo (and corners)
-   const int role = __builtin_amdgcn_readfirstlane(tid < 256 ? 0 : tid < 384 ? 1 : 2);
-   int hx, hy;
-   if (tid < 256) {
-      hx = 2 + tid % MTX;
-      hy = 2 + tid / MTX;
-   } else if (tid < 384) {
-      const int r = (tid - 256) / MTX;
-      hx = 2 + tid % MTX;
-      hy = r < 2 ? r : r + MTY;
-   } else {
-      const int q = tid - 384, c = q % 4, r = q / 4;  // rows 0..7: the tile's, 8..11: the corners'
-      hx = c < 2 ? c : c + MTX;
-      hy = r < MTY ? 2 + r : r < MTY + 2 ? r - MTY : r < MTY + 4 ? r : 2;
-   }
+   int role, hx, hy;
+   march_point(tid, role, hx, hy);
    const bool own = tid < MPL;  // the last 16 threads repeat a point and store nothing
    const Box& b_ = b;
    const int ia = b_.ib + tix * MTX, ja = b_.jb + tjy * MTY;
@@ -573,6 +417,181 @@ k_rhs4curv_march(Box b, int ntx, int nty, int ntiles, int klo, int khi, int kc, 
    }
 }
 
+// The top six rows (k = 1..6, SBP closures along k) with the same grouping
+// and the same threads as the march: the planes k = 1..8 go to LDS once, T of
+// the eight planes and the material of the column's rr stay in registers for
+// all rows; per row the columns form F and G, one barrier, and the outputs
+// are finished.  With rr written as in the march,
+//   rr = 1/(sx sy) sum_q [mu |m|^2 w_a + (mu + lambda) m_a (m . w)]_q,
+//   w_b(k, q) = sum_t acof(k, t, q) u_b(t)  (and ghcof on the ghost plane).
+// block.y takes the rows 1 + block.y, the next gridDim.y on.  Against a
+// thread per point (6049 operations): 384 x 384 points 394 -> 127 us,
+// 65 x 65 40 -> 17.
+template <int CO>
+__global__ void __launch_bounds__(MNT, 1)
+k_rhs4curv_rows(Box b, int ntx, const SbpTables* __restrict__ sbp, CurvG<CO> s, const double* __restrict__ jac,
+                double* __restrict__ lu)
+{
+   __shared__ double su[8 * 3 * MPL];          // u of planes 1..8
+   __shared__ double se[6 * 2 * MPL];          // mu M1^2, lambda M1^2 of the rows' planes
+   __shared__ double sf[2][3 * MHX * MTY];     // F over the tile's rows, i halo included
+   __shared__ double sg[2][3 * MTX * MHY];     // G over the tile's columns, j halo included
+   __shared__ double ssx[MHX], ssy[MHY];
+   const int tix = blockIdx.x % ntx, tjy = blockIdx.x / ntx;
+   const int tid = threadIdx.x;
+   int role, hx, hy;
+   march_point(tid, role, hx, hy);
+   const bool own = tid < MPL;
+   const bool ihalo = role == 2 && tid < 384 + 4 * MTY;
+   const int ia = b.ib + tix * MTX, ja = b.jb + tjy * MTY;
+   const bool active = role == 0 && ia + hx <= b.ie - 2 && ja + hy <= b.je - 2;
+   const int i = min(ia + hx, b.ie), j = min(ja + hy, b.je);
+   const long nij = b.nij, npts = b.npts;
+   const long col = (i - b.ib) + b.ni * (j - b.jb);
+   const double sx = s.SX(i), sy = s.SY(j), isx = 1 / sx, isy = 1 / sy, xy = sx * isy, yx = sy * isx;
+   if (tid < MHX) ssx[tid] = s.SX(min(ia + tid, b.ie));
+   if (tid >= 64 && tid < 64 + MHY) ssy[tid - 64] = s.SY(min(ja + tid - 64, b.je));
+   const int o = hy * MHX + hx;
+   auto D = [](const double* f, int st) { return CC2 * (f[2 * st] - f[-2 * st]) + CC1 * (f[st] - f[-st]); };
+   auto at = [=](int c, long p) { return CO ? p + npts * c : 3 * p + c; };
+   auto met = [=](int c, long p) { return s.met[CO ? p + npts * c : 4 * p + c]; };
+
+   double u[9][3];
+#pragma unroll
+   for (int q = 0; q <= 8; q++) {
+      const long p = col + nij * (q - b.kb);
+#pragma unroll
+      for (int c = 0; c < 3; c++) u[q][c] = s.u[at(c, p)];
+      if (own && q >= 1) {
+#pragma unroll
+         for (int c = 0; c < 3; c++) su[((q - 1) * 3 + c) * MPL + o] = u[q][c];
+         if (q <= 6) {
+            const double m1 = met(0, p);
+            se[(2 * q - 2) * MPL + o] = s.mu[p] * m1 * m1;
+            se[(2 * q - 1) * MPL + o] = s.la[p] * m1 * m1;
+         }
+      }
+   }
+   __syncthreads();
+   // of the planes 1..8: T, and mu |m|^2, mu + lambda, m of rr
+   double T[9][3], mn[9], ml[9], mx_[9], my_[9], mz_[9];
+   if (role == 0) {
+#pragma unroll
+      for (int q = 1; q <= 8; q++) {
+         SW4_SCHED_FENCE;
+         const long pt = col + nij * (q - b.kb);
+         const double mu = s.mu[pt], la = s.la[pt], m1 = met(0, pt), m2 = met(1, pt), m3 = met(2, pt), m4 = met(3, pt);
+         const double* f = su + (q - 1) * 3 * MPL + o;
+         const double p0 = D(f, 1), p1 = D(f + MPL, 1), p2 = D(f + 2 * MPL, 1);
+         const double q0 = D(f, MHX), q1 = D(f + MPL, MHX), q2 = D(f + 2 * MPL, MHX);
+         const double a2 = m2 * m1, a3 = m3 * m1, a4 = m4 * m1, K = 2 * mu + la;
+         T[q][0] = K * a2 * xy * p0 + mu * (a3 * p1 + a4 * isy * p2 + a3 * yx * q0) + la * a2 * q1;
+         T[q][1] = la * a3 * p0 + mu * (a2 * xy * p1 + a2 * q0 + a4 * isx * q2) + K * a3 * yx * q1;
+         T[q][2] = la * a4 * (isy * p0 + isx * q1) + mu * (a2 * xy * p2 + a3 * yx * q2);
+         mx_[q] = m2 * sx;
+         my_[q] = m3 * sy;
+         mz_[q] = m4;
+         mn[q] = mu * (mx_[q] * mx_[q] + my_[q] * my_[q] + mz_[q] * mz_[q]);
+         ml[q] = mu + la;
+      }
+   }
+   int par = 0;
+#pragma unroll 1
+   for (int kr = 1 + (int)blockIdx.y; kr <= 6; kr += (int)gridDim.y) {
+      const long pt = col + nij * (kr - b.kb);
+      const double mu = s.mu[pt], la = s.la[pt], m1 = met(0, pt), m2 = met(1, pt), m3 = met(2, pt), m4 = met(3, pt);
+      const double w = role == 0 ? sx * sy / jac[pt] : 0.0;
+      const double* f = su + (kr - 1) * 3 * MPL + o;
+      double dz[3] = {0, 0, 0}, z[3] = {0, 0, 0};
+#pragma unroll
+      for (int q = 1; q <= 8; q++) {
+         const double bq = sbp->bope[(kr - 1) + 6 * (q - 1)];
+#pragma unroll
+         for (int c = 0; c < 3; c++) dz[c] += bq * u[q][c];
+         if (role == 0) {
+#pragma unroll
+            for (int c = 0; c < 3; c++) z[c] += bq * T[q][c];
+         }
+      }
+      {
+         const double q = m1 * m1, a2 = m2 * m1, a3 = m3 * m1, a4 = m4 * m1, K = 2 * mu + la;
+         if (role == 0 || ihalo) {
+            double* v = &sf[par][(hy - 2) * MHX + hx];
+            v[0] = la * (q * D(f + MPL, MHX) + isy * (a3 * sy * dz[1] + a4 * dz[2])) + K * a2 * xy * dz[0];
+            v[MHX * MTY] = mu * (q * D(f, MHX) + a3 * dz[0] + a2 * xy * dz[1]);
+            v[2 * MHX * MTY] = mu * (a4 * dz[0] + a2 * sx * dz[2]) * isy;
+         }
+         if (role != 2) {
+            double* v = &sg[par][hy * MTX + hx - 2];
+            v[0] = mu * (q * D(f + MPL, 1) + a3 * yx * dz[0] + a2 * dz[1]);
+            v[MTX * MHY] = la * (q * D(f, 1) + a2 * dz[0] + a4 * isx * dz[2]) + K * a3 * yx * dz[1];
+            v[2 * MTX * MHY] = mu * (a3 * sy * dz[2] + a4 * dz[1]) * isx;
+         }
+      }
+      SW4_SCHED_FENCE;
+      if (role == 0) {
+         double rr[3] = {0, 0, 0};
+#pragma unroll
+         for (int q = 1; q <= 8; q++) {
+            double v[3] = {0, 0, 0};
+            if (q == 1) {  // the ghost plane's term carries plane 1's coefficients
+               const double g = sbp->ghcof[kr - 1];
+#pragma unroll
+               for (int c = 0; c < 3; c++) v[c] = g * u[0][c];
+            }
+#pragma unroll
+            for (int e = 1; e <= 8; e++) {
+               const double a = sbp->acof[(kr - 1) + 6 * (e - 1) + 48 * (q - 1)];
+#pragma unroll
+               for (int c = 0; c < 3; c++) v[c] += a * u[e][c];
+            }
+            const double t = ml[q] * (mx_[q] * v[0] + my_[q] * v[1] + mz_[q] * v[2]);
+            rr[0] += mn[q] * v[0] + t * mx_[q];
+            rr[1] += mn[q] * v[1] + t * my_[q];
+            rr[2] += mn[q] * v[2] + t * mz_[q];
+         }
+#pragma unroll
+         for (int c = 0; c < 3; c++) z[c] += isx * isy * rr[c];
+      }
+      __syncthreads();
+      if (active) {
+         const double* pe = se + (2 * kr - 2) * MPL + o;
+         double mx[4], my[4], cx[4], cy[4], am[5], al[5];
+#pragma unroll
+         for (int e = 0; e < 5; e++) {
+            am[e] = pe[e - 2] * ssx[hx + e - 2];
+            al[e] = pe[MPL + e - 2] * ssx[hx + e - 2];
+         }
+         vc4(am, mx);
+         vc4(al, cx);
+#pragma unroll
+         for (int e = 0; e < 5; e++) {
+            am[e] = pe[(e - 2) * MHX] * ssy[hy + e - 2];
+            al[e] = pe[MPL + (e - 2) * MHX] * ssy[hy + e - 2];
+         }
+         vc4(am, my);
+         vc4(al, cy);
+#pragma unroll
+         for (int e = 0; e < 4; e++) {
+            cx[e] += 2 * mx[e];
+            cy[e] += 2 * my[e];
+         }
+         const double* vf = &sf[par][(hy - 2) * MHX + hx];
+         const double* vg = &sg[par][hy * MTX + hx - 2];
+#pragma unroll
+         for (int c = 0; c < 3; c++) {
+            const double* g = f + c * MPL;
+            const double x[5] = {g[-2], g[-1], g[0], g[1], g[2]};
+            const double y[5] = {g[-2 * MHX], g[-MHX], g[0], g[MHX], g[2 * MHX]};
+            const double r = z[c] + (1.0 / 6) * (isy * vs4(c == 0 ? cx : mx, x) + isx * vs4(c == 1 ? cy : my, y)) +
+                             D(vf + c * MHX * MTY, 1) + D(vg + c * MTX * MHY, MTX);
+            lu[at(c, pt)] = r * w;
+         }
+      }
+      par ^= 1;
+   }
+}
+
 // ---------------------------------------------------------------------------
 // Supergrid damping in x and y with rho -> rho jac
 // ---------------------------------------------------------------------------
@@ -617,6 +636,135 @@ k_addsgd4c(Box b, double* __restrict__ up, const double* __restrict__ u, const d
       const double ay = ry[2] * (dy[4] - 2 * dy[3] + dy[2]) - 2 * ry[1] * (dy[3] - 2 * dy[2] + dy[1]) +
                         ry[0] * (dy[2] - 2 * dy[1] + dy[0]);
       up[vidx<CO>(b, c, i, j, k)] -= w * (wx * ax + wy * ay);
+   }
+}
+
+// ---------------------------------------------------------------------------
+// The pointwise stages of the curvilinear step around the operator, in two
+// passes (component-blocked): predictor and acceleration, and corrector with
+// the supergrid damping.  Sources, which act on a few points, follow each.
+// ---------------------------------------------------------------------------
+// up = 2u - um + dt2/rho lu, acc = (up - 2u + um) dt2i on the whole box
+__global__ void __launch_bounds__(256)
+k_curv_pred(long npts, const double* __restrict__ lu, const double* __restrict__ u, const double* __restrict__ um,
+            const double* __restrict__ rho, double* __restrict__ up, double* __restrict__ acc, double dt2, double dt2i)
+{
+   const long p = blockIdx.x * (long)blockDim.x + threadIdx.x;
+   if (p >= npts) return;
+   const double sc = dt2 / rho[p];
+#pragma unroll
+   for (int c = 0; c < 3; c++) {
+      const long q = p + npts * c;
+      const double uv = u[q], mv = um[q], v = 2 * uv - mv + sc * lu[q];
+      up[q] = v;
+      acc[q] = dt2i * (v - 2 * uv + mv);
+   }
+}
+
+// up += c4/rho lu - damping(u - um) (addsgd4c) on the interior columns of a
+// 32 x 8 tile, planes k0..k1.  Tiles that meet an x or y layer stage d = u - um
+// and rho jac of a plane in LDS, loaded one plane ahead by a thread for each
+// point of the tile and its halo (one barrier per plane); the others only add.
+// Bound by memory.
+__global__ void __launch_bounds__(MNT, 2)
+k_curv_corr(Box b, int ntx, int nty, int ntiles, int klo, int khi, int kc, double* __restrict__ up,
+            const double* __restrict__ lu, const double* __restrict__ u, const double* __restrict__ um,
+            const double* __restrict__ rho, const double* __restrict__ jac, SgCoef sg, double c4, double beta)
+{
+   __shared__ double sd[2][3 * MPL];
+   __shared__ double sr[2][MPL];
+   const int per = (ntiles + 7) / 8;
+   const int t = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+   if (t >= ntiles) return;
+   const int tix = t % ntx, tr = t / ntx, tjy = tr % nty, tkz = tr / nty;
+   const int k0 = klo + tkz * kc, k1 = min(khi, k0 + kc - 1);
+   const int tid = threadIdx.x;
+   int role, hx, hy;
+   march_point(tid, role, hx, hy);
+   const int ia = b.ib + tix * MTX, ja = b.jb + tjy * MTY;
+   const bool active = role == 0 && ia + hx <= b.ie - 2 && ja + hy <= b.je - 2;
+   const int ii = min(ia + hx, b.ie) - b.ib, jj = min(ja + hy, b.je) - b.jb;
+   const long nij = b.nij, npts = b.npts;
+   const long col = ii + b.ni * jj;
+   bool meets = false;  // dc of the tile's columns and of one more at each end
+   if (beta != 0 && tid < MTX + 2)
+      meets = sg.dcx[min(tix * MTX + 1 + tid, (int)b.ni - 1)] != 0;
+   else if (beta != 0 && tid >= 64 && tid < 64 + MTY + 2)
+      meets = sg.dcy[min(tjy * MTY + 1 + tid - 64, b.je - b.jb)] != 0;
+   if (!__syncthreads_or(meets)) {
+      if (!active) return;
+      for (int k = k0; k <= k1; k++) {
+         const long p = col + nij * (k - b.kb);
+         const double sc = c4 / rho[p];
+#pragma unroll
+         for (int c = 0; c < 3; c++) up[p + npts * c] += sc * lu[p + npts * c];
+      }
+      return;
+   }
+   const int o = hy * MHX + hx;
+   const bool own = tid < MPL;
+   // of an output's column: dc at -1, 0, +1 and the weights
+   double gx[3] = {0, 0, 0}, gy[3] = {0, 0, 0}, wx = 0, wy = 0;
+   if (active) {
+#pragma unroll
+      for (int e = 0; e < 3; e++) {
+         gx[e] = sg.dcx[ii + e - 1];
+         gy[e] = sg.dcy[jj + e - 1];
+      }
+      wx = sg.strx[ii] * sg.coy[jj];
+      wy = sg.stry[jj] * sg.cox[ii];
+   }
+   const bool damped = gx[0] != 0 || gx[1] != 0 || gx[2] != 0 || gy[0] != 0 || gy[1] != 0 || gy[2] != 0;
+   double nu[3], nm[3], nr, nj, np[3] = {0, 0, 0}, nl[3] = {0, 0, 0};
+   auto load = [&](int k) {
+      const long p = col + nij * (k - b.kb);
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+         nu[c] = u[p + npts * c];
+         nm[c] = um[p + npts * c];
+         if (role == 0) {
+            np[c] = up[p + npts * c];
+            nl[c] = lu[p + npts * c];
+         }
+      }
+      nr = rho[p];
+      nj = jac[p];
+   };
+   load(k0);
+   int par = 0;
+   for (int k = k0; k <= k1; k++) {
+      double d[3], pv[3], lv[3];
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+         d[c] = nu[c] - nm[c];
+         pv[c] = np[c];
+         lv[c] = nl[c];
+      }
+      const double r = nr, rj = nr * nj;
+      if (own) {
+#pragma unroll
+         for (int c = 0; c < 3; c++) sd[par][c * MPL + o] = d[c];
+         sr[par][o] = rj;
+      }
+      __syncthreads();  // plane k is staged; plane k-1 was read from the other half
+      if (k < k1) load(k + 1);
+      if (active) {
+         const double* q = &sr[par][o];
+         const double w = beta / rj, sc = c4 / r;
+         const double x2 = q[1] * gx[2], x1 = rj * gx[1], x0 = q[-1] * gx[0];
+         const double y2 = q[MHX] * gy[2], y1 = rj * gy[1], y0 = q[-MHX] * gy[0];
+#pragma unroll
+         for (int c = 0; c < 3; c++) {
+            const double* e = &sd[par][c * MPL + o];
+            const double ax = x2 * (e[2] - 2 * e[1] + d[c]) - 2 * x1 * (e[1] - 2 * d[c] + e[-1]) +
+                              x0 * (d[c] - 2 * e[-1] + e[-2]);
+            const double ay = y2 * (e[2 * MHX] - 2 * e[MHX] + d[c]) - 2 * y1 * (e[MHX] - 2 * d[c] + e[-MHX]) +
+                              y0 * (d[c] - 2 * e[-MHX] + e[-2 * MHX]);
+            const double v = pv[c] + sc * lv[c];
+            up[col + nij * (k - b.kb) + npts * c] = damped ? v - w * (wx * ax + wy * ay) : v;
+         }
+      }
+      par ^= 1;
    }
 }
 
@@ -753,13 +901,12 @@ template <int CO>
 static void rhs4curv_co(const Box& b, const int* onesided, const SbpTables* d_sbp, const CurvG<CO>& cg,
                         const double* jac, double* lu, hipStream_t s)
 {
-   const int nii = b.ie - b.ib - 3, njj = b.je - b.jb - 3;
-   dim3 blk(64, 4, 1);
+   const int ntx = (int)cdiv(b.ie - b.ib - 3, MTX), nty = (int)cdiv(b.je - b.jb - 3, MTY);
    const int top = onesided[4] == 1;
    const int k1 = top ? 7 : b.kb + 2, k2 = b.ke - 2;
-   if (top) k_rhs4curv<CO><<<dim3(cdiv(nii, 64), cdiv(njj, 4), 6), blk, 0, s>>>(b, 1, 6, d_sbp, cg, jac, lu);
+   if (top)
+      k_rhs4curv_rows<CO><<<dim3(ntx * nty, sbp_rows_spread(ntx * nty, 1)), MNT, 0, s>>>(b, ntx, d_sbp, cg, jac, lu);
    if (k2 >= k1) {
-      const int ntx = (int)cdiv(nii, MTX), nty = (int)cdiv(njj, MTY);
       const int kc = march_kchunk((long)ntx * nty, k2 - k1 + 1, 1);
       const int ntiles = ntx * nty * (int)cdiv(k2 - k1 + 1, kc);
       k_rhs4curv_march<CO><<<8 * cdiv(ntiles, 8), MNT, 0, s>>>(b, ntx, nty, ntiles, k1, k2, kc, cg, jac, lu);
@@ -788,6 +935,25 @@ int launch_addsgd4c(int co, const Box& b, double* up, const double* u, const dou
    else
       k_addsgd4c<0><<<grd, blk, 0, s>>>(b, up, u, um, rho, jac, sg, beta);
    return check_hip(hipGetLastError(), "addsgd4c launch");
+}
+
+int launch_curv_pred(const Box& b, const double* lu, const double* u, const double* um, const double* rho, double* up,
+                     double* acc, double dt, hipStream_t s)
+{
+   k_curv_pred<<<cdiv(b.npts, 256), 256, 0, s>>>(b.npts, lu, u, um, rho, up, acc, dt * dt, 1.0 / (dt * dt));
+   return check_hip(hipGetLastError(), "curvilinear predictor launch");
+}
+
+int launch_curv_corr(const Box& b, int k1, int k2, double* up, const double* lu, const double* u, const double* um,
+                     const double* rho, const double* jac, const SgCoef& sg, double beta, double dt, hipStream_t s)
+{
+   if (k2 < k1) return OK;
+   const int ntx = (int)cdiv(b.ie - b.ib - 3, MTX), nty = (int)cdiv(b.je - b.jb - 3, MTY);
+   const int kc = march_kchunk((long)ntx * nty, k2 - k1 + 1, 2);
+   const int ntiles = ntx * nty * (int)cdiv(k2 - k1 + 1, kc);
+   k_curv_corr<<<8 * cdiv(ntiles, 8), MNT, 0, s>>>(b, ntx, nty, ntiles, k1, k2, kc, up, lu, u, um, rho, jac, sg,
+                                                   dt * dt * dt * dt / 12, beta);
+   return check_hip(hipGetLastError(), "curvilinear corrector launch");
 }
 
 int launch_freesurf_curv(int co, const Box& b, int nz, int side, double* u, const double* mu, const double* la,

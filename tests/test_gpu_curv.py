@@ -157,14 +157,17 @@ def test_freesurfcurvisg(torch, coefs, corder, side, forced):
     assert np.array_equal(got != u0, want != u0)
 
 
-@pytest.mark.parametrize("corder,bc", [(1, [2, 2, 2, 2, 0, 2]), (0, [2, 2, 2, 2, 0, 1]), (1, [1, 2, 2, 1, 2, 2])])
-def test_curvilinear_time_loop(torch, corder, bc):
+@pytest.mark.parametrize("corder,bc,shape", [
+    (1, [2, 2, 2, 2, 0, 2], (33, 29, 24)), (0, [2, 2, 2, 2, 0, 1], (33, 29, 24)), (1, [1, 2, 2, 1, 2, 2], (33, 29, 24)),
+    # tiles that meet a supergrid layer and tiles that do not, whole tiles and a column more
+    (1, [2, 2, 2, 2, 0, 2], (100, 41, 14)), (1, [2, 2, 2, 2, 0, 2], (64, 40, 13))])
+def test_curvilinear_time_loop(torch, corder, bc, shape):
     """The EW time loop on a grid under Gaussian hills (reference stage order
     with rhs4sgcurv, addsgd4cfort and the curved free-surface closure) against
     the oracle's loop: same dt, sources, and displacements after 8 steps."""
     from oracle.loop import OracleRun
     from sw4lite_amd import EW
-    nx, ny, nz, h = 33, 29, 24, 0.05
+    (nx, ny, nz), h = shape, 0.05
     _, z = hills_depth(nx, ny, nz, h, 12)
     box, f = random_inputs(13, nx, ny, nz)
     rho = 1.5 + 0.2 * f["rho"]
