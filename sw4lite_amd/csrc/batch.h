@@ -67,16 +67,18 @@ private:
    std::vector<DampTile*> m_dtiles;  // per shot: its damping tile list (kernel variant 9), or null
    std::vector<int> m_ndtiles;
    std::vector<double*> m_acc;       // per shot: its acceleration field (kernel variant 8 and later), or null
-   std::vector<char> m_useacc;       // [phase][shot]: the sweeps store and stage the acceleration
    std::vector<hipStream_t> m_saved;
    WorkPool m_wpool;  // the shots' gradient work memory
    // the per-grid boundary work of the shots runs on NSIDE streams (default
    // priority) forked from and joined back into m_s, so the small kernels of
    // different grids overlap; the fork/join is captured into the graph too
    static constexpr int NSIDE = 4;
-   hipStream_t m_side[NSIDE] = {nullptr, nullptr, nullptr, nullptr};
+   // one more for the batched sweeps of the grids that take 16-byte loads,
+   // beside those of the others on the batch's own stream
+   static constexpr int WIDE = NSIDE, NSTREAM = NSIDE + 1;
+   hipStream_t m_side[NSTREAM] = {};
    hipEvent_t m_fork = nullptr;
-   hipEvent_t m_join[NSIDE] = {nullptr, nullptr, nullptr, nullptr};
+   hipEvent_t m_join[NSTREAM] = {};
    int fork();
    int join();
 };

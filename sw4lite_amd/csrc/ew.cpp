@@ -74,11 +74,12 @@ int EW::init()
 
 // The whole acceleration for kernel variant 8 (3 npts doubles, allocated at
 // the first step that uses it); null for the other variants and for odd row
-// lengths, whose sweeps cannot stage it.
-int EW::accel_field(double** p)
+// lengths, whose sweeps cannot stage it (always: whatever the variant, for
+// the batch, whose sweeps all do).
+int EW::accel_field(double** p, bool always)
 {
    *p = nullptr;
-   if (m_variant < 8 || (m_box.ni % 2 != 0 && m_variant < 10)) return OK;
+   if (!always && (m_variant < 8 || (m_box.ni % 2 != 0 && m_variant < 10))) return OK;
    if (!m_accf) {
       void* q = nullptr;
       if (hipMalloc(&q, sizeof(double) * 3 * m_box.npts) != hipSuccess) {

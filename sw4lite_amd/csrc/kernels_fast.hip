@@ -1013,14 +1013,6 @@ __device__ __forceinline__ int find_shot(const SweepShot* __restrict__ shots, in
    return s;
 }
 
-template <bool CORR>
-__global__ void __launch_bounds__(NT, 2) k_sweep_batch(const SweepShot* __restrict__ shots, int nshots)
-{
-   const SweepShot& h = shots[find_shot(shots, nshots, blockIdx.x)];
-   sweep_lds_body<CORR, false, false>(blockIdx.x - h.grid0, h.b, h.map, h.kbeg, h.kend, h.kc, h.upin, h.u, h.um, h.mu,
-                                      h.la, h.rho, h.sg, h.out, h.cof, h.dt2i, h.cupd, h.beta);
-}
-
 // A shot's tile of the batched damping sweep: from its tile list where it
 // has one (entry t of the list, each XCD taking one contiguous run), else
 // from its tile map.  false: no tile for this block.
@@ -1079,23 +1071,22 @@ int fill_sweep_shot(bool damping, const Box& b, int k1, int k2, int kc, const do
    return grid0 + 8 * (int)cdiv(sh->map.ntiles, 8);
 }
 
-// Batched predictor of grids whose planes take the 16-byte asynchronous
-// loads (async_loads_fit).
-// (the predictor stores the acceleration in acc where the shot has one)
-__global__ void __launch_bounds__(NT, 2) k_sweep_dma_batch(const SweepShot* __restrict__ shots, int nshots)
+// Batched predictor, storing the acceleration, and batched corrector staging
+// it: 16-byte loads for the grids they fit, four-byte ones (DW) for the others.
+template <bool DW>
+__global__ void __launch_bounds__(NT, 2) k_pred_batch(const SweepShot* __restrict__ shots, int nshots)
 {
    const SweepShot& h = shots[find_shot(shots, nshots, blockIdx.x)];
-   sweep_dma_body<DMA_PRED, false, true>(blockIdx.x - h.grid0, h.b, h.map, h.kbeg, h.kend, h.kc, h.u, h.um, h.mu,
-                                         h.la, h.rho, h.sg, h.out, h.acc, h.cof, h.cupd, h.dt2i);
+   sweep_dma_body<DMA_PRED, DW, true>(blockIdx.x - h.grid0, h.b, h.map, h.kbeg, h.kend, h.kc, h.u, h.um, h.mu, h.la,
+                                      h.rho, h.sg, h.out, h.acc, h.cof, h.cupd, h.dt2i);
 }
 
-// Batched corrector staging the acceleration its predictor stored (acc),
-// for shots that store it.
-__global__ void __launch_bounds__(NT, 2) k_sweep_dma_corr_batch(const SweepShot* __restrict__ shots, int nshots)
+template <bool DW>
+__global__ void __launch_bounds__(NT, 2) k_corr_batch(const SweepShot* __restrict__ shots, int nshots)
 {
    const SweepShot& h = shots[find_shot(shots, nshots, blockIdx.x)];
-   sweep_dma_body<DMA_CORR, false, true>(blockIdx.x - h.grid0, h.b, h.map, h.kbeg, h.kend, h.kc, h.acc, h.upin,
-                                         h.mu, h.la, h.rho, h.sg, h.out, nullptr, h.cof, h.cupd, h.dt2i);
+   sweep_dma_body<DMA_CORR, DW, true>(blockIdx.x - h.grid0, h.b, h.map, h.kbeg, h.kend, h.kc, h.acc, h.upin, h.mu,
+                                      h.la, h.rho, h.sg, h.out, nullptr, h.cof, h.cupd, h.dt2i);
 }
 
 template <bool DW>
@@ -1115,25 +1106,19 @@ bool async_loads_fit(const Box& b, const double* const* arrays, int n)
    return true;
 }
 
-int launch_sweep_batch_async(int kind, const SweepShot* d_shots, int nshots, int nblocks, hipStream_t s)
+int launch_sweep_batch(int kind, bool wide, const SweepShot* d_shots, int nshots, int nblocks, hipStream_t s)
 {
    if (nblocks <= 0) return OK;
-   if (kind == 0)
-      k_sweep_dma_batch<<<nblocks, NT, 0, s>>>(d_shots, nshots);
+   if (kind == 0 && wide)
+      k_pred_batch<false><<<nblocks, NT, 0, s>>>(d_shots, nshots);
+   else if (kind == 0)
+      k_pred_batch<true><<<nblocks, NT, 0, s>>>(d_shots, nshots);
+   else if (kind == 1 && wide)
+      k_corr_batch<false><<<nblocks, NT, 0, s>>>(d_shots, nshots);
    else if (kind == 1)
-      k_sweep_dma_corr_batch<<<nblocks, NT, 0, s>>>(d_shots, nshots);
-   else
+      k_corr_batch<true><<<nblocks, NT, 0, s>>>(d_shots, nshots);
+   else if (wide)
       k_damp_batch<false><<<nblocks, NT, 0, s>>>(d_shots, nshots);
-   return check_hip(hipGetLastError(), "batched asynchronous-load sweep launch");
-}
-
-int launch_sweep_batch(int kind, const SweepShot* d_shots, int nshots, int nblocks, hipStream_t s)
-{
-   if (nblocks <= 0) return OK;
-   if (kind == 0)
-      k_sweep_batch<false><<<nblocks, NT, 0, s>>>(d_shots, nshots);
-   else if (kind == 1)
-      k_sweep_batch<true><<<nblocks, NT, 0, s>>>(d_shots, nshots);
    else
       k_damp_batch<true><<<nblocks, NT, 0, s>>>(d_shots, nshots);
    return check_hip(hipGetLastError(), "batched sweep launch");
