@@ -15,6 +15,7 @@
 #include "kernels_adj.h"
 #include "kernels_fast.h"
 #include "kernels_step.h"
+#include "sbp_rows.h"
 #include "stencil_body.h"
 
 namespace sw4amd {
@@ -36,9 +37,6 @@ RowMap make_rowmap(const Box& b, int nz, const int* onesided)
    return m;
 }
 
-// coefficient of f(a) in d4 = f(-2) - f(2) + 8 (f(1) - f(-1)), a in {-2,-1,1,2}
-__device__ __forceinline__ double cd4(int a) { return a == -2 ? 1.0 : a == -1 ? -8.0 : a == 1 ? 8.0 : -1.0; }
-
 __device__ __forceinline__ bool inbox(const Box& b, int i, int j, int k)
 {
    return i >= b.ib && i <= b.ie && j >= b.jb && j <= b.je && k >= b.kb && k <= b.ke;
@@ -46,11 +44,6 @@ __device__ __forceinline__ bool inbox(const Box& b, int i, int j, int k)
 __device__ __forceinline__ bool int_row(const RowMap& m, int i, int j, int k)
 {
    return i >= 1 && i <= m.nx && j >= 1 && j <= m.ny && k >= m.k1 && k <= m.k2;
-}
-__device__ __forceinline__ bool sbp_row(const RowMap& m, int i, int j, int k)
-{
-   return i >= 1 && i <= m.nx && j >= 1 && j <= m.ny &&
-          ((m.top && k >= 1 && k <= 6) || (m.bot && k >= m.nz - 5 && k <= m.nz));
 }
 // plane k holds rows (of either kind) on its columns 1..nx x 1..ny
 __device__ __forceinline__ bool plane_rows(const RowMap& m, int k)
@@ -67,149 +60,10 @@ struct AdjCtx {
    const double* strx;
    const double* stry;
    const double* strz;
-   __device__ __forceinline__ double vmu(int i, int j, int k) const { return inbox(b, i, j, k) ? mu[sidx(b, i, j, k)] : 0.0; }
-   __device__ __forceinline__ double vla(int i, int j, int k) const { return inbox(b, i, j, k) ? la[sidx(b, i, j, k)] : 0.0; }
    __device__ __forceinline__ double sx(int i) const { return i >= b.ib && i <= b.ie ? strx[i - b.ib] : 1.0; }
    __device__ __forceinline__ double sy(int j) const { return j >= b.jb && j <= b.je ? stry[j - b.jb] : 1.0; }
    __device__ __forceinline__ double sz(int k) const { return k >= b.kb && k <= b.ke ? strz[k - b.kb] : 1.0; }
-   // a component-blocked field, 0 outside the box
-   __device__ __forceinline__ double f(const double* p, int c, int i, int j, int k) const
-   {
-      return inbox(b, i, j, k) ? p[sidx(b, i, j, k) + b.npts * c] : 0.0;
-   }
-   // z on the interior-formula rows / on the SBP rows, 0 elsewhere
-   __device__ __forceinline__ double zi(const double* z, int c, int i, int j, int k) const
-   {
-      return int_row(m, i, j, k) ? z[sidx(b, i, j, k) + b.npts * c] : 0.0;
-   }
-   __device__ __forceinline__ double zb(const double* z, int c, int i, int j, int k) const
-   {
-      return sbp_row(m, i, j, k) ? z[sidx(b, i, j, k) + b.npts * c] : 0.0;
-   }
 };
-
-// x and y parts of the interior formula with the xy mixed terms: the
-// in-plane part of an SBP row (rhs4sg_rev.C:353-629 before the k terms).
-template <class S>
-__device__ __forceinline__ void rhs4_xy_body(const S& s, double r[3])
-{
-   double am[5], al[5], mx[4], lx[4], my[4], ly[4];
-#pragma unroll
-   for (int q = 0; q < 5; q++) {
-      am[q] = s.mu(q - 2, 0, 0) * s.sx(q - 2);
-      al[q] = s.la(q - 2, 0, 0) * s.sx(q - 2);
-   }
-   varcoef4c(am, mx);
-   varcoef4c(al, lx);
-#pragma unroll
-   for (int q = 0; q < 5; q++) {
-      am[q] = s.mu(0, q - 2, 0) * s.sy(q - 2);
-      al[q] = s.la(0, q - 2, 0) * s.sy(q - 2);
-   }
-   varcoef4c(am, my);
-   varcoef4c(al, ly);
-   double cx[4], cy[4];
-#pragma unroll
-   for (int q = 0; q < 4; q++) {
-      cx[q] = 2 * mx[q] + lx[q];
-      cy[q] = 2 * my[q] + ly[q];
-   }
-   const double sx = s.sx(0), sy = s.sy(0);
-#pragma unroll
-   for (int c = 0; c < 3; c++) {
-      double f[5];
-#pragma unroll
-      for (int q = 0; q < 5; q++) f[q] = s.u(c, q - 2, 0, 0);
-      double acc = sx * varsum4c(c == 0 ? cx : mx, f);
-#pragma unroll
-      for (int q = 0; q < 5; q++) f[q] = s.u(c, 0, q - 2, 0);
-      acc += sy * varsum4c(c == 1 ? cy : my, f);
-      r[c] = acc * (1.0 / 6);
-   }
-   const double sxy = sx * sy * (1.0 / 144);
-   r[0] += sxy * (mixed_term<0, 1, 1, true, double>(s) + mixed_term<1, 0, 1, false, double>(s));
-   r[1] += sxy * (mixed_term<0, 1, 0, false, double>(s) + mixed_term<1, 0, 0, true, double>(s));
-}
-
-// k-direction terms of the SBP rows of one side, transposed, at the point
-// (i,j,k): row kr lives on grid plane kbase + sgn (kr-1), plane q (0..8) of
-// the row space on kbase + sgn (q-1).
-__device__ void sbp_col_T(const AdjCtx& A, const double* z, int i, int j, int k, int kbase, int sgn, double r[3])
-{
-   const int q = sgn * (k - kbase) + 1;
-   if (q < 0 || q > 8) return;
-   const SbpTables* sbp = A.sbp;
-   const double i12 = 1.0 / 12;
-   const bool col = i >= 1 && i <= A.m.nx && j >= 1 && j <= A.m.ny;
-   // mu, lambda on the side's planes m = 1..8 of this column
-   double muc[8], lac[8];
-#pragma unroll
-   for (int mm = 0; mm < 8; mm++) {
-      const int kmg = kbase + sgn * mm;
-      muc[mm] = A.vmu(i, j, kmg);
-      lac[mm] = A.vla(i, j, kmg);
-   }
-   // mu, lambda around this point in its plane (x and y taps)
-   double mxa[4], mya[4], lxa[4], lya[4];
-   const double sxa[4] = {A.sx(i + 2), A.sx(i + 1), A.sx(i - 1), A.sx(i - 2)};
-   const double sya[4] = {A.sy(j + 2), A.sy(j + 1), A.sy(j - 1), A.sy(j - 2)};
-#pragma unroll
-   for (int t = 0; t < 4; t++) {
-      const int a = t < 2 ? t - 2 : t - 1;
-      mxa[t] = A.vmu(i - a, j, k);
-      mya[t] = A.vmu(i, j - a, k);
-      lxa[t] = A.vla(i - a, j, k);
-      lya[t] = A.vla(i, j - a, k);
-   }
-#pragma unroll
-   for (int kr = 1; kr <= 6; kr++) {
-      const int krg = kbase + sgn * (kr - 1);
-      const double z0 = A.zb(z, 0, i, j, krg), z1 = A.zb(z, 1, i, j, krg), z2 = A.zb(z, 2, i, j, krg);
-      // acof / ghcof: u_c(q) enters row kr of the same column
-      double amu = 0, a2ml = 0;
-      if (q == 0) {
-         const double gh = sbp->ghcof[kr - 1];
-         amu = gh * muc[0];
-         a2ml = gh * (2 * muc[0] + lac[0]);
-      } else {
-#pragma unroll
-         for (int mm = 0; mm < 8; mm++) {
-            const double a = sbp->acof[(kr - 1) + 6 * (q - 1) + 48 * mm];
-            amu += a * muc[mm];
-            a2ml += a * (2 * muc[mm] + lac[mm]);
-         }
-      }
-      if (col) {
-         r[0] += z0 * amu;
-         r[1] += z1 * amu;
-         r[2] += z2 * a2ml;
-      }
-      if (q < 1) continue;
-      const double bq = sgn * sbp->bope[(kr - 1) + 6 * (q - 1)];
-      double s2 = 0, s0 = 0, s1 = 0;
-      const double lar = lac[kr - 1], mur = muc[kr - 1];
-#pragma unroll
-      for (int t = 0; t < 4; t++) {
-         const int a = t < 2 ? t - 2 : t - 1;
-         const double ca = cd4(a);
-         const double wx0 = sxa[t] * A.zb(z, 0, i - a, j, krg);
-         const double wy1 = sya[t] * A.zb(z, 1, i, j - a, krg);
-         const double wx2 = sxa[t] * A.zb(z, 2, i - a, j, krg);
-         const double wy2 = sya[t] * A.zb(z, 2, i, j - a, krg);
-         // (la w_z)_x, (la w_z)_y: coefficient la at this column, row plane
-         s2 += ca * lar * (wx0 + wy1);
-         // (mu w_x)_z, (mu w_y)_z: coefficient mu at the row's column, plane q
-         s2 += ca * (mxa[t] * wx0 + mya[t] * wy1);
-         // (mu u_z)_x and (la u_x)_z
-         s0 += ca * (mur * wx2 + lxa[t] * wx2);
-         // (mu v_z)_y and (la v_y)_z
-         s1 += ca * (mur * wy2 + lya[t] * wy2);
-      }
-      r[0] += bq * i12 * s0;
-      r[1] += bq * i12 * s1;
-      r[2] += bq * i12 * s2;
-   }
-}
 
 Box pad_box(const Box& b) { return make_box(b.ib - 2, b.ie + 2, b.jb - 2, b.je + 2, b.kb - 2, b.ke + 2); }
 
@@ -253,9 +107,7 @@ __global__ void k_adj_pad_material(Box b, Box pb, const double* __restrict__ mu,
    if (q < pb.ke - pb.kb + 1) szp[q] = (pb.kb + q >= b.kb && pb.kb + q <= b.ke) ? strz[pb.kb + q - b.kb] : 1.0;
 }
 
-// padded W: INPLANE = false: S zI (interior-formula rows, S = sx sy sz);
-// true: sx sy zB (SBP rows)
-template <bool INPLANE>
+// padded W = S zI (interior-formula rows, S = sx sy sz)
 __global__ void k_adj_weight(AdjCtx A, AdjPad P, const double* __restrict__ z)
 {
    const long q = blockIdx.x * (long)blockDim.x + threadIdx.x;
@@ -264,8 +116,8 @@ __global__ void k_adj_weight(AdjCtx A, AdjPad P, const double* __restrict__ z)
    const int i = pb.ib + (int)(q % pb.ni);
    const int j = pb.jb + (int)((q / pb.ni) % (pb.je - pb.jb + 1));
    const int k = pb.kb + (int)(q / pb.nij);
-   const bool row = INPLANE ? sbp_row(A.m, i, j, k) : int_row(A.m, i, j, k);
-   const double s = row ? A.sx(i) * A.sy(j) * (INPLANE ? 1.0 : A.sz(k)) : 0.0;
+   const bool row = int_row(A.m, i, j, k);
+   const double s = row ? A.sx(i) * A.sy(j) * A.sz(k) : 0.0;
    const long p = row ? sidx(A.b, i, j, k) : 0;
    for (int c = 0; c < 3; c++) {
       const double v = row ? s * z[p + A.b.npts * c] : 0.0;
@@ -286,137 +138,203 @@ __global__ void k_adj_crop(Box b, Box pb, const double* __restrict__ o, double* 
    for (int c = 0; c < 3; c++) out[p + b.npts * c] = o[q + pb.npts * c];
 }
 
-// Accessor of rhs4_xy_body over the padded arrays (no checks).
-struct PadSten {
-   const AdjPad& P;
-   int i, j, k;
-   __device__ __forceinline__ double u(int c, int di, int dj, int dk) const
-   {
-      return P.w[sidx(P.pb, i + di, j + dj, k + dk) + P.pb.npts * c];
+// The eight planes of a side over block.y where a grid's tiles leave CUs idle
+// (one workgroup on each of 256).  85 tiles: transposed rows 34.3 -> 21.6 us,
+// material derivative 32.0 -> 21.4 us against one workgroup a tile.
+inline int rows_planes_spread(int tiles) { return std::max(1, std::min(8, 256 / tiles)); }
+
+// SBP rows of one side, transposed: out on the row planes 1..6 and the planes
+// q = 0..8 (row space, rhs4sg_rev.C:353-629) of every column of the box.
+// With W = sx sy z on the rows' columns (0 off them), per row kr the in-plane
+// part is (sx sy)^{-1} Lxy(W), and the k terms of plane q are
+//   r0 = sum_kr z0 (acof mu) + i12 (sum_kr b mu_kr X2 - d4x(la_q sx B2)),
+//   r1 = sum_kr z1 (acof mu) + i12 (sum_kr b mu_kr Y2 - d4y(la_q sy B2)),
+//   r2 = sum_kr z2 (acof (2mu + la)) + i12 (sum_kr b la_kr (X0 + Y1)
+//                                           - d4x(mu_q sx B0) - d4y(mu_q sy B1)),
+// b = bope(kr, q), B_c = sum_kr b z_c, X_c = -d4x(sx z_c), Y_c = -d4y(sy z_c).
+// As in sbp_rows.h each point of a 32 x 8 tile with its halo has a thread and
+// every product is formed once and read by the neighbours: per plane the four
+// x and four y products of a point go to LDS, one barrier.  block.y takes
+// every gridDim.y-th plane (rows_planes_spread).  Against a pass
+// over the padded box for W and two kernels of a thread per point: 128 x 128
+// points 64 -> 21.6 us a side.
+__global__ void __launch_bounds__(RNT, 1)
+k_rhs4sg_T_rows(AdjCtx A, int ntx, int kbase, int sgn, const double* __restrict__ z, Box ob, double* __restrict__ out,
+                double cof)
+{
+   constexpr int FX = RHX * RTY, GY = RTX * RHY;
+   __shared__ double sw[6 * 3 * RPL];                  // W of the rows
+   __shared__ double sm[8 * RPL], sl[8 * RPL];         // mu, lambda of the planes 1..8
+   __shared__ double sf[2][4 * FX], sg[2][4 * GY];     // x and y products
+   __shared__ double ssx[RHX], ssy[RHY];
+   const Box& b = A.b;
+   const int tix = blockIdx.x % ntx, tjy = blockIdx.x / ntx, tid = threadIdx.x;
+   int role, hx, hy;
+   rows_point(tid, role, hx, hy);
+   const bool own = tid < RPL, ihalo = role == 2 && tid < 384 + 4 * RTY;
+   const int ia = b.ib - 2 + tix * RTX, ja = b.jb - 2 + tjy * RTY;
+   const int i = ia + hx, j = ja + hy;
+   const bool in = i >= b.ib && i <= b.ie && j >= b.jb && j <= b.je;
+   const bool active = role == 0 && in;
+   const bool rowcol = i >= 1 && i <= A.m.nx && j >= 1 && j <= A.m.ny;
+   const long nij = b.nij, npts = b.npts;
+   const long col = in ? (i - b.ib) + b.ni * (j - b.jb) : 0;  // a valid address where off the box
+   const double sx = A.sx(i), sy = A.sy(j);
+   const int o = hy * RHX + hx;
+   const double i12 = 1.0 / 12;
+   const SbpTables* __restrict__ sbp = A.sbp;
+   auto d4s = [](const double* f, int st) { return f[-2 * st] - f[2 * st] + 8 * (f[st] - f[-st]); };
+
+   double zr[6][3], m[8], l[8];
+#pragma unroll
+   for (int q = 0; q < 8; q++) {
+      const long p = col + nij * (kbase + sgn * q - b.kb);
+      const double vm = A.mu[p], vl = A.la[p];
+      m[q] = in ? vm : 0.0;
+      l[q] = in ? vl : 0.0;
+      if (q < 6) {
+#pragma unroll
+         for (int c = 0; c < 3; c++) {
+            const double v = z[p + npts * c];
+            zr[q][c] = rowcol ? v : 0.0;
+            if (own) sw[(q * 3 + c) * RPL + o] = sx * sy * zr[q][c];
+         }
+      }
+      if (own) {
+         sm[q * RPL + o] = m[q];
+         sl[q * RPL + o] = l[q];
+      }
    }
-   __device__ __forceinline__ double mu(int di, int dj, int dk) const { return P.mu[sidx(P.pb, i + di, j + dj, k + dk)]; }
-   __device__ __forceinline__ double la(int di, int dj, int dk) const { return P.la[sidx(P.pb, i + di, j + dj, k + dk)]; }
-   __device__ __forceinline__ double sx(int d) const { return P.sx[i + d - P.pb.ib]; }
-   __device__ __forceinline__ double sy(int d) const { return P.sy[j + d - P.pb.jb]; }
-   __device__ __forceinline__ double sz(int d) const { return P.sz[k + d - P.pb.kb]; }
-};
-
-// SBP rows, in-plane part on the row planes of one side: out += cof
-// (sx sy)^{-1} Lxy(W), W = sx sy zB
-__global__ void __launch_bounds__(256) k_rhs4sg_T_xy(AdjCtx A, AdjPad P, int kbase, int sgn, Box ob,
-                                                     double* __restrict__ out, double cof)
-{
-   const Box& b = A.b;
-   const int i = b.ib + blockIdx.x * blockDim.x + threadIdx.x;
-   const int j = b.jb + blockIdx.y * blockDim.y + threadIdx.y;
-   const int k = kbase + sgn * (int)blockIdx.z;  // rows 1..6
-   if (i > b.ie || j > b.je) return;
-   const PadSten s{P, i, j, k};
-   double r[3];
-   rhs4_xy_body(s, r);
-   const double sc = cof / (A.sx(i) * A.sy(j));
-   const long p = sidx(ob, i, j, k);
-   for (int c = 0; c < 3; c++) out[p + ob.npts * c] += sc * r[c];
-}
-
-// SBP rows, k-direction terms on the planes 0..8 of one side
-__global__ void __launch_bounds__(256) k_rhs4sg_T_col(AdjCtx A, int kbase, int sgn, const double* __restrict__ z,
-                                                      Box ob, double* __restrict__ out, double cof)
-{
-   const Box& b = A.b;
-   const int i = b.ib + blockIdx.x * blockDim.x + threadIdx.x;
-   const int j = b.jb + blockIdx.y * blockDim.y + threadIdx.y;
-   const int k = kbase + sgn * ((int)blockIdx.z - 1);  // planes q = 0..8
-   if (i > b.ie || j > b.je || k < b.kb || k > b.ke) return;
-   double r[3] = {0, 0, 0};
-   sbp_col_T(A, z, i, j, k, kbase, sgn, r);
-   const long p = sidx(ob, i, j, k);
-   for (int c = 0; c < 3; c++) out[p + ob.npts * c] += cof * r[c];
+   if (tid < RHX) ssx[tid] = A.sx(ia + tid);
+   if (tid >= 64 && tid < 64 + RHY) ssy[tid - 64] = A.sy(ja + tid - 64);
+   __syncthreads();
+   // of the rows: mu X2, mu Y2, la (X0 + Y1)
+   double P[6][3];
+   if (role == 0) {
+      const double isx = 1 / sx, isy = 1 / sy;
+#pragma unroll
+      for (int q = 0; q < 6; q++) {
+         const double* f = sw + q * 3 * RPL + o;
+         P[q][0] = -m[q] * isy * d4s(f + 2 * RPL, 1);
+         P[q][1] = -m[q] * isx * d4s(f + 2 * RPL, RHX);
+         P[q][2] = -l[q] * (isy * d4s(f, 1) + isx * d4s(f + RPL, RHX));
+      }
+   }
+   if (active && blockIdx.y == gridDim.y - 1 && kbase - sgn >= b.kb && kbase - sgn <= b.ke) {  // the ghost plane, q = 0
+      double r[3] = {0, 0, 0};
+#pragma unroll
+      for (int kr = 0; kr < 6; kr++) {
+         const double g = sbp->ghcof[kr];
+         r[0] += zr[kr][0] * (g * m[0]);
+         r[1] += zr[kr][1] * (g * m[0]);
+         r[2] += zr[kr][2] * (g * (2 * m[0] + l[0]));
+      }
+      const long p = sidx(ob, i, j, kbase - sgn);
+#pragma unroll
+      for (int c = 0; c < 3; c++) out[p + ob.npts * c] += cof * r[c];
+   }
+   int par = 0;
+#pragma unroll 1
+   for (int q = 1 + (int)blockIdx.y; q <= 8; q += (int)gridDim.y) {
+      const double* f = sw + (q - 1) * 3 * RPL + o;  // the row on this plane (q = 1..6)
+      const double mq = sm[(q - 1) * RPL + o], lq = sl[(q - 1) * RPL + o];
+      const long p = sidx(ob, in ? i : b.ib, in ? j : b.jb, kbase + sgn * (q - 1));
+      double r[3] = {0, 0, 0}, old[3];
+#pragma unroll
+      for (int c = 0; c < 3; c++) old[c] = role == 0 ? out[p + ob.npts * c] : 0.0;
+      double B[3] = {0, 0, 0};
+#pragma unroll
+      for (int kr = 0; kr < 6; kr++) {
+         const double bq = sgn * sbp->bope[kr + 6 * (q - 1)];
+#pragma unroll
+         for (int c = 0; c < 3; c++) {
+            B[c] += bq * zr[kr][c];
+            if (role == 0) r[c] += bq * i12 * P[kr][c];
+         }
+      }
+      if (role == 0 || ihalo) {
+         double* w = &sf[par][(hy - 2) * RHX + hx];
+         w[0] = mq * (sx * B[0]);
+         w[FX] = lq * (sx * B[2]);
+         if (q <= 6) {
+            w[2 * FX] = lq * d4s(f + RPL, RHX);
+            w[3 * FX] = mq * d4s(f, RHX);
+         }
+      }
+      if (role != 2) {
+         double* w = &sg[par][hy * RTX + hx - 2];
+         w[0] = mq * (sy * B[1]);
+         w[GY] = lq * (sy * B[2]);
+         if (q <= 6) {
+            w[2 * GY] = mq * d4s(f + RPL, 1);
+            w[3 * GY] = lq * d4s(f, 1);
+         }
+      }
+      if (role == 0) {
+#pragma unroll
+         for (int kr = 0; kr < 6; kr++) {
+            double am = 0, ak = 0;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+               const double a = sbp->acof[kr + 6 * (q - 1) + 48 * e];
+               am += a * m[e];
+               ak += a * (2 * m[e] + l[e]);
+            }
+            r[0] += zr[kr][0] * am;
+            r[1] += zr[kr][1] * am;
+            r[2] += zr[kr][2] * ak;
+         }
+      }
+      __syncthreads();  // the products of plane q; the other half's were read before the last barrier
+      if (active) {
+         const double* wf = &sf[par][(hy - 2) * RHX + hx];
+         const double* wg = &sg[par][hy * RTX + hx - 2];
+         r[0] -= i12 * d4s(wf + FX, 1);
+         r[1] -= i12 * d4s(wg + GY, RTX);
+         r[2] -= i12 * (d4s(wf, 1) + d4s(wg, RTX));
+         if (q <= 6) {  // the row's in-plane part
+            double am[5], al[5], mx[4], my[4], cx[4], cy[4];
+            const double *pm = sm + (q - 1) * RPL + o, *pl = sl + (q - 1) * RPL + o;
+#pragma unroll
+            for (int t = 0; t < 5; t++) {
+               am[t] = pm[t - 2] * ssx[hx + t - 2];
+               al[t] = pl[t - 2] * ssx[hx + t - 2];
+            }
+            varcoef4c(am, mx);
+            varcoef4c(al, cx);
+#pragma unroll
+            for (int t = 0; t < 5; t++) {
+               am[t] = pm[(t - 2) * RHX] * ssy[hy + t - 2];
+               al[t] = pl[(t - 2) * RHX] * ssy[hy + t - 2];
+            }
+            varcoef4c(am, my);
+            varcoef4c(al, cy);
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+               cx[t] += 2 * mx[t];
+               cy[t] += 2 * my[t];
+            }
+            const double isxy = 1 / (sx * sy);
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+               const double* g = f + c * RPL;
+               const double x[5] = {g[-2], g[-1], g[0], g[1], g[2]};
+               const double y[5] = {g[-2 * RHX], g[-RHX], g[0], g[RHX], g[2 * RHX]};
+               r[c] += isxy * ((1.0 / 6) * (sx * varsum4c(c == 0 ? cx : mx, x) + sy * varsum4c(c == 1 ? cy : my, y)));
+            }
+            r[0] += (1.0 / 144) * (d4s(wf + 2 * FX, 1) + d4s(wg + 2 * GY, RTX));
+            r[1] += (1.0 / 144) * (d4s(wf + 3 * FX, 1) + d4s(wg + 3 * GY, RTX));
+         }
+#pragma unroll
+         for (int c = 0; c < 3; c++) out[p + ob.npts * c] = old[c] + cof * r[c];
+      }
+      par ^= 1;
+   }
 }
 
 // ---------------------------------------------------------------------------
 // Material derivatives
 // ---------------------------------------------------------------------------
-// acof / ghcof / bope terms of the SBP rows of one side at p
-__device__ void sbp_col_grad(const AdjCtx& A, const double* z, const double* u, int i, int j, int k, int kbase,
-                             int sgn, double& gm, double& gl)
-{
-   const int q = sgn * (k - kbase) + 1;
-   if (q < 1 || q > 8) return;
-   const SbpTables* sbp = A.sbp;
-   const double i12 = 1.0 / 12;
-   const bool col = i >= 1 && i <= A.m.nx && j >= 1 && j <= A.m.ny;
-   // u on the side's planes 1..8 of this column, and on its ghost plane
-   double uk[8][3], ug[3];
-#pragma unroll
-   for (int qq = 0; qq < 8; qq++) {
-      const int kq = kbase + sgn * qq;
-#pragma unroll
-      for (int c = 0; c < 3; c++) uk[qq][c] = A.f(u, c, i, j, kq);
-   }
-#pragma unroll
-   for (int c = 0; c < 3; c++) ug[c] = A.f(u, c, i, j, kbase - sgn);
-   // x and y differences of u in this point's plane
-   double dx2 = 0, dy2 = 0, dx0 = 0, dy1 = 0;
-#pragma unroll
-   for (int t = 0; t < 4; t++) {
-      const int a = t < 2 ? t - 2 : t - 1;
-      dx2 += cd4(a) * A.f(u, 2, i + a, j, k);
-      dy2 += cd4(a) * A.f(u, 2, i, j + a, k);
-      dx0 += cd4(a) * A.f(u, 0, i + a, j, k);
-      dy1 += cd4(a) * A.f(u, 1, i, j + a, k);
-   }
-   const double sxi = A.sx(i), syj = A.sy(j);
-#pragma unroll
-   for (int kr = 1; kr <= 6; kr++) {
-      const int krg = kbase + sgn * (kr - 1);
-      const double z0 = A.zb(z, 0, i, j, krg), z1 = A.zb(z, 1, i, j, krg), z2 = A.zb(z, 2, i, j, krg);
-      if (col) {
-         // mu, la at plane m = q enter row kr through acof(kr, q', q) u(q')
-         double sm = 0, sl = 0;
-#pragma unroll
-         for (int qq = 0; qq < 8; qq++) {
-            const double a = sbp->acof[(kr - 1) + 6 * qq + 48 * (q - 1)];
-            sm += a * (z0 * uk[qq][0] + z1 * uk[qq][1] + 2 * z2 * uk[qq][2]);
-            sl += a * z2 * uk[qq][2];
-         }
-         if (q == 1) {  // ghost term gh mu(1) u(0)
-            const double gh = sbp->ghcof[kr - 1];
-            sm += gh * (z0 * ug[0] + z1 * ug[1] + 2 * z2 * ug[2]);
-            sl += gh * z2 * ug[2];
-         }
-         gm += sm;
-         gl += sl;
-      }
-      // (mu w_x)_z, (mu w_y)_z, (la u_x)_z, (la v_y)_z: coefficient at (i,j) plane q, row (i,j,kr)
-      const double bq = sgn * sbp->bope[(kr - 1) + 6 * (q - 1)];
-      gm += bq * i12 * (sxi * dx2 * z0 + syj * dy2 * z1);
-      gl += bq * i12 * (sxi * dx0 + syj * dy1) * z2;
-   }
-   // (la w_z)_x, (la w_z)_y, (mu u_z)_x, (mu v_z)_y: coefficient at p on row plane kr = q
-   if (q <= 6) {
-      double bu0 = 0, bu1 = 0, bu2 = 0;
-#pragma unroll
-      for (int qq = 0; qq < 8; qq++) {
-         const double bq = sgn * sbp->bope[(q - 1) + 6 * qq];
-         bu0 += bq * uk[qq][0];
-         bu1 += bq * uk[qq][1];
-         bu2 += bq * uk[qq][2];
-      }
-      double wx0 = 0, wy1 = 0, wx2 = 0, wy2 = 0;
-#pragma unroll
-      for (int t = 0; t < 4; t++) {
-         const int a = t < 2 ? t - 2 : t - 1;
-         wx0 += cd4(a) * A.sx(i - a) * A.zb(z, 0, i - a, j, k);
-         wy1 += cd4(a) * A.sy(j - a) * A.zb(z, 1, i, j - a, k);
-         wx2 += cd4(a) * A.sx(i - a) * A.zb(z, 2, i - a, j, k);
-         wy2 += cd4(a) * A.sy(j - a) * A.zb(z, 2, i, j - a, k);
-      }
-      gl += i12 * bu2 * (wx0 + wy1);
-      gm += i12 * (bu0 * wx2 + bu1 * wy2);
-   }
-}
-
 // Interior-row terms of G_mu, G_la at every point p of the box (ghosts
 // included), marching along k.  A workgroup owns a 32 x 8 tile of (i,j)
 // columns.  Plane k of u (0 off the box) and of z (0 off the interior-formula
@@ -433,7 +351,7 @@ __device__ void sbp_col_grad(const AdjCtx& A, const double* z, const double* u, 
 // terms (coef D_a u_b)_d are D[a][b] = d4 of u_b along a at p times
 // V[r][d] = d4 of s_d z_r along d, taken with its sign reversed, at p.
 namespace {
-constexpr int GTX = 32, GTY = 8, GNT = GTX * GTY;
+constexpr int GTX = RTX, GTY = RTY, GNT = GTX * GTY;
 constexpr int GHX = GTX + 4, GHY = GTY + 4, GPL = GHX * GHY;  // plane with a halo of 2
 constexpr int GSL = (GPL + GNT - 1) / GNT;                      // staging slots per thread
 }  // namespace
@@ -448,7 +366,7 @@ __device__ __forceinline__ double second_form(const double w[5], const double y[
    const double k4 = y[3] - 0.75 * y[2] - 0.25 * y[4];
    return w[0] * k0 + w[1] * k1 + w[2] * k2 + w[3] * k3 + w[4] * k4;
 }
-// d4 at e = 0: sum_a cd4(a) f(a), and the same of f(-a)
+// d4 = f(-2) - f(2) + 8 (f(1) - f(-1)) at e = 0, and the same of f(-e)
 __device__ __forceinline__ double d4w(const double f[5]) { return f[0] - f[4] + 8 * (f[3] - f[1]); }
 __device__ __forceinline__ double d4r(const double f[5]) { return f[4] - f[0] + 8 * (f[1] - f[3]); }
 
@@ -600,7 +518,7 @@ __global__ void __launch_bounds__(GNT, 2) k_rhs4sg_matgrad_march(AdjCtx A, int n
             if (c == 2) gd += S;
          }
          // on an SBP row plane only the in-plane terms belong to the rows
-         // (their k terms are the acof/bope stencils of k_rhs4sg_matgrad_sbp)
+         // (their k terms are the acof/bope stencils of k_rhs4sg_matgrad_rows)
          const double fi = k >= m.k1 && k <= m.k2 ? 1.0 : 0.0;
          const double s0 = sxo[2], s1 = syo[2], s2 = szr[2], s2i = fi * s2;
          const double ml = V[0][0] * (s1 * D[1][1] + s2i * D[2][2]) + V[1][1] * (s0 * D[0][0] + s2i * D[2][2]) +
@@ -625,22 +543,111 @@ __global__ void __launch_bounds__(GNT, 2) k_rhs4sg_matgrad_march(AdjCtx A, int n
    }
 }
 
-// SBP rows of one side on its planes 0..8: in-plane part (row planes) and
-// the k-direction terms
-__global__ void __launch_bounds__(256) k_rhs4sg_matgrad_sbp(AdjCtx A, int kbase, int sgn, const double* __restrict__ z,
-                                                            const double* __restrict__ u, double* __restrict__ gmu,
-                                                            double* __restrict__ gla, double cof)
+// SBP rows of one side, k-direction terms, at the planes q = 1..8 of every
+// column of the box: with A_c = sum_q' acof(kr, q', q) u_c(q') (and the ghost
+// term of q = 1), B_c = sum_kr b z_c and b = bope,
+//   gmu += sum_kr (z0 A0 + z1 A1 + 2 z2 A2) + i12 (d4x u2 B0 + d4y u2 B1)
+//          - i12 (bu0 d4x(sx z2) + bu1 d4y(sy z2)),
+//   gla += sum_kr z2 A2 + i12 (d4x u0 + d4y u1) B2
+//          - i12 bu2 (d4x(sx z0) + d4y(sy z1)),
+// the second lines on the row planes q = 1..6, bu_c = sum_q' bope(q, q') u_c.
+// A thread keeps its column of u and z in registers and reads the in-plane
+// taps from LDS (one barrier), where a thread per point loaded the column
+// again on each of eight planes; block.y takes every gridDim.y-th plane
+// (rows_planes_spread).  128 x 128 points 22 -> 14.0 us a side (all eight
+// planes in one workgroup 32: a tile's loads are what it waits for).
+__global__ void __launch_bounds__(RNT, 1)
+k_rhs4sg_matgrad_rows(AdjCtx A, int ntx, int kbase, int sgn, const double* __restrict__ z, const double* __restrict__ u,
+                      double* __restrict__ gmu, double* __restrict__ gla, double cof)
 {
+   __shared__ double su[8 * 3 * RPL];  // u on the planes
+   __shared__ double sz[6 * 3 * RPL];  // sx sy z of the rows
    const Box& b = A.b;
-   const int i = b.ib + blockIdx.x * blockDim.x + threadIdx.x;
-   const int j = b.jb + blockIdx.y * blockDim.y + threadIdx.y;
-   const int k = kbase + sgn * (int)blockIdx.z;  // planes 1..8 of the side
-   if (i > b.ie || j > b.je || k < b.kb || k > b.ke) return;
-   double gm = 0, gl = 0;
-   sbp_col_grad(A, z, u, i, j, k, kbase, sgn, gm, gl);
-   const long p = sidx(b, i, j, k);
-   gmu[p] += cof * gm;
-   gla[p] += cof * gl;
+   const int tix = blockIdx.x % ntx, tjy = blockIdx.x / ntx, tid = threadIdx.x;
+   int role, hx, hy;
+   rows_point(tid, role, hx, hy);
+   const bool own = tid < RPL;
+   const int i = b.ib - 2 + tix * RTX + hx, j = b.jb - 2 + tjy * RTY + hy;
+   const bool in = i >= b.ib && i <= b.ie && j >= b.jb && j <= b.je;
+   const bool rowcol = i >= 1 && i <= A.m.nx && j >= 1 && j <= A.m.ny;
+   const long nij = b.nij, npts = b.npts;
+   const long col = in ? (i - b.ib) + b.ni * (j - b.jb) : 0;  // a valid address where off the box
+   const double sx = A.sx(i), sy = A.sy(j);
+   const int o = hy * RHX + hx;
+   const double i12 = 1.0 / 12;
+   const SbpTables* __restrict__ sbp = A.sbp;
+   auto d4s = [](const double* f, int st) { return f[-2 * st] - f[2 * st] + 8 * (f[st] - f[-st]); };
+
+   double uk[8][3], ug[3], zr[6][3];
+   auto mine = [&](int q) { return q % (int)gridDim.y == (int)blockIdx.y; };  // this workgroup's planes
+#pragma unroll
+   for (int q = 0; q < 8; q++) {
+      const long p = col + nij * (kbase + sgn * q - b.kb);
+      if (role == 0 || mine(q)) {  // the halo is read on those alone
+#pragma unroll
+         for (int c = 0; c < 3; c++) {
+            const double v = u[p + npts * c];
+            uk[q][c] = in ? v : 0.0;
+            if (q < 6) {
+               const double w = z[p + npts * c];
+               zr[q][c] = rowcol ? w : 0.0;
+            }
+         }
+      }
+   }
+#pragma unroll
+   for (int q = 0; q < 8; q++) {
+      if (own && mine(q)) {
+#pragma unroll
+         for (int c = 0; c < 3; c++) {
+            su[(q * 3 + c) * RPL + o] = uk[q][c];
+            if (q < 6) sz[(q * 3 + c) * RPL + o] = sx * sy * zr[q][c];
+         }
+      }
+   }
+#pragma unroll
+   for (int c = 0; c < 3; c++) ug[c] = u[col + nij * (kbase - sgn - b.kb) + npts * c];
+   __syncthreads();
+   if (role != 0 || !in) return;
+   const double isx = 1 / sx, isy = 1 / sy;
+#pragma unroll 1
+   for (int q = (int)blockIdx.y; q < 8; q += (int)gridDim.y) {
+      const double* f = su + q * 3 * RPL + o;
+      const long p = col + nij * (kbase + sgn * q - b.kb);
+      const double gm0 = gmu[p], gl0 = gla[p];
+      double gm = 0, gl = 0, B[3] = {0, 0, 0};
+#pragma unroll
+      for (int kr = 0; kr < 6; kr++) {
+         const double bq = sgn * sbp->bope[kr + 6 * q];
+         double a[3];
+#pragma unroll
+         for (int c = 0; c < 3; c++) {
+            a[c] = q == 0 ? sbp->ghcof[kr] * ug[c] : 0.0;
+#pragma unroll
+            for (int e = 0; e < 8; e++) a[c] += sbp->acof[kr + 6 * e + 48 * q] * uk[e][c];
+            B[c] += bq * zr[kr][c];
+         }
+         const double t = zr[kr][2] * a[2];
+         gm += zr[kr][0] * a[0] + zr[kr][1] * a[1] + 2 * t;
+         gl += t;
+      }
+      gm += i12 * (sx * d4s(f + 2 * RPL, 1) * B[0] + sy * d4s(f + 2 * RPL, RHX) * B[1]);
+      gl += i12 * (sx * d4s(f, 1) + sy * d4s(f + RPL, RHX)) * B[2];
+      if (q < 6) {
+         const double* w = sz + q * 3 * RPL + o;
+         double bu[3] = {0, 0, 0};
+#pragma unroll
+         for (int e = 0; e < 8; e++) {
+            const double bq = sgn * sbp->bope[q + 6 * e];
+#pragma unroll
+            for (int c = 0; c < 3; c++) bu[c] += bq * uk[e][c];
+         }
+         gm -= i12 * (bu[0] * isy * d4s(w + 2 * RPL, 1) + bu[1] * isx * d4s(w + 2 * RPL, RHX));
+         gl -= i12 * bu[2] * (isy * d4s(w, 1) + isx * d4s(w + RPL, RHX));
+      }
+      gmu[p] = gm0 + cof * gm;
+      gla[p] = gl0 + cof * gl;
+   }
 }
 
 // ---------------------------------------------------------------------------
@@ -892,11 +899,23 @@ struct WinT {
    int i0, i1, j0, j1, k0, k1;
 };
 
-__global__ void k_bc_zero_T(Box b, WinT w, double* __restrict__ y)
+// Sides with zero data that follow each other, in one launch: thread q of the
+// windows laid end to end (off[s] is where window s begins).
+struct WinListT {
+   WinT w[6];
+   long off[7];
+   int n;
+};
+
+__global__ void k_bc_zero_T(Box b, WinListT l, double* __restrict__ y)
 {
-   const long wi = w.i1 - w.i0 + 1, wj = w.j1 - w.j0 + 1, wk = w.k1 - w.k0 + 1;
-   const long q = blockIdx.x * (long)blockDim.x + threadIdx.x;
-   if (q >= wi * wj * wk) return;
+   long q = blockIdx.x * (long)blockDim.x + threadIdx.x;
+   if (q >= l.off[l.n]) return;
+   int s = 0;
+   while (s + 1 < l.n && q >= l.off[s + 1]) s++;
+   const WinT w = l.w[s];
+   q -= l.off[s];
+   const long wi = w.i1 - w.i0 + 1, wj = w.j1 - w.j0 + 1;
    const int i = w.i0 + (int)(q % wi);
    const int j = w.j0 + (int)((q / wi) % wj);
    const int k = w.k0 + (int)(q / (wi * wj));
@@ -921,61 +940,89 @@ __global__ void k_freesurf_take(Box b, int k, int kl, double* __restrict__ y, do
 
 // phase 2: gather into the points the closure reads (freesurf_point,
 // ew-cfromfort.C:683-742) and the derivatives of g2 in mu, la at plane k.
-__global__ void k_freesurf_push(Box b, int k, int kl, double h, const SbpTables* __restrict__ sbp,
+// One plane of columns leaves the device nearly idle, so a thread's time is
+// the chain of its loads: all are issued first, off the closure's columns
+// from a clamped address, and nothing is loaded behind a test of a loaded
+// value (128 x 128 points: 14 -> 9.5 us).
+__global__ void __launch_bounds__(256)
+k_freesurf_push(Box b, int k, int kl, const SbpTables* __restrict__ sbp,
                                 const double* __restrict__ plane, const double* __restrict__ fwd,
                                 const double* __restrict__ mu, const double* __restrict__ la,
                                 const double* __restrict__ strx, const double* __restrict__ stry,
                                 double* __restrict__ y, double* __restrict__ gmu, double* __restrict__ gla)
 {
-   (void)h;
    const int i = b.ib + blockIdx.x * blockDim.x + threadIdx.x;
    const int j = b.jb + blockIdx.y * blockDim.y + threadIdx.y;
    if (i > b.ie || j > b.je) return;
    const long nij = b.nij;
    const double* sbop = sbp->sbop;
    const double d4a = 2.0 / 3.0, d4b = -1.0 / 12.0;
+   auto on = [&](int ii, int jj) { return ii >= b.ib + 2 && ii <= b.ie - 2 && jj >= b.jb + 2 && jj <= b.je - 2; };
+   auto at = [&](int ii, int jj) {  // clamped in-plane offset
+      return (min(max(ii, b.ib), b.ie) - b.ib) + b.ni * (long)(min(max(jj, b.jb), b.je) - b.jb);
+   };
    auto G = [&](int c, int ii, int jj) {  // ghost adjoint at column (ii,jj), 0 off the closure's columns
-      if (ii < b.ib + 2 || ii > b.ie - 2 || jj < b.jb + 2 || jj > b.je - 2) return 0.0;
-      return plane[(ii - b.ib) + b.ni * (jj - b.jb) + nij * c];
+      const double v = plane[at(ii, jj) + nij * c];
+      return on(ii, jj) ? v : 0.0;
    };
-   auto K = [&](int ii, int jj) {  // d g2 / d ux = -kl la / (2 mu + la) / sbop0
-      if (ii < b.ib + 2 || ii > b.ie - 2 || jj < b.jb + 2 || jj > b.je - 2) return 0.0;
-      const long pp = sidx(b, ii, jj, k);
-      return -kl * la[pp] / (2 * mu[pp] + la[pp]) / sbop[0];
-   };
-   // column terms: g_c = -sum_m sbop[m] u_c(k + kl (m-1)) / sbop0 + ...
-   for (int c = 0; c < 3; c++) {
-      const double gc = G(c, i, j);
-      if (gc != 0.0)
-         for (int m = 1; m <= 4; m++) y[vidx<1>(b, c, i, j, k + kl * (m - 1))] -= sbop[m] / sbop[0] * gc;
-   }
-   // in-plane first differences at plane k
-   double a0 = 0, a1 = 0, a2 = 0;
+   const long pk = nij * (k - b.kb), q = at(i, j);
    const int off[4] = {-2, -1, 1, 2};
-   const double cp[4] = {-d4b, -d4a, d4a, d4b};  // coefficient of u(i+off) in d4a(u+1 - u-1) + d4b(u+2 - u-2)
-   for (int t = 0; t < 4; t++) {
-      const int d = off[t];
-      const int ir = i - d, jr = j - d;  // closure columns that read (i,j) at offset d
-      const double sxr = ir >= b.ib && ir <= b.ie ? strx[ir - b.ib] : 1.0;
-      const double syr = jr >= b.jb && jr <= b.je ? stry[jr - b.jb] : 1.0;
-      a2 += -kl / sbop[0] * cp[t] * (G(0, ir, j) * sxr + G(1, i, jr) * syr);
-      a0 += K(ir, j) * G(2, ir, j) * sxr * cp[t];
-      a1 += K(i, jr) * G(2, i, jr) * syr * cp[t];
+   double yv[3][4], gx[4][2], gy[4][2], mx[4], lx[4], my[4], ly[4], fx[4], fy[4], sxr[4], syr[4], gc[3];
+#pragma unroll
+   for (int c = 0; c < 3; c++) {
+      gc[c] = G(c, i, j);
+#pragma unroll
+      for (int m = 0; m < 4; m++) yv[c][m] = y[vidx<1>(b, c, i, j, k + kl * m)];
    }
-   y[vidx<1>(b, 0, i, j, k)] += a0;
-   y[vidx<1>(b, 1, i, j, k)] += a1;
-   y[vidx<1>(b, 2, i, j, k)] += a2;
+#pragma unroll
+   for (int t = 0; t < 4; t++) {
+      const int ir = i - off[t], jr = j - off[t];  // closure columns that read (i,j) at this offset
+      gx[t][0] = G(0, ir, j);
+      gx[t][1] = G(2, ir, j);
+      gy[t][0] = G(1, i, jr);
+      gy[t][1] = G(2, i, jr);
+      mx[t] = mu[pk + at(ir, j)];
+      lx[t] = la[pk + at(ir, j)];
+      my[t] = mu[pk + at(i, jr)];
+      ly[t] = la[pk + at(i, jr)];
+      fx[t] = fwd[pk + at(i + off[t], j)];
+      fy[t] = fwd[pk + at(i, j + off[t]) + b.npts];
+      sxr[t] = strx[min(max(ir, b.ib), b.ie) - b.ib];
+      syr[t] = stry[min(max(jr, b.jb), b.je) - b.jb];
+   }
+   const double m0 = mu[pk + q], l0 = la[pk + q], gm = gmu[pk + q], gl = gla[pk + q];
+   const double sx = strx[i - b.ib], sy = stry[j - b.jb];
+   // column terms: g_c = -sum_m sbop[m] u_c(k + kl (m-1)) / sbop0 + ...
+#pragma unroll
+   for (int c = 0; c < 3; c++)
+#pragma unroll
+      for (int m = 0; m < 4; m++) yv[c][m] -= sbop[m + 1] / sbop[0] * gc[c];
+   // in-plane first differences at plane k; d g2 / d ux = -kl la / (2 mu + la) / sbop0
+   double a0 = 0, a1 = 0, a2 = 0;
+   const double cp[4] = {-d4b, -d4a, d4a, d4b};  // coefficient of u(i+off) in d4a(u+1 - u-1) + d4b(u+2 - u-2)
+#pragma unroll
+   for (int t = 0; t < 4; t++) {
+      const double kx = on(i - off[t], j) ? -kl * lx[t] / (2 * mx[t] + lx[t]) / sbop[0] : 0.0;
+      const double ky = on(i, j - off[t]) ? -kl * ly[t] / (2 * my[t] + ly[t]) / sbop[0] : 0.0;
+      a2 += -kl / sbop[0] * cp[t] * (gx[t][0] * sxr[t] + gy[t][0] * syr[t]);
+      a0 += kx * gx[t][1] * sxr[t] * cp[t];
+      a1 += ky * gy[t][1] * syr[t] * cp[t];
+   }
+   yv[0][0] += a0;
+   yv[1][0] += a1;
+   yv[2][0] += a2;
+#pragma unroll
+   for (int c = 0; c < 3; c++)
+#pragma unroll
+      for (int m = 0; m < 4; m++) y[vidx<1>(b, c, i, j, k + kl * m)] = yv[c][m];
    // mu, la derivatives of g2 = (-dz2 - kl la (ux + vy) / (2 mu + la)) / sbop0
-   const double g2 = G(2, i, j);
+   const double g2 = gc[2];
    if (g2 != 0.0) {
-      auto U = [&](int c, int ii, int jj) { return fwd[vidx<1>(b, c, ii, jj, k)]; };
-      const double sx = strx[i - b.ib], sy = stry[j - b.jb];
-      const double ux = sx * (d4a * (U(0, i + 1, j) - U(0, i - 1, j)) + d4b * (U(0, i + 2, j) - U(0, i - 2, j)));
-      const double vy = sy * (d4a * (U(1, i, j + 1) - U(1, i, j - 1)) + d4b * (U(1, i, j + 2) - U(1, i, j - 2)));
-      const long pp = sidx(b, i, j, k);
-      const double m0 = mu[pp], l0 = la[pp], den = 2 * m0 + l0, S = ux + vy;
-      gmu[pp] += g2 * kl * l0 * S * 2 / (den * den) / sbop[0];
-      gla[pp] += -g2 * kl * S * 2 * m0 / (den * den) / sbop[0];
+      const double ux = sx * (d4a * (fx[2] - fx[1]) + d4b * (fx[3] - fx[0]));
+      const double vy = sy * (d4a * (fy[2] - fy[1]) + d4b * (fy[3] - fy[0]));
+      const double den = 2 * m0 + l0, S = ux + vy;
+      gmu[pk + q] = gm + g2 * kl * l0 * S * 2 / (den * den) / sbop[0];
+      gla[pk + q] = gl - g2 * kl * S * 2 * m0 / (den * den) / sbop[0];
    }
 }
 
@@ -1107,12 +1154,10 @@ int launch_rhs4sg_T(const Box& b, const RowMap& m, const SbpTables* d_sbp, const
 {
    const AdjCtx A{b, m, d_sbp, mu, la, strx, stry, strz};
    const double cof = 1.0 / (h * h);
-   const dim3 blk(64, 4, 1);
-   const unsigned gi = cdiv(b.ni, 64), gj = cdiv(b.je - b.jb + 1, 4);
    // interior rows: S^{-1} L(S zI) on every point of the box, by the LDS
    // predictor sweep over the padded box in its transposed mode (cof L(W)/S;
    // W, mu and lambda vanish in the pad, the stretching is 1 there)
-   if (!weighted) k_adj_weight<false><<<cdiv(P.pb.npts, 256), 256, 0, s>>>(A, P, z);
+   if (!weighted) k_adj_weight<<<cdiv(P.pb.npts, 256), 256, 0, s>>>(A, P, z);
    SgCoef sg{};
    sg.strx = P.sx;
    sg.stry = P.sy;
@@ -1126,14 +1171,10 @@ int launch_rhs4sg_T(const Box& b, const RowMap& m, const SbpTables* d_sbp, const
    const Box ob = out ? b : pb;
    double* const dst = out ? out : P.o;
    if (out) k_adj_crop<<<cdiv(b.npts, 256), 256, 0, s>>>(b, pb, P.o, out);
-   // SBP rows: in-plane part from (sx sy) zB, then the k-direction terms
-   if (m.top || m.bot) {
-      k_adj_weight<true><<<cdiv(P.pb.npts, 256), 256, 0, s>>>(A, P, z);
-      if (m.top) k_rhs4sg_T_xy<<<dim3(gi, gj, 6), blk, 0, s>>>(A, P, 1, 1, ob, dst, cof);
-      if (m.bot) k_rhs4sg_T_xy<<<dim3(gi, gj, 6), blk, 0, s>>>(A, P, m.nz, -1, ob, dst, cof);
-      if (m.top) k_rhs4sg_T_col<<<dim3(gi, gj, 9), blk, 0, s>>>(A, 1, 1, z, ob, dst, cof);
-      if (m.bot) k_rhs4sg_T_col<<<dim3(gi, gj, 9), blk, 0, s>>>(A, m.nz, -1, z, ob, dst, cof);
-   }
+   const int ntx = (int)cdiv(b.ni, RTX), tl = ntx * (int)cdiv(b.je - b.jb + 1, RTY);
+   const dim3 grd(tl, rows_planes_spread(tl));
+   if (m.top) k_rhs4sg_T_rows<<<grd, RNT, 0, s>>>(A, ntx, 1, 1, z, ob, dst, cof);
+   if (m.bot) k_rhs4sg_T_rows<<<grd, RNT, 0, s>>>(A, ntx, m.nz, -1, z, ob, dst, cof);
    return check_hip(hipGetLastError(), "rhs4sg transpose launch");
 }
 
@@ -1143,15 +1184,12 @@ int launch_rhs4sg_matgrad(const Box& b, const RowMap& m, const SbpTables* d_sbp,
 {
    const AdjCtx A{b, m, d_sbp, mu, la, strx, stry, strz};
    const double cof = 1.0 / (h * h);
-   const dim3 blk(64, 4, 1);
-   const unsigned gi = cdiv(b.ni, 64), gj = cdiv(b.je - b.jb + 1, 4);
-   {
-      const int ntx = (int)cdiv(b.ni, GTX), nty = (int)cdiv(b.je - b.jb + 1, GTY);
-      const int kc = march_kchunk((long)ntx * nty, b.ke - b.kb + 1, 2), nkc = (int)cdiv(b.ke - b.kb + 1, kc);
-      k_rhs4sg_matgrad_march<<<ntx * nty * nkc, GNT, 0, s>>>(A, ntx, nty, kc, z, u, gmu, gla, cof);
-   }
-   if (m.top) k_rhs4sg_matgrad_sbp<<<dim3(gi, gj, 8), blk, 0, s>>>(A, 1, 1, z, u, gmu, gla, cof);
-   if (m.bot) k_rhs4sg_matgrad_sbp<<<dim3(gi, gj, 8), blk, 0, s>>>(A, m.nz, -1, z, u, gmu, gla, cof);
+   const int ntx = (int)cdiv(b.ni, GTX), nty = (int)cdiv(b.je - b.jb + 1, GTY);  // RTX x RTY is the same tile
+   const int kc = march_kchunk((long)ntx * nty, b.ke - b.kb + 1, 2), nkc = (int)cdiv(b.ke - b.kb + 1, kc);
+   k_rhs4sg_matgrad_march<<<ntx * nty * nkc, GNT, 0, s>>>(A, ntx, nty, kc, z, u, gmu, gla, cof);
+   const dim3 grd(ntx * nty, rows_planes_spread(ntx * nty));
+   if (m.top) k_rhs4sg_matgrad_rows<<<grd, RNT, 0, s>>>(A, ntx, 1, 1, z, u, gmu, gla, cof);
+   if (m.bot) k_rhs4sg_matgrad_rows<<<grd, RNT, 0, s>>>(A, ntx, m.nz, -1, z, u, gmu, gla, cof);
    return check_hip(hipGetLastError(), "rhs4sg material-derivative launch");
 }
 
@@ -1215,22 +1253,31 @@ int launch_bcfortsg_T(const Box& b, const int* wind, int nx, int ny, int nz, con
 {
    (void)nx;
    (void)ny;
+   WinListT zero{};
+   auto flush = [&]() {
+      if (zero.n > 0) k_bc_zero_T<<<cdiv(zero.off[zero.n], 256), 256, 0, s>>>(b, zero, y);
+      zero.n = 0;
+   };
    for (int side = 5; side >= 0; side--) {
       const int* w = wind + 6 * side;
-      const WinT win{w[0], w[1], w[2], w[3], w[4], w[5]};
       const long n = (long)(w[1] - w[0] + 1) * (w[3] - w[2] + 1) * (w[5] - w[4] + 1);
       if (bccnd[side] == 1 || bccnd[side] == 2) {
-         if (n > 0) k_bc_zero_T<<<cdiv(n, 256), 256, 0, s>>>(b, win, y);
+         if (n <= 0) continue;
+         zero.w[zero.n] = WinT{w[0], w[1], w[2], w[3], w[4], w[5]};
+         zero.off[zero.n + 1] = zero.off[zero.n] + n;
+         zero.n++;
       } else if (bccnd[side] == 0) {
          if (side != 4 && side != 5) return set_error(E_INVAL, "bcfortsg transpose: free surface only on sides 4, 5");
+         flush();
          const int k = side == 4 ? 1 : nz, kl = side == 4 ? 1 : -1;
          dim3 blk(64, 4, 1), grd(cdiv(b.ni, 64), cdiv(b.je - b.jb + 1, 4), 1);
          k_freesurf_take<<<grd, blk, 0, s>>>(b, k, kl, y, plane);
-         k_freesurf_push<<<grd, blk, 0, s>>>(b, k, kl, h, d_sbp, plane, fwd, mu, la, strx, stry, y, gmu, gla);
+         k_freesurf_push<<<grd, blk, 0, s>>>(b, k, kl, d_sbp, plane, fwd, mu, la, strx, stry, y, gmu, gla);
       } else if (bccnd[side] == 3) {
          return set_error(E_INVAL, "the adjoint does not support periodic sides");
       }
    }
+   flush();
    return check_hip(hipGetLastError(), "bcfortsg transpose launch");
 }
 

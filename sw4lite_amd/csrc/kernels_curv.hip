@@ -172,26 +172,7 @@ __device__ __forceinline__ void t_terms(const S& s, int i, int j, int m, double 
 // (the scheduler would otherwise hoist the shared-memory reads of a whole
 // plane to its start and spill)
 #define SW4_SCHED_FENCE __builtin_amdgcn_sched_barrier(0)
-constexpr int MTX = 32, MTY = 8, MHX = MTX + 4, MHY = MTY + 4, MPL = MHX * MHY, MNT = 448;
-
-// A thread's point of the tile with its halo, and its part: 0 output, 1 j
-// halo, 2 i halo and corners (whole waves; the last 16 threads repeat a point).
-__device__ __forceinline__ void march_point(int tid, int& role, int& hx, int& hy)
-{
-   role = __builtin_amdgcn_readfirstlane(tid < 256 ? 0 : tid < 384 ? 1 : 2);
-   if (tid < 256) {
-      hx = 2 + tid % MTX;
-      hy = 2 + tid / MTX;
-   } else if (tid < 384) {
-      const int r = (tid - 256) / MTX;
-      hx = 2 + tid % MTX;
-      hy = r < 2 ? r : r + MTY;
-   } else {
-      const int q = tid - 384, c = q % 4, r = q / 4;  // rows 0..7: the tile's, 8..11: the corners'
-      hx = c < 2 ? c : c + MTX;
-      hy = r < MTY ? 2 + r : r < MTY + 2 ? r - MTY : r < MTY + 4 ? r : 2;
-   }
-}
+constexpr int MTX = RTX, MTY = RTY, MHX = RHX, MHY = RHY, MPL = RPL, MNT = RNT;  // the tile of sbp_rows.h (rows_point)
 
 template <int CO>
 __global__ void __launch_bounds__(MNT, 1)
@@ -211,7 +192,7 @@ k_rhs4curv_march(Box b, int ntx, int nty, int ntiles, int klo, int khi, int kc, 
    const int k0 = klo + tkz * kc, k1 = min(khi, k0 + kc - 1);
    const int tid = threadIdx.x;
    int role, hx, hy;
-   march_point(tid, role, hx, hy);
+   rows_point(tid, role, hx, hy);
    const bool own = tid < MPL;  // the last 16 threads repeat a point and store nothing
    const Box& b_ = b;
    const int ia = b_.ib + tix * MTX, ja = b_.jb + tjy * MTY;
@@ -440,7 +421,7 @@ k_rhs4curv_rows(Box b, int ntx, const SbpTables* __restrict__ sbp, CurvG<CO> s, 
    const int tix = blockIdx.x % ntx, tjy = blockIdx.x / ntx;
    const int tid = threadIdx.x;
    int role, hx, hy;
-   march_point(tid, role, hx, hy);
+   rows_point(tid, role, hx, hy);
    const bool own = tid < MPL;
    const bool ihalo = role == 2 && tid < 384 + 4 * MTY;
    const int ia = b.ib + tix * MTX, ja = b.jb + tjy * MTY;
@@ -680,7 +661,7 @@ k_curv_corr(Box b, int ntx, int nty, int ntiles, int klo, int khi, int kc, doubl
    const int k0 = klo + tkz * kc, k1 = min(khi, k0 + kc - 1);
    const int tid = threadIdx.x;
    int role, hx, hy;
-   march_point(tid, role, hx, hy);
+   rows_point(tid, role, hx, hy);
    const int ia = b.ib + tix * MTX, ja = b.jb + tjy * MTY;
    const bool active = role == 0 && ia + hx <= b.ie - 2 && ja + hy <= b.je - 2;
    const int ii = min(ia + hx, b.ie) - b.ib, jj = min(ja + hy, b.je) - b.jb;

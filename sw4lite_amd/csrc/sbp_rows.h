@@ -27,6 +27,25 @@ namespace sw4amd {
 
 constexpr int RTX = 32, RTY = 8, RHX = RTX + 4, RHY = RTY + 4, RPL = RHX * RHY, RNT = 448;
 
+// A thread's point of the tile with its halo, and its part: 0 output, 1 j
+// halo, 2 i halo and corners (whole waves; the last 16 threads repeat a point).
+__device__ __forceinline__ void rows_point(int tid, int& role, int& hx, int& hy)
+{
+   role = __builtin_amdgcn_readfirstlane(tid < 256 ? 0 : tid < 384 ? 1 : 2);
+   if (tid < 256) {
+      hx = 2 + tid % RTX;
+      hy = 2 + tid / RTX;
+   } else if (tid < 384) {
+      const int r = (tid - 256) / RTX;
+      hx = 2 + tid % RTX;
+      hy = r < 2 ? r : r + RTY;
+   } else {
+      const int q = tid - 384, c = q % 4, r = q / 4;  // rows 0..7: the tile's, 8..11: the corners'
+      hx = c < 2 ? c : c + RTX;
+      hy = r < RTY ? 2 + r : r < RTY + 2 ? r - RTY : r < RTY + 4 ? r : 2;
+   }
+}
+
 template <class R, class Load, class Epi>
 __device__ __forceinline__ void sbp_rows_body(const Box& b, int top, int nk, int ntx,
                                               const SbpTablesT<R>* __restrict__ sbp, const R* __restrict__ mu,
@@ -40,20 +59,8 @@ __device__ __forceinline__ void sbp_rows_body(const Box& b, int top, int nk, int
    __shared__ R ssx[RHX], ssy[RHY];
    const int tix = blockIdx.x % ntx, tjy = blockIdx.x / ntx;
    const int tid = threadIdx.x;
-   const int role = __builtin_amdgcn_readfirstlane(tid < 256 ? 0 : tid < 384 ? 1 : 2);  // output, j halo, i halo
-   int hx, hy;
-   if (tid < 256) {
-      hx = 2 + tid % RTX;
-      hy = 2 + tid / RTX;
-   } else if (tid < 384) {
-      const int r = (tid - 256) / RTX;
-      hx = 2 + tid % RTX;
-      hy = r < 2 ? r : r + RTY;
-   } else {
-      const int q = tid - 384, c = q % 4, r = q / 4;  // rows 0..7: the tile's, 8..11: the corners'
-      hx = c < 2 ? c : c + RTX;
-      hy = r < RTY ? 2 + r : r < RTY + 2 ? r - RTY : r < RTY + 4 ? r : 2;
-   }
+   int role, hx, hy;
+   rows_point(tid, role, hx, hy);
    const bool own = tid < RPL;  // the last 16 threads repeat a point and store nothing
    const bool ihalo = role == 2 && tid < 384 + 4 * RTY;
    const int ia = b.ib + tix * RTX, ja = b.jb + tjy * RTY;

@@ -125,6 +125,17 @@ def test_rhs4sg_material_derivative(torch, coefs, os45, shape):
     assert dot_rel(a_m, b_m) < DOT_TOL and dot_rel(a_l, b_l) < DOT_TOL
 
 
+@pytest.mark.parametrize("shape", [(28, 4, 12), (29, 5, 13), (130, 127, 14), (260, 250, 12)])
+def test_rows_transpose_over_tiles(torch, coefs, shape):
+    """The SBP rows of both sides, transposed and differentiated: one whole
+    tile, a column and a row more, and grids whose tiles leave room for a few
+    planes' workgroups each and for one (five tiles by 17, nine by 32).  The
+    bar is that of the smaller shapes: rounding of the dot products' sums
+    grows with the square root of the terms and is relative to them."""
+    test_rhs4sg_transpose(torch, coefs, (1, 1), shape)
+    test_rhs4sg_material_derivative(torch, coefs, (1, 1), shape)
+
+
 @pytest.mark.parametrize("shape", [(23, 17, 19), (37, 11, 70)])
 def test_addsgd4_transpose(torch, shape):
     from sw4lite_amd import ew
