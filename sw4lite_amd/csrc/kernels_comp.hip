@@ -317,22 +317,28 @@ k_comp_sweep(Box b, CompTiles map, int kbeg, int kend, int kc, const float* __re
 // C (or rho) are issued after the barrier and used after the stencil, the
 // column values one plane ahead.  Rings: the staged field in six slots
 // (planes k-2..k+3), D in four (k..k+3), mu, lambda (and rho) in two.  Same
-// arithmetic in the same order as k_comp_sweep.  Needs ni % 4 == 0 and
-// 16-byte aligned arrays (every quad of floats in one row, aligned).  The
-// predictor runs at 4 waves/SIMD (128 registers, 2 of them spilled: faster
-// than 3 waves without the spill).
+// arithmetic in the same order as k_comp_sweep.  The 16-byte loads need
+// ni % 4 == 0 and 16-byte aligned arrays (every quad of floats in one row,
+// aligned).  DW: one float a load, any row and alignment, four times the load
+// instructions; the corrector gains by it (two workgroups a CU either way,
+// 301 x 301 x 171 points: 564 us register-staged, 525), the predictor
+// does not (its extra addresses spill at 4 waves/SIMD: 344 us against 428).
+// The predictor runs at 4 waves/SIMD (128 registers, 2 of them spilled:
+// faster than 3 waves without the spill).
 #define SW4_LDSF(p) ((__attribute__((address_space(3))) void*)(p))
-template <bool CORR>
+template <bool CORR, bool DW>
 __global__ void __launch_bounds__(NT, CORR ? 2 : 4)
 k_comp_dma(Box b, CompTiles map, int kbeg, int kend, int kc, const float* __restrict__ stg,
            const float* __restrict__ mu, const float* __restrict__ la, const float* __restrict__ rho, SgCoefF sg,
            const float* __restrict__ dold, float* __restrict__ dnew, float* __restrict__ uu,
            float* __restrict__ cc, float* __restrict__ aout, float cof, float dt2, float c4, float beta)
 {
-   constexpr int QP = 3 * PL / 4;          // quads of a staged 3-component plane
-   constexpr int NQ = (QP + NT - 1) / NT;  // asynchronous loads per thread and plane
-   constexpr int QM = PL / 4;              // quads of a scalar plane
-   static_assert(HX % 4 == 0 && QM <= NT, "quads must tile the rows; one material load per thread");
+   constexpr int LW = DW ? 1 : 4;          // floats of one load
+   constexpr int QP = 3 * PL / LW;         // loads of a staged 3-component plane
+   constexpr int NQ = (QP + NT - 1) / NT;  // and per thread
+   constexpr int QM = PL / LW;             // loads of a scalar plane
+   constexpr int NM = (QM + NT - 1) / NT;
+   static_assert(HX % 4 == 0, "quads must tile the rows");
    __shared__ __align__(16) float su[6 * 3 * PL];              // plane kp in slot (kp - k0 + 2) % 6
    __shared__ __align__(16) float sd[CORR ? 4 * 3 * PL : 4];   // D of plane kp in slot (kp - k0) % 4
    __shared__ __align__(16) float sm[2 * PL], sl[2 * PL];      // plane kp in half (kp - k0) & 1
@@ -354,36 +360,46 @@ k_comp_dma(Box b, CompTiles map, int kbeg, int kend, int kc, const float* __rest
    const long col = active ? (i - b.ib) + ni * (j - b.jb) : 0;
    const int o = (ty + 2) * HX + tx + 2;
 
-   // quad m = tid + p NT of the staged (c, jj, ii) tile: offset of its first float
+   // load m = tid + p NT of the staged (c, jj, ii) tile: offset of its first float
    long goff[NQ];
 #pragma unroll
    for (int p = 0; p < NQ; p++) {
-      const int e = 4 * (tid + p * NT);
+      const int e = LW * (tid + p * NT);
       const int c = e / PL, r = e - c * PL, jj = r / HX, ii = r - jj * HX;
       const int gi = ia + ii, gj = ja + jj;
       const bool ok = e < 3 * PL && gi <= b.ie && gj <= b.je;
       goff[p] = ok ? (gi - b.ib) + ni * (gj - b.jb) + npts * c : 0;
    }
-   long moff;
-   {
-      const int e = 4 * tid, jj = e / HX, ii = e - jj * HX;
+   long moff[NM];
+#pragma unroll
+   for (int p = 0; p < NM; p++) {
+      const int e = LW * (tid + p * NT), jj = e / HX, ii = e - jj * HX;
       const int gi = ia + ii, gj = ja + jj;
-      moff = e < PL && gi <= b.ie && gj <= b.je ? (gi - b.ib) + ni * (gj - b.jb) : 0;
+      moff[p] = e < PL && gi <= b.ie && gj <= b.je ? (gi - b.ib) + ni * (gj - b.jb) : 0;
    }
+   auto load = [&](const float* g, float* dst) {
+      if constexpr (DW)
+         __builtin_amdgcn_global_load_lds(g, SW4_LDSF(dst), 4, 0, 0);
+      else
+         __builtin_amdgcn_global_load_lds(g, SW4_LDSF(dst), 16, 0, 0);
+   };
    auto dma3 = [&](const float* src, float* ring, int kp, int slot) {
       const float* g = src + nij * (kp - b.kb);
-      float* dst = ring + slot * 3 * PL + 4 * 64 * wv;
+      float* dst = ring + slot * 3 * PL + LW * 64 * wv;
 #pragma unroll
       for (int p = 0; p < NQ; p++)
-         if (tid + p * NT < QP) __builtin_amdgcn_global_load_lds(g + goff[p], SW4_LDSF(dst + 4 * p * NT), 16, 0, 0);
+         if (tid + p * NT < QP) load(g + goff[p], dst + LW * p * NT);
    };
    auto dma_mat = [&](int kp, int half) {
-      if (tid < QM) {
-         const long pb = nij * (kp - b.kb);
-         __builtin_amdgcn_global_load_lds(mu + pb + moff, SW4_LDSF(sm + half * PL + 4 * 64 * wv), 16, 0, 0);
-         __builtin_amdgcn_global_load_lds(la + pb + moff, SW4_LDSF(sl + half * PL + 4 * 64 * wv), 16, 0, 0);
-         if (CORR)
-            __builtin_amdgcn_global_load_lds(rho + pb + moff, SW4_LDSF(sr + half * PL + 4 * 64 * wv), 16, 0, 0);
+      const long pb = nij * (kp - b.kb);
+#pragma unroll
+      for (int p = 0; p < NM; p++) {
+         if (tid + p * NT < QM) {
+            const int d = half * PL + LW * (64 * wv + p * NT);
+            load(mu + pb + moff[p], sm + d);
+            load(la + pb + moff[p], sl + d);
+            if (CORR) load(rho + pb + moff[p], sr + d);
+         }
       }
    };
 
@@ -902,13 +918,16 @@ int comp_sweep(bool corr, const Box& b, int k1, int k2, int kc, const CompState&
    auto al = [](const float* p) { return ((uintptr_t)p & 15) == 0; };
    const bool fits = async && b.ni % 4 == 0 && al(st.mu) && al(st.la) && al(st.rho) && (corr ? al(st.A) && al(st.D) : al(st.U));
    if (corr && fits)
-      k_comp_dma<true><<<grd, NT, 0, s>>>(b, map, k1, k2, kc, st.A, st.mu, st.la, st.rho, sg, st.D, st.Dn, st.U, st.C,
+      k_comp_dma<true, false><<<grd, NT, 0, s>>>(b, map, k1, k2, kc, st.A, st.mu, st.la, st.rho, sg, st.D, st.Dn, st.U, st.C,
                                           nullptr, cof, dt2, c4, beta);
+   else if (corr && async)
+      k_comp_dma<true, true><<<grd, NT, 0, s>>>(b, map, k1, k2, kc, st.A, st.mu, st.la, st.rho, sg, st.D, st.Dn, st.U,
+                                                st.C, nullptr, cof, dt2, c4, beta);
    else if (corr)
       k_comp_sweep<true><<<grd, NT, 0, s>>>(b, map, k1, k2, kc, st.A, st.mu, st.la, st.rho, sg, st.D, st.Dn, st.U,
                                             st.C, nullptr, cof, dt2, c4, beta);
    else if (fits)
-      k_comp_dma<false><<<grd, NT, 0, s>>>(b, map, k1, k2, kc, st.U, st.mu, st.la, st.rho, sg, nullptr, nullptr,
+      k_comp_dma<false, false><<<grd, NT, 0, s>>>(b, map, k1, k2, kc, st.U, st.mu, st.la, st.rho, sg, nullptr, nullptr,
                                            nullptr, nullptr, st.A, cof, dt2, c4, beta);
    else
       k_comp_sweep<false><<<grd, NT, 0, s>>>(b, map, k1, k2, kc, st.U, st.mu, st.la, st.rho, sg, nullptr, nullptr,
