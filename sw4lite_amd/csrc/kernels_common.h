@@ -289,6 +289,19 @@ __device__ __forceinline__ void rhs_sbp_point(const Box& b, int i, int j, int k,
 #undef KK
 }
 
+// Stores v where p holds other bits: for ghost values that are zero already in
+// almost every step, where a frame's columns would write a few bytes of a
+// cache line each.  512^3: the FP32 corrector's shell 258 -> 192 us, its
+// predictor's 170 -> 144, the FP64 ones 138 -> 121 on average.
+__device__ __forceinline__ void put_changed(double* p, double v)
+{
+   if (__double_as_longlong(*p) != __double_as_longlong(v)) *p = v;
+}
+__device__ __forceinline__ void put_changed(float* p, float v)
+{
+   if (__float_as_int(*p) != __float_as_int(v)) *p = v;
+}
+
 // Point q of the ghost shell, the 2-point frame outside [1,nx]x[1,ny]x[1,nz]
 // (the k planes kb, kb+1, ke-1, ke first, then the j and i frames of the
 // remaining planes); false past the last shell point.

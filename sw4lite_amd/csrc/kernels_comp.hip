@@ -733,10 +733,11 @@ struct PredView {
    {
       return ((double)U[q] + (double)C[q]) + ((double)D[q] + dt2 * (double)A[q]);
    }
-   __device__ __forceinline__ void set(long q, double g) const
+   __device__ __forceinline__ float value(long q, double g) const
    {
-      A[q] = (float)(((g - ((double)U[q] + (double)C[q])) - (double)D[q]) / dt2);
+      return (float)(((g - ((double)U[q] + (double)C[q])) - (double)D[q]) / dt2);
    }
+   __device__ __forceinline__ void set(long q, double g) const { A[q] = value(q, g); }
 };
 // Corrector: u^{n+1} = U + C; a ghost value g replaces it, and Dn takes the
 // same change.
@@ -791,17 +792,19 @@ __global__ void k_comp_shell_fill(Box b, CompState st, float dt2, double dt2d, i
    for (int c = 0; c < 3; c++) {
       const long v = p + b.npts * c;
       if (!CORR) {
-         st.A[v] = 0.0f;
-         if (zero) PredView{st.U, st.C, st.D, st.A, dt2d}.set(v, 0.0);
+         if (zero)
+            put_changed(st.A + v, PredView{st.U, st.C, st.D, st.A, dt2d}.value(v, 0.0));
+         else
+            st.A[v] = 0.0f;
       } else {
          const float dn = st.D[v] + dt2 * st.A[v];
          float U = st.U[v], C = st.C[v];
          comp_add(U, C, dn);
          if (zero) {
             const double u = (double)U + (double)C;
-            st.Dn[v] = (float)((double)dn + (0.0 - u));
-            st.U[v] = 0.0f;
-            st.C[v] = 0.0f;
+            put_changed(st.Dn + v, (float)((double)dn + (0.0 - u)));
+            put_changed(st.U + v, 0.0f);
+            put_changed(st.C + v, 0.0f);
          } else {
             st.Dn[v] = dn;
             st.U[v] = U;

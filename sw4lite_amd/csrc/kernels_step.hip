@@ -172,16 +172,24 @@ __global__ void k_shell(Box b, int mode, const double* __restrict__ a, const dou
 #pragma unroll
       for (int c = 0; c < 3; c++) {
          const long v = p + b.npts * c;
-         const double uv = u[v], mv = um[v], o = zero ? 0.0 : 2 * uv - mv;
-         out[v] = o;
-         acc[v] = dt2i * (o - 2 * uv + mv);
+         const double uv = u[v], mv = um[v], o = zero ? 0.0 : 2 * uv - mv, a2 = dt2i * (o - 2 * uv + mv);
+         if (zero) {
+            put_changed(out + v, o);
+            put_changed(acc + v, a2);
+         } else {
+            out[v] = o;
+            acc[v] = a2;
+         }
       }
       return;
    }
 #pragma unroll
    for (int c = 0; c < 3; c++) {
       const long v = p + b.npts * c;
-      out[v] = zero ? 0.0 : mode == 0 ? 2 * u[v] - um[v] : a[v];
+      if (zero)
+         put_changed(out + v, 0.0);
+      else
+         out[v] = mode == 0 ? 2 * u[v] - um[v] : a[v];
    }
 }
 

@@ -255,3 +255,31 @@ def test_comp_async_sweeps_match_oracle(torch):
     err = field_errors(u, um, ref)
     print("FP32 asynchronous-load sweeps vs oracle", err, flush=True)
     assert err["u"] < FP32_TOL and err["um"] < FP32_TOL
+
+
+@pytest.mark.parametrize("mode", [0, 2])
+@pytest.mark.parametrize("nsteps", [1, 2, 4])
+def test_zero_ghosts_from_nonzero_ones(torch, mode, nsteps):
+    """The zero ghost values of supergrid and Dirichlet sides are stored where
+    they change: from a state whose ghost points are not zero, every field of
+    the rotation holds the zeros, and the step meets the reference order's."""
+    from sw4lite_amd import EW
+    nx, ny, nz, h = 21, 18, 16, 0.1
+    rho, mu, la = layered_material(nx, ny, nz, h, 3)
+    rng = np.random.default_rng(12)
+    n = 3 * (nx + 4) * (ny + 4) * (nz + 4)
+    u = rng.uniform(-1, 1, n)
+    um = u - 1e-3 * rng.uniform(-1, 1, n)
+    res = []
+    for m in (mode, 1):
+        e = EW(nx, ny, nz, h, [2, 1, 2, 2, 0, 1], corder=1, sg_gp_thickness=4)
+        e.set_material(rho, mu, la)
+        e.setup(nsteps=nsteps)
+        e.set_solution(u, um)
+        e.timesteploop(nsteps, mode=m)
+        res.append(e.get_solution()[0])
+        e.close()
+    got = res[0].reshape(3, nz + 4, ny + 4, nx + 4)
+    for side in (got[..., :2], got[..., -2:], got[:, :, :2], got[:, :, -2:], got[:, -2:]):
+        assert not np.any(side)
+    assert relerr(res[0], res[1]) < (1e-12 if mode == 0 else FP32_TOL)
