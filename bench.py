@@ -77,8 +77,7 @@ def parse():
                         "9 as 8 with the damping sweep only over the supergrid layers, "
                         "10 as 9 with rows of odd length staged by four-byte asynchronous loads")
     p.add_argument("--kchunk", type=int, default=0,
-                   help="planes per workgroup of the LDS sweeps (0: the library's defaults, 64 for the predictor "
-                        "and corrector sweeps, 32 for the damping sweep)")
+                   help="planes per workgroup of the LDS sweeps (0: chosen from the grid's size)")
     p.add_argument("--calibrate-copy", action="store_true",
                    help="also launch a plain device copy of 1 GiB (PMC scaling)")
     p.add_argument("--workload", choices=["cartesian", "curvilinear", "precision", "adjoint", "batch",
@@ -401,7 +400,7 @@ def main_curvilinear(a, torch):
                           "source": "one double couple, Ricker 4 Hz"},
         },
         "roofline": {"bound": "fp64", "achieved": tflops, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
-                     "frac": tflops / FP64_PEAK_TFLOPS, "traffic": None, "kernel": "k_rhs4curv",
+                     "frac": tflops / FP64_PEAK_TFLOPS, "traffic": None, "kernel": "k_rhs4curv_march",
                      "flop_per_launch": flop, "avg_launch_ms": ms_rhs},
         "cpu_baseline": None,
     }
@@ -435,7 +434,7 @@ def bench_fp32(a, e, torch, n, fp64_value):
         "pred_interior_GBps": corr_pts * COMP_PRED_BYTES_PER_PT / (pred_ms * 1e-3) / 1e9,
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS,
-                     "kernel": "k_comp_dma<true>" if a.variant >= 7 and (n + 4) % 4 == 0 else "k_comp_sweep<true>",
+                     "kernel": "k_comp_dma" if a.variant >= 7 else "k_comp_sweep",
                      "bytes_per_launch": corr_pts * COMP_CORR_BYTES_PER_PT, "avg_launch_ms": corr_ms},
     }
 
