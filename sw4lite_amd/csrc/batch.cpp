@@ -105,7 +105,9 @@ int Batch::init()
       m_ndtiles[q] = (int)v.size();
    }
    // the predictor stores the acceleration in the shot's own field and the
-   // corrector stages it, as the single-grid step does
+   // corrector stages it, for the kernel variants that do so in the
+   // single-grid step; the others' corrector forms it from Up, U and Um, and
+   // so does that of odd rows where memory is short
    m_acc.assign(n, nullptr);
    for (int q = 0; q < n; q++) {
       EW* e = m_shots[q];
@@ -113,7 +115,7 @@ int Batch::init()
       const GridSetup& g = e->m_opt.grid;
       const int k1 = e->m_onesided[4] == 1 ? 7 : b.kb + 2;
       const int k2 = e->m_onesided[5] == 1 ? g.nz - 6 : b.ke - 2;
-      if (k2 >= k1 && (rc = e->accel_field(&m_acc[q], true))) return rc;
+      if (k2 >= k1 && (rc = e->accel_field(&m_acc[q])) && b.ni % 2 == 0) return rc;
    }
    return refresh();
 }
@@ -166,10 +168,13 @@ int Batch::build_tables()
       kchunk = march_kchunk(tiles, npl, 2);
    }
    for (int ph = 0; ph < 3; ph++) {
-      // the grids whose planes take the 16-byte loads first (their own launch,
-      // block ids from 0), then the others, by four-byte loads
-      int g0[3] = {0, 0, 0}, ga[3] = {0, 0, 0}, slot[3] = {0, 0, 0};
-      for (int pass = 0; pass < 2; pass++)
+      // a launch of its own (block ids from 0) for each way to bring the
+      // planes: the grids that take 16-byte loads first, then those of
+      // four-byte loads, then the correctors without a stored acceleration
+      int slot[3] = {0, 0, 0};
+      for (int pass = 0; pass < 3; pass++) {
+         int next[3] = {0, 0, 0};  // free block id of each kind's launch
+         const int first[3] = {slot[0], slot[1], slot[2]};
          for (int q = 0; q < n; q++) {
             EW* e = m_shots[q];
             const GridSetup& g = e->m_opt.grid;
@@ -184,12 +189,13 @@ int Batch::build_tables()
             const double* pa[3] = {u, e->mMu.dev, e->mLambda.dev};
             const double* da[4] = {u, um, e->mRho.dev, up2};
             const double* ca[4] = {m_acc[q], e->mUp.dev, e->mMu.dev, e->mLambda.dev};
-            const bool fa[3] = {async_loads_fit(b, pa, 3), m_acc[q] && async_loads_fit(b, ca, 4),
-                                async_loads_fit(b, da, 4)};
+            const int list[3] = {async_loads_fit(b, pa, 3) ? LOADS_WIDE : LOADS_NARROW,
+                                 !m_acc[q] ? LOADS_STAGED : async_loads_fit(b, ca, 4) ? LOADS_WIDE : LOADS_NARROW,
+                                 async_loads_fit(b, da, 4) ? LOADS_WIDE : LOADS_NARROW};
             const bool damp = e->m_opt.beta != 0;
             for (int k = 0; k < 3; k++) {
-               if (fa[k] != (pass == 0)) continue;
-               int& gc = fa[k] ? ga[k] : g0[k];
+               if (list[k] != pass) continue;
+               int& gc = next[k];
                SweepShot* d = &t[k * n + slot[k]++];
                if (k == 0)
                   gc = fill_sweep_shot(false, b, k1, k2, kchunk, nullptr, u, um, e->mMu.dev, e->mLambda.dev,
@@ -204,12 +210,11 @@ int Batch::build_tables()
                                        e->mRho.dev, c, up2, g.h, e->mDt, e->m_opt.beta, true, gc, d, m_dtiles[q],
                                        m_ndtiles[q]);
             }
-            if (pass == 0)
-               for (int k = 0; k < 3; k++) m_nasync[ph][k] = slot[k];
          }
-      for (int k = 0; k < 3; k++) {
-         m_nblk[ph][k] = g0[k];
-         m_nblk_async[ph][k] = ga[k];
+         for (int k = 0; k < 3; k++) {
+            m_nlist[ph][k][pass] = slot[k] - first[k];
+            m_nblk[ph][k][pass] = next[k];
+         }
       }
    }
    if (m_exec) {
@@ -224,13 +229,16 @@ int Batch::one_step(int ph)
    const int n = (int)m_shots.size();
    const SweepShot* tab = m_dtab + (ph * 3) * n;
    int rc;
-   // the two lists of a sweep side by side, between a fork and a join: each
+   // the 16-byte list of a sweep beside the others, between a fork and a join: each
    // fills the other's last round of workgroups (six shots: 17.0 -> 16.6 ms for six steps)
    auto sweeps = [&](int kind) {
-      const int a = m_nasync[ph][kind];
       const SweepShot* t = tab + kind * n;
-      const int r = launch_sweep_batch(kind, true, t, a, m_nblk_async[ph][kind], m_nblk[ph][kind] ? m_side[WIDE] : m_s);
-      return r ? r : launch_sweep_batch(kind, false, t + a, n - a, m_nblk[ph][kind], m_s);
+      const int *ns = m_nlist[ph][kind], *nb = m_nblk[ph][kind];
+      int r = OK;
+      for (int l = 0; l < 3 && r == OK; t += ns[l++])
+         r = launch_sweep_batch(kind, (SweepLoads)l, t, ns[l], nb[l],
+                                l == LOADS_WIDE && nb[LOADS_NARROW] + nb[LOADS_STAGED] ? m_side[WIDE] : m_s);
+      return r;
    };
    // each grid's SBP rows and ghost shell (which write only the planes and
    // points the interior sweeps do not, from inputs the sweeps do not

@@ -50,23 +50,22 @@ private:
    std::vector<EW*> m_shots;
    hipStream_t m_s = nullptr;
    SweepShot* m_dtab = nullptr;     // [phase 0..2][kind 0..2][shot]
-   int m_nblk[3][3] = {{0}};        // workgroups of each kind's launch of four-byte loads
-   // the first m_nasync shots of a table take the sixteen-byte loads (their
-   // own launch of m_nblk_async workgroups)
-   int m_nasync[3][3] = {{0}};
-   int m_nblk_async[3][3] = {{0}};
+   // [phase][kind][SweepLoads]: the shots of a table are ordered by how their
+   // planes are brought; shots and workgroups of each list's launch
+   int m_nlist[3][3][3] = {};
+   int m_nblk[3][3][3] = {};
    double* m_clk_t = nullptr;       // per shot: time, dt
    double* m_clk_dt = nullptr;
    int* m_clk_s = nullptr;          // per shot: sample count, maximum
    int* m_clk_max = nullptr;
    std::vector<double*> m_base;     // per shot: Um, U, Up2 of phase 0
    int m_phase = 0;
-   int m_kchunk = 0;  // planes per workgroup of the batched sweeps; 0: from the shots' sizes
+   int m_kchunk = 0;  // planes per workgroup of every batched sweep; 0: from all shots' tiles
    hipGraphExec_t m_exec = nullptr;
    std::vector<void*> m_allocs;
    std::vector<DampTile*> m_dtiles;  // per shot: its damping tile list (kernel variant 9), or null
    std::vector<int> m_ndtiles;
-   std::vector<double*> m_acc;       // per shot: its acceleration field (kernel variant 8 and later), or null
+   std::vector<double*> m_acc;       // per shot: its acceleration field (EW::accel_field), or null
    std::vector<hipStream_t> m_saved;
    WorkPool m_wpool;  // the shots' gradient work memory
    // the per-grid boundary work of the shots runs on NSIDE streams (default

@@ -72,14 +72,13 @@ int EW::init()
    return OK;
 }
 
-// The whole acceleration for kernel variant 8 (3 npts doubles, allocated at
-// the first step that uses it); null for the other variants and for odd row
-// lengths, whose sweeps cannot stage it (always: whatever the variant, for
-// the batch, whose sweeps all do).
-int EW::accel_field(double** p, bool always)
+// The whole acceleration (3 npts doubles, allocated at the first step that
+// uses it) for kernel variant 10, and for 8 and 9 on rows of even length;
+// null for the others, which form it where they read it.
+int EW::accel_field(double** p)
 {
    *p = nullptr;
-   if (!always && (m_variant < 8 || (m_box.ni % 2 != 0 && m_variant < 10))) return OK;
+   if (m_variant < 8 || (m_box.ni % 2 != 0 && m_variant < 10)) return OK;
    if (!m_accf) {
       void* q = nullptr;
       if (hipMalloc(&q, sizeof(double) * 3 * m_box.npts) != hipSuccess) {

@@ -190,7 +190,7 @@ public:
    std::vector<double> m_zhost;
    double* m_dacc = nullptr;  // acceleration on the planes the corrector's SBP rows read
    double* m_accf = nullptr;  // the whole acceleration (kernel variant 8), allocated at its first step
-   int accel_field(double** p, bool always = false);
+   int accel_field(double** p);
    // kernel variant 9: the damping sweep's tiles (damp_tiles) for planes
    // k1..k2 and the current k-chunk, made and uploaded on first use
    int damp_tile_list(int k1, int k2, const DampTile** tiles, int* n);

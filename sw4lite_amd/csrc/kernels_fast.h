@@ -40,8 +40,8 @@ struct SweepShot {
    SgCoef sg;
    double* out;
    double cof, dt2i, cupd, beta;
-   // predictor: where to store the acceleration; corrector: the stored
-   // acceleration it stages
+   // predictor: where to store the acceleration, or null; corrector: the
+   // stored acceleration it stages, or null (LOADS_STAGED)
    double* acc;
 };
 // Fill sh for planes k1..k2 of one grid (damping: the 32 x 8 damping sweep,
@@ -52,12 +52,15 @@ int fill_sweep_shot(bool damping, const Box& b, int k1, int k2, int kc, const do
                     const double* um, const double* mu, const double* la, const double* rho, const SgCoef& sg,
                     double* out, double h, double dt, double beta, bool corr, int grid0, SweepShot* sh,
                     const DampTile* tiles = nullptr, int ntiles = 0, double* acc = nullptr);
-// kind 0 predictor (storing the acceleration), 1 corrector (staging it), 2
-// damping sweeps of nshots grids in one launch of nblocks workgroups (d_shots
-// in device memory); wide: 16-byte asynchronous loads, for grids where
-// async_loads_fit (even row length, 16-byte aligned arrays), else four-byte
-// ones.
-int launch_sweep_batch(int kind, bool wide, const SweepShot* d_shots, int nshots, int nblocks, hipStream_t s);
+// How a batched sweep brings its planes: 16-byte asynchronous loads, for
+// grids where async_loads_fit (even row length, 16-byte aligned arrays),
+// four-byte ones, or (corrector only) through registers, the acceleration
+// formed from Up, U and Um on the way, for shots that do not store it.
+enum SweepLoads { LOADS_WIDE = 0, LOADS_NARROW = 1, LOADS_STAGED = 2 };
+// kind 0 predictor (storing the acceleration where the shot has a field), 1
+// corrector, 2 damping sweeps of nshots grids in one launch of nblocks
+// workgroups (d_shots in device memory).
+int launch_sweep_batch(int kind, SweepLoads loads, const SweepShot* d_shots, int nshots, int nblocks, hipStream_t s);
 bool async_loads_fit(const Box& b, const double* const* arrays, int n);
 
 // Interior planes k1..k2 of the predictor (corr = false: out = Up from u, um)

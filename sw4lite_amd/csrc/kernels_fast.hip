@@ -1071,8 +1071,9 @@ int fill_sweep_shot(bool damping, const Box& b, int k1, int k2, int kc, const do
    return grid0 + 8 * (int)cdiv(sh->map.ntiles, 8);
 }
 
-// Batched predictor, storing the acceleration, and batched corrector staging
-// it: 16-byte loads for the grids they fit, four-byte ones (DW) for the others.
+// Batched predictor, storing the acceleration where the shot has a field, and
+// batched corrector staging it: 16-byte loads for the grids they fit,
+// four-byte ones (DW) for the others.
 template <bool DW>
 __global__ void __launch_bounds__(NT, 2) k_pred_batch(const SweepShot* __restrict__ shots, int nshots)
 {
@@ -1087,6 +1088,14 @@ __global__ void __launch_bounds__(NT, 2) k_corr_batch(const SweepShot* __restric
    const SweepShot& h = shots[find_shot(shots, nshots, blockIdx.x)];
    sweep_dma_body<DMA_CORR, DW, true>(blockIdx.x - h.grid0, h.b, h.map, h.kbeg, h.kend, h.kc, h.acc, h.upin, h.mu,
                                       h.la, h.rho, h.sg, h.out, nullptr, h.cof, h.cupd, h.dt2i);
+}
+
+// Batched corrector of the shots without a stored acceleration.
+__global__ void __launch_bounds__(NT, 2) k_corr_batch_staged(const SweepShot* __restrict__ shots, int nshots)
+{
+   const SweepShot& h = shots[find_shot(shots, nshots, blockIdx.x)];
+   sweep_lds_body<true, false, false>(blockIdx.x - h.grid0, h.b, h.map, h.kbeg, h.kend, h.kc, h.upin, h.u, h.um, h.mu,
+                                      h.la, h.rho, h.sg, h.out, h.cof, h.dt2i, h.cupd, h.beta);
 }
 
 template <bool DW>
@@ -1106,10 +1115,13 @@ bool async_loads_fit(const Box& b, const double* const* arrays, int n)
    return true;
 }
 
-int launch_sweep_batch(int kind, bool wide, const SweepShot* d_shots, int nshots, int nblocks, hipStream_t s)
+int launch_sweep_batch(int kind, SweepLoads loads, const SweepShot* d_shots, int nshots, int nblocks, hipStream_t s)
 {
    if (nblocks <= 0) return OK;
-   if (kind == 0 && wide)
+   const bool wide = loads == LOADS_WIDE;
+   if (loads == LOADS_STAGED)
+      k_corr_batch_staged<<<nblocks, NT, 0, s>>>(d_shots, nshots);
+   else if (kind == 0 && wide)
       k_pred_batch<false><<<nblocks, NT, 0, s>>>(d_shots, nshots);
    else if (kind == 0)
       k_pred_batch<true><<<nblocks, NT, 0, s>>>(d_shots, nshots);

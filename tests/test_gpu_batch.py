@@ -14,10 +14,10 @@ from test_gpu_parity import SOURCES, layered_material
 pytestmark = pytest.mark.gpu
 TOL = 1e-13
 
-# even and odd row lengths: the sweeps of the first and last grids take the
-# asynchronous-load kernels (the predictor storing the acceleration, the
-# corrector staging it), the second grid's the register-staged ones, in
-# launches of their own
+# even and odd row lengths: the sweeps of the first and last grids take
+# sixteen-byte asynchronous loads, the second grid's four-byte ones, in
+# launches of their own (both the predictor storing the acceleration and the
+# corrector staging it)
 SHAPES = [(30, 28, 26, 0.08, [2, 2, 2, 2, 0, 2]), (25, 22, 20, 0.1, [2, 2, 2, 2, 2, 2]),
           (36, 20, 24, 0.09, [1, 2, 2, 1, 0, 0])]
 RECS = [(1.0, 1.05, 0.0, 0), (1.53, 0.77, 0.41, 1), (0.7, 0.6, 0.9, 0)]
@@ -31,12 +31,14 @@ def torch():
     return _t
 
 
-def make_shots(nsteps):
+def make_shots(nsteps, shapes=SHAPES, variant=None):
     from sw4lite_amd import EW
     shots = []
-    for q, (nx, ny, nz, h, bc) in enumerate(SHAPES):
+    for q, (nx, ny, nz, h, bc) in enumerate(shapes):
         rho, mu, la = layered_material(nx, ny, nz, h, 20 + q)
         e = EW(nx, ny, nz, h, bc, corder=1, sg_gp_thickness=5)
+        if variant is not None:
+            e.set_kernel_variant(variant)
         e.set_material(rho, mu, la)
         for s in SOURCES[: 1 + q % 3]:
             e.add_moment_source(s["x"], s["y"], s["z"], s["m"], s["t0"], s["freq"], s["tfkind"])
@@ -85,6 +87,62 @@ def test_batch_matches_single_shots(torch, graph):
         got = e.receivers()
         assert got.shape == want_tr[q].shape
         assert relerr(got, want_tr[q]) < TOL
+    b.close()
+    for e in shots:
+        e.close()
+
+
+EVEN, ODD, EVEN2 = SHAPES
+ODD2 = (33, 19, 21, 0.1, [2, 2, 2, 2, 0, 2])
+THIN = [(44, 19, 12, 0.1, [2, 2, 2, 2, 0, 0]), (41, 20, 12, 0.1, [2, 2, 2, 2, 0, 0])]
+
+
+@pytest.mark.parametrize("shapes", [[EVEN, EVEN2], [ODD, ODD2], THIN, SHAPES], ids=["even", "odd", "thin", "mixed"])
+@pytest.mark.parametrize("variant", [6, 7, 9, 10])
+def test_batch_lists(torch, variant, shapes):
+    """The lists of a batched sweep one by one and together: rows of one
+    kind only (a single launch, on the batch's own stream), grids whose
+    sweeps have no plane between the SBP rows of both ends, and the kernel
+    variants that do not store the acceleration (the corrector forms it) or
+    damp without a tile list."""
+    from sw4lite_amd.ew import Batch
+    steps = 4  # a replayed period and one eager step
+    alone = make_shots(steps, shapes, variant)
+    want = []
+    for e in alone:
+        e.timesteploop(steps, mode=0)
+        want.append(e.get_solution())
+        e.close()
+    shots = make_shots(steps, shapes, variant)
+    b = Batch(shots)
+    b.step(steps, graph=True)
+    for q, e in enumerate(shots):
+        u, um = e.get_solution()
+        err = max(relerr(u, want[q][0]), relerr(um, want[q][1]))
+        print("batch variant", variant, "shot", q, "relerr", err, flush=True)
+        assert np.max(np.abs(want[q][0])) > 0 and err < TOL
+    b.close()
+    for e in shots:
+        e.close()
+
+
+@pytest.mark.parametrize("variant,fields", [(7, 0), (9, 1), (10, 2)])
+def test_batch_memory_follows_the_variant(torch, variant, fields):
+    """The acceleration field (three words a point) is allocated for the
+    shots whose kernel variant stores it in the single-grid step, and for no
+    others: none for 7, the even rows' for 9, both for 10."""
+    from sw4lite_amd.ew import Batch
+    shapes = [(n, 100, 100, 0.1, [2] * 6) for n in (100, 101)]
+    field = [3 * 8 * (nx + 4) * (ny + 4) * (nz + 4) for nx, ny, nz, _, _ in shapes]
+    Batch(make_shots(3, THIN)).close()  # what the library allocates once (scratch, queues)
+    shots = make_shots(3, shapes, variant)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    b = Batch(shots)
+    used = free - torch.cuda.mem_get_info()[0]
+    print("batch variant", variant, "takes", used, "bytes, fields", field, flush=True)
+    want = sum(field[:fields])
+    assert abs(used - want) < min(field) // 2
     b.close()
     for e in shots:
         e.close()
