@@ -139,9 +139,9 @@ __global__ void k_adj_crop(Box b, Box pb, const double* __restrict__ o, double* 
 }
 
 // The eight planes of a side over block.y where a grid's tiles leave CUs idle
-// (one workgroup on each of 256).  85 tiles: transposed rows 34.3 -> 21.6 us,
+// (one workgroup on each).  85 tiles on 256 CUs: transposed rows 34.3 -> 21.6 us,
 // material derivative 32.0 -> 21.4 us against one workgroup a tile.
-inline int rows_planes_spread(int tiles) { return std::max(1, std::min(8, 256 / tiles)); }
+inline int rows_planes_spread(int tiles) { return std::max(1, std::min(8, compute_units() / tiles)); }
 
 // SBP rows of one side, transposed: out on the row planes 1..6 and the planes
 // q = 0..8 (row space, rhs4sg_rev.C:353-629) of every column of the box.

@@ -10,6 +10,9 @@ struct TileMap {
    int ntx, nty, ntiles;  // tiles along i and j, tiles in all
 };
 
+// Compute units of the device (256 on a whole MI355X).
+int compute_units();
+
 // Planes per workgroup for an LDS k-march of `tiles` column tiles over `npl`
 // planes when `per_cu` workgroups fit on a CU: the k-block count that
 // minimises (rounds of resident workgroups) x (planes per workgroup + the

@@ -23,6 +23,8 @@ namespace {
 constexpr int TX = 32, TY = 8, HX = TX + 4, HY = TY + 4, NT = TX * TY, PL = HX * HY;
 inline unsigned cdiv(long a, long b) { return (unsigned)((a + b - 1) / b); }
 
+}  // namespace
+
 int compute_units()
 {
    static const int cus = [] {
@@ -36,7 +38,6 @@ int compute_units()
    }();
    return cus;
 }
-}  // namespace
 
 int march_kchunk(long tiles, int npl, int per_cu)
 {

@@ -22,6 +22,7 @@
 // 301 x 301; FP32 67 + 82 -> 28 + 60 (its damping included: 74) at 301 x 301.
 #pragma once
 #include "kernels_common.h"
+#include "kernels_fast.h"
 
 namespace sw4amd {
 
@@ -207,10 +208,10 @@ __device__ __forceinline__ void sbp_rows_body(const Box& b, int top, int nk, int
 }
 
 // Rows over block.y: where a grid's tiles leave workgroup slots idle
-// (per_cu workgroups on each of 256 CUs) the rows are spread over them.
+// (per_cu workgroups on each CU) the rows are spread over them.
 inline int sbp_rows_spread(int tiles, int per_cu)
 {
-   const int slots = 256 * per_cu;
+   const int slots = compute_units() * per_cu;
    return 6 * tiles <= slots ? 6 : 3 * tiles <= slots ? 3 : 2 * tiles <= slots ? 2 : 1;
 }
 
