@@ -559,10 +559,14 @@ k_comp_dma(Box b, CompTiles map, int kbeg, int kend, int kc, const float* __rest
 }
 
 // The damping of the corrector on the six SBP rows, into Dn, where
-// k_comp_rows takes it from: its 46 loads a point beside the rows' columns
-// would take that kernel 245 registers and with them the second workgroup
-// per CU.  A thread walks the six rows of a column with D's column in
-// registers.  Columns and rows no damping coefficient reaches get the exact
+// k_comp_rows takes it from.  That kernel has one workgroup per CU with or
+// without the damping (185 or 252 registers), and its two waves/SIMD do not
+// hide the damping's 46 loads a point; four waves/SIMD and no barrier do
+// here.  Corrector rows with the damping inside against 118 + 22 us in two
+// passes: 199 us at 512 x 512 points, 70 against 48 + 10 at 301 x 301, 43
+// against 26 + 12 at 200 x 200; below that the second launch costs as much as
+// it gives (128 x 128: 20 against 15 + 9).  A thread walks the six rows of a
+// column with D's column in registers.  Columns and rows no damping coefficient reaches get the exact
 // zero they would have.
 __global__ void __launch_bounds__(256)
 k_comp_rows_damp(Box b, int top, int nk, const float* __restrict__ dold, const float* __restrict__ rho, SgCoefF sg,
@@ -641,7 +645,7 @@ k_comp_rows(Box b, int top, int nk, int ntx, const SbpTablesT<float>* __restrict
              for (int c = 0; c < 3; c++) aout[p + npts * c] = sc * r[c];
           } else {
              // its loads stay behind the stencil and their addresses are formed here, not kept over
-             // the rows: 128 registers
+             // the rows
              __builtin_amdgcn_sched_barrier(0);
              asm volatile("" : "+v"(p));
              const float sc = c4 / rho[p];
@@ -946,7 +950,11 @@ int comp_rows(bool corr, const Box& b, int side, int nk, const SbpTablesT<float>
    const long nx = b.ie - b.ib - 3, ny = b.je - b.jb - 3;
    const int ntx = (int)cdiv(nx, TX), nty = (int)cdiv(ny, TY);
    const int tiles = ntx * nty;
-   const dim3 grd(tiles, sbp_rows_spread(tiles, 2));
+   // workgroups a CU by registers: one of the corrector's (185), two of the
+   // predictor's (123).  Spread as if two of the corrector's fitted, each
+   // loads its columns again in a second round: 17.2 against 15.2 us at 128 x
+   // 128 points, 23.7 against 18.8 at 160 x 160, 28.8 against 26.2 at 200 x 200
+   const dim3 grd(tiles, sbp_rows_spread(tiles, corr ? 1 : 2));
    if (corr && beta != 0)
       k_comp_rows_damp<<<dim3(cdiv(nx, 64), cdiv(ny, 4)), dim3(64, 4), 0, s>>>(b, side == 4, nk, st.D, st.rho, sg,
                                                                                st.Dn, beta);

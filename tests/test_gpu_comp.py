@@ -257,6 +257,33 @@ def test_comp_async_sweeps_match_oracle(torch):
     assert err["u"] < FP32_TOL and err["um"] < FP32_TOL
 
 
+@pytest.mark.parametrize("shape", [(32, 16, 12), (33, 17, 13), (130, 90, 13), (160, 160, 13), (200, 150, 14)])
+def test_comp_rows_over_tiles(torch, shape):
+    """The FP32 SBP rows at both ends: whole 32 x 8 tiles, one column and row
+    more, and grids whose six rows are spread over six, three, two and one
+    workgroup per tile (corrector and predictor differently), from random
+    fields, against the reference order in FP64."""
+    from sw4lite_amd import EW
+    nx, ny, nz = shape
+    rho, mu, la = layered_material(nx, ny, nz, 0.1, 3)
+    rng = np.random.default_rng(13)
+    n = 3 * (nx + 4) * (ny + 4) * (nz + 4)
+    u = rng.uniform(-1, 1, n)
+    um = u - 1e-3 * rng.uniform(-1, 1, n)
+    res = []
+    for m in (2, 1):
+        e = EW(nx, ny, nz, 0.1, [2, 2, 2, 2, 0, 0], corder=1, sg_gp_thickness=4)
+        e.set_material(rho, mu, la)
+        e.setup(nsteps=2)
+        e.set_solution(u, um)
+        e.timesteploop(2, mode=m)
+        res.append(e.get_solution()[0])
+        e.close()
+    err = relerr(*res)
+    print("FP32 rows over tiles", shape, "relerr", err, flush=True)
+    assert err < FP32_TOL
+
+
 @pytest.mark.parametrize("mode", [0, 2])
 @pytest.mark.parametrize("nsteps", [1, 2, 4])
 def test_zero_ghosts_from_nonzero_ones(torch, mode, nsteps):
