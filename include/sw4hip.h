@@ -437,8 +437,9 @@ int sw4hip_ew_device_array(sw4hip_ew* ew, int which, double** ptr);
 typedef struct sw4hip_batch sw4hip_batch;
 int sw4hip_batch_create(sw4hip_ew* const* shots, int nshots, sw4hip_batch** batch);
 int sw4hip_batch_destroy(sw4hip_batch* batch);
-/* Planes per workgroup of the batched sweeps (until the first call or
- * autotuning: chosen from each shot's size). */
+/* Planes per workgroup of the batched sweeps, at least 1 (until the first
+ * call or autotuning: one value for the batch, from the tiles of all its
+ * shots and the largest nz). */
 int sw4hip_batch_set_kchunk(sw4hip_batch* batch, int kchunk);
 /* Autotuner: time one batch step for each candidate k-block (cand NULL:
  * 16, 24, 32, 40, 48, 64, 96), keep the fastest (*best, per-candidate ms in ms[] when

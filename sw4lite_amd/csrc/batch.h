@@ -63,7 +63,7 @@ private:
    int m_kchunk = 0;  // planes per workgroup of every batched sweep; 0: from all shots' tiles
    hipGraphExec_t m_exec = nullptr;
    std::vector<void*> m_allocs;
-   std::vector<DampTile*> m_dtiles;  // per shot: its damping tile list (kernel variant 9), or null
+   std::vector<DampTile*> m_dtiles;  // per shot: its damping tile list (kernel variants 9 and 10), or null
    std::vector<int> m_ndtiles;
    std::vector<double*> m_acc;       // per shot: its acceleration field (EW::accel_field), or null
    std::vector<hipStream_t> m_saved;

@@ -189,7 +189,7 @@ public:
    Sarray mMetric, mJ;     // curvilinear grid only
    std::vector<double> m_zhost;
    double* m_dacc = nullptr;  // acceleration on the planes the corrector's SBP rows read
-   double* m_accf = nullptr;  // the whole acceleration (kernel variant 8), allocated at its first step
+   double* m_accf = nullptr;  // the whole acceleration (accel_field), allocated at its first use
    int accel_field(double** p);
    // kernel variant 9: the damping sweep's tiles (damp_tiles) for planes
    // k1..k2 and the current k-chunk, made and uploaded on first use

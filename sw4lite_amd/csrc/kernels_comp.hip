@@ -320,9 +320,15 @@ k_comp_sweep(Box b, CompTiles map, int kbeg, int kend, int kc, const float* __re
 // arithmetic in the same order as k_comp_sweep.  The 16-byte loads need
 // ni % 4 == 0 and 16-byte aligned arrays (every quad of floats in one row,
 // aligned).  DW: one float a load, any row and alignment, four times the load
-// instructions; the corrector gains by it (two workgroups a CU either way,
-// 301 x 301 x 171 points: 564 us register-staged, 525), the predictor
-// does not (its extra addresses spill at 4 waves/SIMD: 344 us against 428).
+// instructions; the corrector gains by it at every size (two workgroups a CU
+// either way; register-staged -> four-byte: 29.5 -> 26.2 us at 65 x 65 x 103
+// points, 165 -> 152 at 201 x 201 x 101, 535 -> 500 at 301 x 301 x 171, 1684 ->
+// 1557 at 511 x 511 x 200).  For the predictor the two trade places (20 and
+// 20, 112 and 87, 326 and 322, 916 and 958 us: eight registers spill at 4
+// waves/SIMD), so its rows of other lengths stay register-staged.
+// Bound at 512^3: the predictor by vector issue (95% of the time), the
+// corrector by neither memory (14.3 GB at 3.9 TB/s) nor issue (66%) alone, at 2
+// waves/SIMD.
 // The predictor runs at 4 waves/SIMD (128 registers, 2 of them spilled:
 // faster than 3 waves without the spill).
 #define SW4_LDSF(p) ((__attribute__((address_space(3))) void*)(p))
@@ -922,8 +928,8 @@ int comp_sweep(bool corr, const Box& b, int k1, int k2, int kc, const CompState&
    map.ntiles = map.ntx * map.nty * (int)cdiv(k2 - k1 + 1, kc);
    const unsigned grd = 8 * cdiv(map.ntiles, 8);
    // asynchronous loads of four floats where every staged quad lies in one
-   // row, aligned; elsewhere of one float in the corrector (525 us against 564
-   // register-staged at 301 x 301 x 171), none in the predictor (428 against 344)
+   // row, aligned; elsewhere of one float in the corrector, none in the
+   // predictor (both sides measured at k_comp_dma)
    auto al = [](const float* p) { return ((uintptr_t)p & 15) == 0; };
    const bool fits = async && b.ni % 4 == 0 && al(st.mu) && al(st.la) && al(st.rho) && (corr ? al(st.A) && al(st.D) : al(st.U));
    if (corr && fits)

@@ -166,7 +166,7 @@ __device__ __forceinline__ void t_terms(const S& s, int i, int j, int m, double 
 // next barrier) and rr + D_r T; plane n-3 is finished.  The rings have five
 // slots and the plane loop is unrolled by five, so every index is a constant
 // and nothing is moved between registers.
-// Bound by latency and VALU issue at 2 waves/SIMD (one workgroup per CU, 252
+// Bound by latency and VALU issue at 2 waves/SIMD (one workgroup per CU, 234
 // registers): 384x384x256 points 1.90 ms against 6.7 ms of a thread per point reading every
 // neighbour through the caches (2126 operations, 256 registers).
 // (the scheduler would otherwise hoist the shared-memory reads of a whole
@@ -400,8 +400,8 @@ k_rhs4curv_march(Box b, int ntx, int nty, int ntiles, int klo, int khi, int kc, 
 
 // The top six rows (k = 1..6, SBP closures along k) with the same grouping
 // and the same threads as the march: the planes k = 1..8 go to LDS once, T of
-// the eight planes and the material of the column's rr stay in registers for
-// all rows; per row the columns form F and G, one barrier, and the outputs
+// the eight planes and the material of the column's rr are kept for all rows
+// (256 registers and 22-24 spilled); per row the columns form F and G, one barrier, and the outputs
 // are finished.  With rr written as in the march,
 //   rr = 1/(sx sy) sum_q [mu |m|^2 w_a + (mu + lambda) m_a (m . w)]_q,
 //   w_b(k, q) = sum_t acof(k, t, q) u_b(t)  (and ghcof on the ghost plane).

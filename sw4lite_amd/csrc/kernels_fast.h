@@ -66,16 +66,6 @@ enum SweepLoads { LOADS_WIDE = 0, LOADS_NARROW = 1, LOADS_STAGED = 2 };
 int launch_sweep_batch(int kind, SweepLoads loads, const SweepShot* d_shots, int nshots, int nblocks, hipStream_t s);
 bool async_loads_fit(const Box& b, const double* const* arrays, int n);
 
-// Interior planes k1..k2 of the predictor (corr = false: out = Up from u, um)
-// or corrector sweep (corr = true: out = Up' from upin = Up, u, um), chunks of
-// kc planes per workgroup.
-// variant 1: plain k-march, 2 waves/SIMD; 2: register prefetch of the next
-// plane, 2 waves/SIMD; 3: prefetch, 1 wave/SIMD; 4: as 3 with the corrector's
-// supergrid damping (beta != 0) applied in the same sweep; 5: corrector as 4,
-// predictor as 1; 6: both as 1, the damping by launch_damp; 7: as 6, the
-// predictor by asynchronous global-to-LDS loads where the rows allow it; 8:
-// as 7, with acc the acceleration stored and staged (below); 9: as 8, the
-// damping sweep restricted to the supergrid layers (damp_tiles).
 // out = L(u) on planes k1..k2 (rhs4sg's interior rows) of either array
 // layout, the columns of the box two points inside its i and j ends.
 int launch_rhs4_march(int co, const Box& b, int k1, int k2, const double* u, const double* mu, const double* la,
@@ -103,13 +93,24 @@ std::vector<DampTile> damp_tiles(const Box& b, int k1, int k2, int kc, const dou
 // with tiles (device array of damp_tiles for the same k1, k2, kc) only those
 // tiles run (else the whole box).
 int launch_damp(const Box& b, int k1, int k2, int kc, double* up, const double* u, const double* um,
-                    const double* rho, const SgCoef& sg, double beta, hipStream_t s,
-                    const DampTile* tiles = nullptr, int ntiles = 0);
-// Variant 8 with acc (3 npts doubles, even row length, aligned arrays): the
+                const double* rho, const SgCoef& sg, double beta, hipStream_t s, const DampTile* tiles = nullptr,
+                int ntiles = 0);
+// Interior planes k1..k2 of the predictor (corr = false: out = Up from u, um)
+// or corrector sweep (corr = true: out = Up' from upin = Up, u, um), chunks of
+// kc planes per workgroup.
+// variant 1: plain k-march, 2 waves/SIMD; 2: register prefetch of the next
+// plane, 2 waves/SIMD; 3: prefetch, 1 wave/SIMD; 4: as 3 with the corrector's
+// supergrid damping (beta != 0) applied in the same sweep; 5: corrector as 4,
+// predictor as 1; 6: both as 1, the damping by launch_damp; 7: as 6, the
+// predictor by asynchronous global-to-LDS loads where the rows allow it; 8:
+// as 7, with acc the acceleration stored and staged; 9: as 8, the damping
+// sweep restricted to the supergrid layers (damp_tiles); 10: as 9, rows of
+// odd length and arrays off 16 bytes by four-byte asynchronous loads.
+// acc (3 npts doubles; variants 8 and 9: even row length, aligned arrays): the
 // predictor also stores the acceleration (up - 2u + um)/dt^2 at the points
 // it computes, the corrector stages acc instead of forming it; between the
 // two, launch_accel_fix and launch_accel_points complete acc from the final
-// Up.  Without acc, variant 8 is variant 7.
+// Up.  Without acc the corrector forms it (as variant 7).
 int launch_sweep_lds(bool corr, int variant, const Box& b, int k1, int k2, int kc, const double* upin,
                      const double* u, const double* um, const double* mu, const double* la, const double* rho,
                      const SgCoef& sg, double* out, double h, double dt, double beta, hipStream_t s,

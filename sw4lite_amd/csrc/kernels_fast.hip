@@ -3,13 +3,18 @@
 // A workgroup owns a 32 x 8 tile of (i,j) columns and marches along k over a
 // chunk of planes.  The five displacement planes k-2..k+2 the 4th-order
 // stencil touches are kept, with their 2-point (i,j) halo, in an LDS ring;
-// each new plane is loaded once from HBM (coalesced rows of 36 doubles) and
-// read ~135 times from LDS.  mu and lambda of the current plane sit in LDS for
-// the in-plane terms, the column values k+-1, k+-2 rotate in registers.  The
-// corrector stages (Up - 2U + Um)/dt^2 instead of U, so the acceleration is
-// never stored.  The arithmetic is rhs4_interior_body, shared with the
-// global-memory kernels (same results to rounding).  The supergrid damping
-// of the corrector sweep runs as k_addsgd4_planes right after it.
+// each new plane is loaded once from HBM (rows of 36 doubles) and read ~135
+// times from LDS.  mu and lambda of the current plane sit in LDS for the
+// in-plane terms, the column values k+-1, k+-2 rotate in registers.
+// By default (kernel variant 10) the planes come by asynchronous
+// global-to-LDS loads into a ring of six (sweep_dma_body), the predictor
+// stores the acceleration (Up - 2U + Um)/dt^2 and the corrector stages it;
+// variants up to 7, and 8 and 9 on rows of odd length, stage the corrector's
+// planes through registers (sweep_lds_body) and form the acceleration on the
+// way.  The arithmetic is rhs4_interior_body, shared with the global-memory
+// kernels (same results to rounding).  The supergrid damping of the corrector
+// is a sweep of its own right after it (k_damp_tiles over the layers' tiles
+// from variant 9 on).
 #include <algorithm>
 
 #include "kernels_common.h"
@@ -713,7 +718,9 @@ static bool dma_fits(const Box& b, const double* u, const double* mu, const doub
 // three workgroups per CU.  Same conditions as sweep_dma_body (even ni,
 // 16-byte aligned arrays); DW: rows of any length by four-byte loads
 // (301 x 301 x 171 points: 358 us against 417 us staged through registers;
-// 512^3 1.22 ms).  A column march with d in registers and LDS that loads
+// 512^3 1.22 ms).  Bound by memory at 512^3: 8.0 GB of measured traffic at 6.5
+// TB/s, twice the algorithmic bytes (tile halos, tiles that reach only partly
+// into a layer).  A column march with d in registers and LDS that loads
 // every value once was slower (410 us, 1.27 ms): two workgroups per CU
 // instead of three, and loads no further ahead.
 // Column tile (tix, tjy), planes k0..k1.  POINT: points that no damping
@@ -1045,7 +1052,6 @@ int fill_sweep_shot(bool damping, const Box& b, int k1, int k2, int kc, const do
                     const DampTile* tiles, int ntiles, double* acc)
 {
    const long nx = b.ie - b.ib - 3, ny = b.je - b.jb - 3;
-   if (kc <= 0) kc = 64;
    sh->b = b;
    sh->map.ntx = (int)cdiv(nx, TX);
    sh->map.nty = (int)cdiv(ny, damping ? 8 : TY);

@@ -19,7 +19,8 @@
 // Predictor and corrector rows of the step, against rows evaluated one after
 // the other by one wave per SIMD with all neighbours' derivatives formed
 // again: 62 + 60 -> 9 + 9 us at 40 x 36 points, 157 + 181 -> 55 + 55 at
-// 301 x 301; FP32 67 + 82 -> 28 + 60 (its damping included: 74) at 301 x 301.
+// 301 x 301; FP32 there 67 + 82 -> 25 + 58, the damping (10, a pass of its own)
+// included.
 #pragma once
 #include "kernels_common.h"
 #include "kernels_fast.h"
